@@ -384,7 +384,7 @@ int pk_launch_act_records(const float *x, int n, int32_t *rec, hipStream_t st) {
 }
 
 // compute units of the current device (cached per device)
-static int pk_device_cus() {
+int pk_device_cus() {
     static int cus[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;

@@ -215,6 +215,12 @@ static int route_rows(pk_engine *e, const rows_scratch &sc, int layer, const flo
                                 e->stream);
 }
 
+// (token, expert) pairs from which the fp32 chains run on k_i4_rows: with
+// fewer, the pair grouping's launch costs more than the shared decodes give
+// (20B layer, 3 tokens 135.6 us either way, 6 tokens 164 against 158 us; 128
+// experts, 3 tokens 142 against 149).
+constexpr int ROWS_MIN_PAIRS = 24;
+
 // The MoE of forward_prefill (picchio.c:1829-1916) for T tokens x [T][D]:
 // out[t] = (residual ? residual[t] : 0) + sum over the token's experts, in the
 // batch's expert order, of (w_k * routed_scale) * expert_k(x[t]). With
@@ -243,19 +249,25 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
         gu.xq = sc.xq; gu.xq_stride = xq_row;
         gu.yq = sc.actq; gu.yq_stride = aq_row;
     }
-    // with the integer dot, pairs of one expert share each weight load (tiles of 4)
+    // pairs of one expert share each weight load: tiles of 4 on the integer
+    // dot (the tile kernel keeps 4 pairs' group sums in LDS: rows of at most
+    // 64 groups), of 8 on the fp32 chains
     const int P = T * K;
     const int mt = P / 4 + 1 + E;
     pk_i4_tiles tl{sc.pairs, sc.tiles, sc.tiles + mt, sc.tiles + 2 * mt, sc.tiles + 3 * mt};
-    // (the tile kernel keeps 4 pairs' group sums in LDS: rows of at most 64 groups)
     const bool tiled = dot && !e->dot_tiles_off && e->ex.gu.NG <= 64 && e->ex.dn.NG <= 64 && E <= 128;
-    if (tiled)
+    const bool rows = !dot && E <= 128 && P >= ROWS_MIN_PAIRS && pk_i4_rows_ok(gu, PK_EPI_SWIGLU);
+    const int tile = tiled ? 4 : PK_ROWS_TILE, max_tiles = P / tile + 1 + E;
+    if (tiled || rows)
         PK_TRY(pk_launch_group_pairs(sc.sel, P, E, sc.pairs, sc.tiles, sc.tiles + mt,
-                                     sc.tiles + 2 * mt, sc.tiles + 3 * mt, e->stream, 4));
+                                     sc.tiles + 2 * mt, sc.tiles + 3 * mt, e->stream, tile));
     int ps = pk_prof_begin(e, PK_PROF_EXPERT_GATE_UP);
     if (tiled)
-        PK_TRY(pk_launch_i4_dot_tiles(gu, tl, e->ex.gu, PK_EPI_SWIGLU, c->swiglu_limit, c->swiglu_alpha, mt,
+        PK_TRY(pk_launch_i4_dot_tiles(gu, tl, e->ex.gu, PK_EPI_SWIGLU, c->swiglu_limit, c->swiglu_alpha, max_tiles,
                                       e->stream));
+    else if (rows)
+        PK_TRY(pk_launch_i4_rows(gu, &tl, e->ex.gu, PK_EPI_SWIGLU, c->swiglu_limit, c->swiglu_alpha, max_tiles,
+                                 e->stream));
     else
         PK_TRY(pk_launch_i4_gemv(gu, e->ex.gu, PK_EPI_SWIGLU, c->swiglu_limit, c->swiglu_alpha, nullptr,
                                  e->stream));
@@ -270,7 +282,9 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
     }
     ps = pk_prof_begin(e, PK_PROF_EXPERT_DOWN);
     if (tiled)
-        PK_TRY(pk_launch_i4_dot_tiles(dn, tl, e->ex.dn, PK_EPI_PLAIN, 0.f, 0.f, mt, e->stream));
+        PK_TRY(pk_launch_i4_dot_tiles(dn, tl, e->ex.dn, PK_EPI_PLAIN, 0.f, 0.f, max_tiles, e->stream));
+    else if (rows)
+        PK_TRY(pk_launch_i4_rows(dn, &tl, e->ex.dn, PK_EPI_PLAIN, 0.f, 0.f, max_tiles, e->stream));
     else
         PK_TRY(pk_launch_i4_gemv(dn, e->ex.dn, PK_EPI_PLAIN, 0.f, 0.f, nullptr, e->stream));
     PK_TRY(pk_prof_end(e, ps));

@@ -1,0 +1,56 @@
+"""The INT4 GEMV of several input rows on the fp32 matrix instructions
+(k_i4_rows): bit-identical to matmul_i4_gs (quant.h:259-319) at the edges of
+its tiles (8 input rows, 64 matrix rows, spans of 48 groups), and to the
+per-pair kernels inside the batched MoE."""
+import numpy as np
+import pytest
+
+from helpers import bits_equal, first_mismatch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rand(shape, seed, scale=1.0):
+    return (np.random.default_rng(seed).standard_normal(shape) * scale).astype(np.float32)
+
+
+@pytest.mark.parametrize("offset", [0, 1], ids=["aligned", "unaligned"])
+@pytest.mark.parametrize("O,I,S", [(64, 64, 257), (130, 128, 87), (200, 3136, 65), (70, 6208, 131), (4000, 128, 5),
+                                   (2880, 2880, 17), (720, 2880, 31)])
+def test_i4_rows_matmul_bitexact(gpu, oracle, O, I, S, offset):
+    """offset 1: input rows that are not 16-byte aligned take the per-row kernel."""
+    import picchio_amd as pa
+    import torch
+    q4, s = oracle.quant_gs(_rand((O, I), 5 + O + I, 0.02), 64)
+    x = _rand((S, I), 9 + S)
+    # the chains hold q/16: exact while a sum's last bit, at least 2^-24 of the
+    # smallest term x/16, stays above the least denormal 2^-149 (|x| > 2^-121)
+    x[0, ::7] *= 1e-30
+    y_ref = oracle.mm_i4_gs(x, q4, s, O, I, 64)
+    with pa.Engine(pa.gptoss_cfg(n_layers=1, n_experts=4, ctx_len=16, vocab=64)) as eng:
+        qt = eng.qt_upload(pa.FMT_INT4, q4, s, O, I, 64)
+        buf = eng.to_dev(np.concatenate([np.zeros(offset, np.float32), x.ravel()]))
+        yd = eng.empty((S, O), torch.float32)
+        eng.matmul_qt(yd, buf[offset:], qt, S)
+        y = eng.to_host(yd)
+        eng.qt_free(qt)
+    assert bits_equal(y, y_ref), first_mismatch(y, y_ref)
+
+
+@pytest.mark.parametrize("T", [23, 24, 70])
+def test_i4_rows_moe_matches_single_tokens(gpu, T):
+    """With one expert per token the batch's expert order does not matter:
+    every row of the grouped launch has the bits of the token's own call."""
+    import picchio_amd as pa
+    import torch
+    cfg = pa.gptoss_cfg(n_layers=1, n_experts=8, topk=1, ctx_len=16, vocab=64)
+    with pa.Engine(cfg) as eng:
+        eng.build_synthetic(11, 1)
+        xd = eng.to_dev(_rand((T, cfg.hidden), 3 + T))
+        out = eng.empty((T, cfg.hidden), torch.float32)
+        one = eng.empty((T, cfg.hidden), torch.float32)
+        eng.moe_forward_batch(0, xd, out)
+        for t in range(T):
+            eng.moe_forward_batch(0, xd[t:t + 1], one[t:t + 1])
+        a, b = eng.to_host(out), eng.to_host(one)
+    assert bits_equal(a, b), first_mismatch(a, b)
