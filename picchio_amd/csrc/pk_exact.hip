@@ -25,147 +25,377 @@
 #include "pk_engine.h"
 #include "pk_i4_device.h"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace {
 
 // ───────────────────────── matmul_f32 for S rows ─────────────────────────
-// grid (ceil(O / 32), ceil(S / 64)), 256 threads. Wave w owns outputs
-// o0 + 8w .. +7 of the block; lane l = 8 g + j owns chain j of rows
-// s0 + 8g .. +7 for those 8 outputs (64 accumulators). Column chunks of 64
-// (8 chain steps) are staged in LDS as [step][j][row] and [step][j][output]
-// so each lane reads its eight x and eight w values as two 16-byte loads.
-constexpr int CH_KC = 64;                 // columns per staged chunk
-constexpr int CH_ROWS = 64, CH_OUTS = 32;
+// fp32 matrix instructions with K = 1 are one correctly rounded fused
+// multiply-add per element (denormals kept: checked against fmaf over 12
+// million random operands), so their accumulators are the reference's
+// chains. They share the VALU's multipliers (28 ns per 2048 products and
+// SIMD, v_fma 40), so what bounds these kernels is the weight stream for a
+// few rows, the multipliers and how evenly the waves cover the SIMDs for
+// many; a chain is serial over the columns, so K is never split.
+//
+// k_gemm_chain8, few rows: a workgroup of two waves computes 16 outputs of 16
+// input rows (MF) or of NS = 1 or 2. The weights and inputs pass through LDS
+// in chunks of 128 columns (two buffers, one barrier per chunk, two chunks'
+// loads in flight in registers). Lane l = 16 b + r of wave h reads column
+// 8k + 4h + b of weight row r and input row r (the row pitch of 4 mod 64
+// floats puts the 64 lanes on 64 banks).
+//  * MF: v_mfma_f32_16x16x1_4b_f32, the four blocks being chains 4h .. 4h + 3.
+//  * NS: the same chains as v_fma, one per lane and input row.
+// The second wave's chains join the first's through LDS for hsum256's tree.
+// Measured (us, fp32, against the kernel before it: 64 rows x 32 outputs per
+// workgroup on v_fma): 5120 x 2880, 1 row 179 -> 17.5, 64 rows 178 -> 55;
+// INT8 201088 x 2880, 1 row 4100 -> 230 (k_gemv_chain8_q8: 132).
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
+constexpr int CH_OUTS = 16;
+constexpr int CH_THREADS = 128;
+constexpr int CH_KC = 128;                // columns per staged chunk
+constexpr int CH_MAX_Y = 65535;           // grid.y; further rows in grid.z
+
+// Sixteen stored int8 weights as floats at d.
+__device__ __forceinline__ void ch_put_i8(float *d, uint4 w) {
+    const uint32_t v[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        *reinterpret_cast<float4 *>(d + 4 * k) = make_float4((float)(int8_t)v[k], (float)(int8_t)(v[k] >> 8),
+                                                             (float)(int8_t)(v[k] >> 16), (float)(int8_t)(v[k] >> 24));
+}
+
+// Output (s, o) from the tree a of its chains: the columns past the last
+// whole 8, the row scale, bias and residual.
+template <typename TW>
+__device__ __forceinline__ void ch_finish(const float *X, int64_t ldx, const TW *W, const float *rscale,
+                                          const float *bias, float *out, int64_t ldo, int S, int I, int O,
+                                          int add_res, float a, int s, int o) {
+    if (s >= S || o >= O) return;
+    const TW *wr = W + (int64_t)o * I;
+    const float *xr = X + (int64_t)s * ldx;
+    int c = I & ~7;
+    if constexpr (sizeof(TW) == 4) {
+        if (I - c >= 4) {
+            const float p0 = xr[c] * wr[c], p1 = xr[c + 1] * wr[c + 1];
+            const float p2 = xr[c + 2] * wr[c + 2], p3 = xr[c + 3] * wr[c + 3];
+            a = a + p0; a = a + p1; a = a + p2; a = a + p3;
+            c += 4;
+        }
+    }
+    for (; c < I; ++c) a = __builtin_fmaf(xr[c], (float)wr[c], a);
+    if (rscale) a = a * rscale[o];
+    if (bias) a = a + bias[o];
+    float *y = out + (int64_t)s * ldo + o;
+    *y = add_res ? *y + a : a;
+}
 
 // TW = int8_t: matmul_q8 (quant.h:152-186), the same chains over the weights
 // converted to float, the tail as contracted FMAs, the sum times the row scale.
-// VEC (fp32 weights, 16-byte aligned rows, ldx and I multiples of 4): each
-// chunk's 64 x 64 inputs and 32 x 64 weights load as six float4 per thread,
-// the next chunk's while the current one is multiplied (the scalar loops
-// wait for every load on its own).
-template <typename TW, bool VEC = false>
-__global__ __launch_bounds__(256) void k_gemm_chain8(const float *__restrict__ X, int64_t ldx,
-                                                     const TW *__restrict__ W, const float *__restrict__ rscale,
-                                                     const float *__restrict__ bias, float *out, int64_t ldo,
-                                                     int S, int I, int O, int add_res) {
-    __shared__ __attribute__((aligned(16))) float xs[CH_KC / 8][8][CH_ROWS];
-    __shared__ __attribute__((aligned(16))) float ws[CH_KC / 8][8][CH_OUTS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int j = lane & 7, g = lane >> 3;
-    const int o0 = blockIdx.x * CH_OUTS, s0 = blockIdx.y * CH_ROWS;
-    const int I8 = I & ~7;
-    float acc[8][8];
+// VEC: 16-byte loads (16-byte aligned rows of X and W, I a multiple of 4, or
+// of 16 for int8 weights).
+template <typename TW, bool VEC, bool MF, int NS>
+__global__ __launch_bounds__(CH_THREADS) void k_gemm_chain8(const float *__restrict__ X, int64_t ldx,
+                                                            const TW *__restrict__ W,
+                                                            const float *__restrict__ rscale,
+                                                            const float *__restrict__ bias, float *out, int64_t ldo,
+                                                            int S, int I, int O, int add_res) {
+    constexpr int KC = CH_KC, P = KC + 4, XR = MF ? 16 : NS;
+    constexpr int WV = VEC ? 16 / sizeof(TW) : 1, XV = VEC ? 4 : 1;     // values per load
+    constexpr int WN = (CH_OUTS * KC / WV + CH_THREADS - 1) / CH_THREADS;
+    constexpr int XN = (XR * KC / XV + CH_THREADS - 1) / CH_THREADS;
+    constexpr int BUF = (CH_OUTS + XR) * P;
+    __shared__ __attribute__((aligned(16))) float lds[2 * BUF];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int h = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int o0 = blockIdx.x * CH_OUTS;
+    const int s0 = ((int)blockIdx.y + CH_MAX_Y * (int)blockIdx.z) * XR;
+    const int I8 = I & ~7, chunks = (I8 + KC - 1) / KC;
+
+    struct stage {
+        typename std::conditional<VEC, uint4, TW>::type w[WN];
+        typename std::conditional<VEC, float4, float>::type x[XN];
+    };
+    // load e of a chunk: row e / (KC / V), columns V (e % (KC / V)) .. (rows
+    // and columns past the end repeat the last ones; they are not used)
+    auto load = [&](stage &st, int c0) {
+        const int nc = min(KC, I8 - c0);
 #pragma unroll
-    for (int m = 0; m < 8; ++m)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[m][i] = 0.0f;
-    float4 xv4[4], wv4[2];
-    // float4 e = tid + 256 u of the chunk: row e / 16, columns 4 (e % 16) .. +3
-    auto load = [&](int c0) {
-        const int nc = min(CH_KC, I8 - c0);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u, r = e >> 4, c = 4 * (e & 15), sr = min(s0 + r, S - 1);
-            const float4 v = *reinterpret_cast<const float4 *>(X + (int64_t)sr * ldx + c0 + min(c, nc - 4));
-            xv4[u] = c < nc && s0 + r < S ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int u = 0; u < WN; ++u) {
+            const int e = min(tid + CH_THREADS * u, CH_OUTS * KC / WV - 1), r = e / (KC / WV);
+            const int c = min(WV * (e % (KC / WV)), nc - WV);
+            const TW *p = W + (int64_t)min(o0 + r, O - 1) * I + c0 + c;
+            if constexpr (VEC) st.w[u] = pk_load_nt(reinterpret_cast<const uint4 *>(p));
+            else st.w[u] = *p;
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = tid + 256 * u, r = e >> 4, c = 4 * (e & 15), orow = min(o0 + r, O - 1);
-            const float4 v =
-                *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(W) + (int64_t)orow * I + c0 +
-                                                  min(c, nc - 4));
-            wv4[u] = c < nc && o0 + r < O ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int u = 0; u < XN; ++u) {
+            const int e = min(tid + CH_THREADS * u, XR * KC / XV - 1), r = e / (KC / XV);
+            const int c = min(XV * (e % (KC / XV)), nc - XV);
+            const float *p = X + (int64_t)min(s0 + r, S - 1) * ldx + c0 + c;
+            if constexpr (VEC) st.x[u] = *reinterpret_cast<const float4 *>(p);
+            else st.x[u] = *p;
         }
     };
-    if constexpr (VEC)
-        if (I8 > 0) load(0);
-    for (int c0 = 0; c0 < I8; c0 += CH_KC) {
-        const int nc = min(CH_KC, I8 - c0);    // a multiple of 8
-        __syncthreads();
-        if constexpr (VEC) {
+    auto store = [&](const stage &st, float *wl, float *xl) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int e = tid + 256 * u, r = e >> 4, c = 4 * (e & 15);
-                xs[c >> 3][(c & 7) + 0][r] = xv4[u].x;
-                xs[c >> 3][(c & 7) + 1][r] = xv4[u].y;
-                xs[c >> 3][(c & 7) + 2][r] = xv4[u].z;
-                xs[c >> 3][(c & 7) + 3][r] = xv4[u].w;
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int e = tid + 256 * u, r = e >> 4, c = 4 * (e & 15);
-                ws[c >> 3][(c & 7) + 0][r] = wv4[u].x;
-                ws[c >> 3][(c & 7) + 1][r] = wv4[u].y;
-                ws[c >> 3][(c & 7) + 2][r] = wv4[u].z;
-                ws[c >> 3][(c & 7) + 3][r] = wv4[u].w;
-            }
-        } else {
-            // X chunk: 64 rows x nc columns (zeros past S), 16 per thread
-            for (int e = tid; e < CH_ROWS * CH_KC; e += 256) {
-                const int r = e / CH_KC, c = e - r * CH_KC;
-                const int s = s0 + r;
-                xs[c >> 3][c & 7][r] = (c < nc && s < S) ? X[(int64_t)s * ldx + c0 + c] : 0.0f;
-            }
-            for (int e = tid; e < CH_OUTS * CH_KC; e += 256) {
-                const int r = e / CH_KC, c = e - r * CH_KC;
-                const int o = o0 + r;
-                ws[c >> 3][c & 7][r] = (c < nc && o < O) ? (float)W[(int64_t)o * I + c0 + c] : 0.0f;
+        for (int u = 0; u < WN; ++u) {
+            const int e = tid + CH_THREADS * u, r = e / (KC / WV), c = WV * (e % (KC / WV));
+            if (WN * CH_THREADS > CH_OUTS * KC / WV && e >= CH_OUTS * KC / WV) break;
+            float *d = wl + r * P + c;
+            if constexpr (VEC && sizeof(TW) == 4) {
+                *reinterpret_cast<uint4 *>(d) = st.w[u];
+            } else if constexpr (VEC) {
+                ch_put_i8(d, st.w[u]);
+            } else {
+                *d = (float)st.w[u];
             }
         }
-        __syncthreads();
-        if constexpr (VEC)
-            if (c0 + CH_KC < I8) load(c0 + CH_KC);
-        for (int k = 0; k < nc / 8; ++k) {
-            const float4 xa = *reinterpret_cast<const float4 *>(&xs[k][j][8 * g]);
-            const float4 xb = *reinterpret_cast<const float4 *>(&xs[k][j][8 * g + 4]);
-            const float4 wa = *reinterpret_cast<const float4 *>(&ws[k][j][8 * wave]);
-            const float4 wb = *reinterpret_cast<const float4 *>(&ws[k][j][8 * wave + 4]);
-            const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-            const float wv[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
 #pragma unroll
-            for (int m = 0; m < 8; ++m)
+        for (int u = 0; u < XN; ++u) {
+            const int e = tid + CH_THREADS * u, r = e / (KC / XV), c = XV * (e % (KC / XV));
+            if (XN * CH_THREADS > XR * KC / XV && e >= XR * KC / XV) break;
+            if constexpr (VEC) *reinterpret_cast<float4 *>(xl + r * P + c) = st.x[u];
+            else xl[r * P + c] = st.x[u];
+        }
+    };
+
+    const int r = lane & 15, b = lane >> 4;
+    f32x16 acc;
+    float a1[NS ? NS : 1];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) acc[m][i] = __builtin_fmaf(xv[i], wv[m], acc[m][i]);
+    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NS; ++t) a1[t] = 0.0f;
+    auto multiply = [&](const float *wl, const float *xl, int steps) {
+        const float *wp = wl + r * P + 4 * h + b, *xp = xl + (MF ? r * P : 0) + 4 * h + b;
+        auto step = [&](int k) {
+            const float w = wp[8 * k];
+            if constexpr (MF) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xp[8 * k], w, acc, 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < NS; ++t) a1[t] = __builtin_fmaf(xp[t * P + 8 * k], w, a1[t]);
+        };
+        if (steps == KC / 8) {
+#pragma unroll
+            for (int k = 0; k < KC / 8; ++k) step(k);
+        } else {
+            for (int k = 0; k < steps; ++k) step(k);
+        }
+    };
+    stage st[2];
+    if (chunks > 0) {
+        load(st[0], 0);
+        load(st[1], min(1, chunks - 1) * KC);
+    }
+    for (int n = 0; n < chunks; n += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (n + u < chunks) {
+                float *wl = lds + u * BUF, *xl = wl + CH_OUTS * P;
+                store(st[u], wl, xl);
+                load(st[u], min(n + u + 2, chunks - 1) * KC);
+                __syncthreads();
+                multiply(wl, xl, min(KC, I8 - (n + u) * KC) / 8);
+            }
         }
     }
-    // hsum256 across the eight chain lanes: lane j = 0 ends with the row value
+    // hsum256: ((c0+c4)+(c2+c6))+((c1+c5)+(c3+c7)); wave 1 holds c4 .. c7
+    __syncthreads();
+    if (h == 1) {
+        if constexpr (MF) {
 #pragma unroll
-    for (int m = 0; m < 8; ++m)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            float v = acc[m][i];
-            v = v + __shfl_xor(v, 4, 64);
-            v = v + __shfl_xor(v, 2, 64);
-            v = v + __shfl_xor(v, 1, 64);
-            acc[m][i] = v;
+            for (int i = 0; i < 16; ++i) lds[i * 64 + lane] = acc[i];
         }
-    if (j != 0) return;
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        const int o = o0 + 8 * wave + m;
-        if (o >= O) continue;
-        const TW *wr = W + (int64_t)o * I;
+        for (int t = 0; t < NS; ++t) lds[t * 64 + lane] = a1[t];
+    }
+    __syncthreads();
+    if (h == 1) return;
+    if constexpr (MF) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int s = s0 + 8 * g + i;
-            if (s >= S) continue;
-            const float *xr = X + (int64_t)s * ldx;
-            float a = acc[m][i];
-            int c = I8;
+        for (int i = 0; i < 4; ++i) {
+            // register 4 b + i: chain b, input row 4 (lane / 16) + i, output lane % 16
+            const float b0 = acc[i] + lds[i * 64 + lane], b1 = acc[4 + i] + lds[(4 + i) * 64 + lane];
+            const float b2 = acc[8 + i] + lds[(8 + i) * 64 + lane], b3 = acc[12 + i] + lds[(12 + i) * 64 + lane];
+            ch_finish(X, ldx, W, rscale, bias, out, ldo, S, I, O, add_res, (b0 + b2) + (b1 + b3), s0 + 4 * b + i,
+                      o0 + r);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+        float v = a1[t] + lds[t * 64 + lane];        // lane 16 b + r: c_b + c_{b+4}
+        v = v + __shfl_xor(v, 32, 64);
+        v = v + __shfl_xor(v, 16, 64);
+        if (b == 0) ch_finish(X, ldx, W, rscale, bias, out, ldo, S, I, O, add_res, v, s0 + t, o0 + r);
+    }
+}
+
+// One to four rows of many int8 outputs: a wave computes 64 outputs, lane =
+// weight row with its eight chains in registers, the inputs in scalar
+// registers. The wave's 64 x 128 byte chunk passes through its own LDS (rows
+// 144 bytes apart: 16-byte reads of 16 rows on distinct banks), the next
+// chunk's loads in flight. Per weight one conversion and NS fused
+// multiply-adds (2.2 + 1.25 NS ns per 64 and SIMD), so it is bound by the
+// weight stream. 201088 x 2880, 1 row: 132 us = 4.4 TB/s;
+// k_gemm_chain8 230 (it keeps the weights in LDS as floats).
+constexpr int GQ_KC = 128, GQ_P = GQ_KC + 16;
+template <int NS>
+__global__ __launch_bounds__(64) void k_gemv_chain8_q8(const float *__restrict__ X, const int8_t *__restrict__ W,
+                                                       const float *__restrict__ rscale, float *out, int S, int I,
+                                                       int O) {
+    __shared__ __attribute__((aligned(16))) uint8_t wl[64 * GQ_P];
+    const int lane = threadIdx.x, o0 = blockIdx.x * 64;
+    const int chunks = (I + GQ_KC - 1) / GQ_KC;      // (I % 16 == 0)
+    uint4 st[8];
+    // load u: rows 8 u + lane / 8, 16 bytes at 16 (lane % 8)
+    const int lr = lane >> 3, lc = 16 * (lane & 7);
+    auto load = [&](int c0) {
+        const int c = min(c0 + lc, I - 16);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            st[u] = pk_load_nt(reinterpret_cast<const uint4 *>(W + (int64_t)min(o0 + 8 * u + lr, O - 1) * I + c));
+    };
+    float acc[NS][8];
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[t][j] = 0.0f;
+    const pk_cptr<float> x = pk_const(X);
+    load(0);
+    for (int n = 0; n < chunks; ++n) {
+        const int c0 = n * GQ_KC;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) *reinterpret_cast<uint4 *>(wl + (8 * u + lr) * GQ_P + lc) = st[u];
+        __builtin_amdgcn_wave_barrier();
+        load(min(n + 1, chunks - 1) * GQ_KC);
+        const int pieces = min(GQ_KC, I - c0) / 16;
+        for (int m = 0; m < pieces; ++m) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(wl + lane * GQ_P + 16 * m);
+            const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float w = (float)(int8_t)(d[q] >> (8 * i));
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) {
+                        const int j = 4 * (q & 1) + i;
+                        acc[t][j] = __builtin_fmaf(x[(int64_t)min(t, S - 1) * I + c0 + 16 * m + 4 * q + i], w, acc[t][j]);
+                    }
+                }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+        const float b0 = acc[t][0] + acc[t][4], b1 = acc[t][1] + acc[t][5];
+        const float b2 = acc[t][2] + acc[t][6], b3 = acc[t][3] + acc[t][7];
+        ch_finish<int8_t>(X, I, W, rscale, nullptr, out, O, S, I, O, 0, (b0 + b2) + (b1 + b3), t, o0 + lane);
+    }
+}
+
+// Many rows (fp32 or int8 weights, 16-byte loads): a workgroup of four waves
+// computes 64 outputs of 64 input rows, wave (p, q) outputs 32 p .. and rows
+// 32 q .. with v_mfma_f32_32x32x1_2b_f32: lane l = 32 b + r reads columns
+// 8k + 4b .. + 3 of weight row r and input row r as one float4 each, and
+// instruction i multiplies component i, its two blocks being chains i and
+// 4 + i. Chunks of 32 columns, staged as above. 5120 x 2880, 512 rows: 183 us
+// (82 TFLOP/s; 367 in 16-row tiles).
+constexpr int CT_TILE = 64, CT_KC = 32, CT_P = CT_KC + 4;
+template <typename TW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_chain8_tile(
+    const float *__restrict__ X, int64_t ldx, const TW *__restrict__ W, const float *__restrict__ rscale,
+    const float *__restrict__ bias, float *out, int64_t ldo, int S, int I, int O, int add_res) {
+    constexpr int WV = 16 / sizeof(TW);
+    constexpr int WN = CT_TILE * CT_KC / WV / 256 > 0 ? CT_TILE * CT_KC / WV / 256 : 1, XN = CT_TILE * CT_KC / 4 / 256;
+    constexpr int BUF = 2 * CT_TILE * CT_P;
+    __shared__ __attribute__((aligned(16))) float lds[2 * BUF];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p = wave & 1, q = wave >> 1;
+    const int o0 = blockIdx.x * CT_TILE, s0 = blockIdx.y * CT_TILE;
+    const int I8 = I & ~7, chunks = (I8 + CT_KC - 1) / CT_KC;
+    const int we = min(tid, CT_TILE * CT_KC / WV - 1);          // (int8: 128 loads of 16 columns)
+    struct stage {
+        pk_f32x4 w[WN];
+        pk_f32x4 x[XN];
+    };
+    auto load = [&](stage &st, int c0) {
+        const int nc = min(CT_KC, I8 - c0);
+#pragma unroll
+        for (int u = 0; u < WN; ++u) {
+            const int e = we + 256 * u, r = e / (CT_KC / WV), c = min(WV * (e % (CT_KC / WV)), nc - WV);
+            st.w[u] = *reinterpret_cast<const pk_f32x4 *>(W + (int64_t)min(o0 + r, O - 1) * I + c0 + c);
+        }
+#pragma unroll
+        for (int u = 0; u < XN; ++u) {
+            const int e = tid + 256 * u, r = e / (CT_KC / 4), c = min(4 * (e % (CT_KC / 4)), nc - 4);
+            st.x[u] = *reinterpret_cast<const pk_f32x4 *>(X + (int64_t)min(s0 + r, S - 1) * ldx + c0 + c);
+        }
+    };
+    auto store = [&](const stage &st, float *wl, float *xl) {
+#pragma unroll
+        for (int u = 0; u < WN; ++u) {
+            const int e = we + 256 * u, r = e / (CT_KC / WV);
+            float *d = wl + r * CT_P + WV * (e % (CT_KC / WV));
             if constexpr (sizeof(TW) == 4) {
-                if (I - c >= 4) {
-                    const float p0 = xr[c] * wr[c], p1 = xr[c + 1] * wr[c + 1];
-                    const float p2 = xr[c + 2] * wr[c + 2], p3 = xr[c + 3] * wr[c + 3];
-                    a = a + p0; a = a + p1; a = a + p2; a = a + p3;
-                    c += 4;
+                *reinterpret_cast<pk_f32x4 *>(d) = st.w[u];
+            } else if (tid == we) {
+                ch_put_i8(d, __builtin_bit_cast(uint4, st.w[u]));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < XN; ++u) {
+            const int e = tid + 256 * u;
+            *reinterpret_cast<pk_f32x4 *>(xl + e / (CT_KC / 4) * CT_P + 4 * (e % (CT_KC / 4))) = st.x[u];
+        }
+    };
+    f32x32 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int k = 0; k < 32; ++k) acc[i][k] = 0.0f;
+    const int r = lane & 31, b = lane >> 5;
+    stage st[2];
+    if (chunks > 0) {
+        load(st[0], 0);
+        load(st[1], min(1, chunks - 1) * CT_KC);
+    }
+    for (int n = 0; n < chunks; n += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (n + u < chunks) {
+                float *wl = lds + u * BUF, *xl = wl + CT_TILE * CT_P;
+                store(st[u], wl, xl);
+                load(st[u], min(n + u + 2, chunks - 1) * CT_KC);
+                __syncthreads();
+                const int steps = min(CT_KC, I8 - (n + u) * CT_KC) / 8;
+                const float *wp = wl + (32 * p + r) * CT_P + 4 * b, *xp = xl + (32 * q + r) * CT_P + 4 * b;
+#pragma unroll
+                for (int k = 0; k < CT_KC / 8; ++k) {
+                    if (k < steps) {
+                        const float4 w = *reinterpret_cast<const float4 *>(wp + 8 * k);
+                        const float4 x = *reinterpret_cast<const float4 *>(xp + 8 * k);
+                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.x, w.x, acc[0], 0, 0, 0);
+                        acc[1] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.y, w.y, acc[1], 0, 0, 0);
+                        acc[2] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.z, w.z, acc[2], 0, 0, 0);
+                        acc[3] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.w, w.w, acc[3], 0, 0, 0);
+                    }
                 }
             }
-            for (; c < I; ++c) a = __builtin_fmaf(xr[c], (float)wr[c], a);
-            if (rscale) a = a * rscale[o];
-            if (bias) a = a + bias[o];
-            float *y = out + (int64_t)s * ldo + o;
-            *y = add_res ? *y + a : a;
         }
+    }
+    // registers k / 16 + k: block k / 16 (chains i, 4 + i), input row
+    // 8 (k % 16 / 4) + 4 b + k % 4, output r
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const float b0 = acc[0][k] + acc[0][16 + k], b1 = acc[1][k] + acc[1][16 + k];
+        const float b2 = acc[2][k] + acc[2][16 + k], b3 = acc[3][k] + acc[3][16 + k];
+        ch_finish(X, ldx, W, rscale, bias, out, ldo, S, I, O, add_res, (b0 + b2) + (b1 + b3),
+                  s0 + 32 * q + 8 * (k >> 2) + 4 * b + (k & 3), o0 + 32 * p + r);
     }
 }
 
@@ -360,29 +590,60 @@ __global__ __launch_bounds__(128) void k_router_seq4(const float *__restrict__ X
 
 }  // namespace
 
-int pk_launch_gemm_chain8(const float *X, int64_t ldx, const float *W, const float *bias, float *out, int64_t ldo,
-                          int S, int I, int O, bool add_res, hipStream_t st) {
+// 64 x 64 tiles from about 5 for 8 CUs (a tile's serial columns take ~95 us
+// however few there are; 5120 x 2880: 128 rows 95 against 105 us in 16-row
+// tiles, 512 rows 183 against 367, 64 rows 55 in 16-row tiles); else 16-row
+// tiles, one or two rows on v_fma.
+template <typename TW>
+static int launch_chain8(const float *X, int64_t ldx, const TW *W, const float *rscale, const float *bias, float *out,
+                         int64_t ldo, int S, int I, int O, bool add_res, hipStream_t st) {
     PK_CHECK(S > 0 && I > 0 && O > 0, PK_ERR_ARG, "gemm chain8: bad shape");
-    PK_CHECK((S + CH_ROWS - 1) / CH_ROWS <= 65535, PK_ERR_UNSUPPORTED, "gemm chain8: %d rows", S);
-    const bool vec = (ldx & 3) == 0 && (I & 3) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
-    if (vec)
-        hipLaunchKernelGGL((k_gemm_chain8<float, true>), dim3((O + CH_OUTS - 1) / CH_OUTS, (S + CH_ROWS - 1) / CH_ROWS),
-                           dim3(256), 0, st, X, ldx, W, nullptr, bias, out, ldo, S, I, O, add_res ? 1 : 0);
-    else
-        hipLaunchKernelGGL((k_gemm_chain8<float, false>), dim3((O + CH_OUTS - 1) / CH_OUTS, (S + CH_ROWS - 1) / CH_ROWS),
-                           dim3(256), 0, st, X, ldx, W, nullptr, bias, out, ldo, S, I, O, add_res ? 1 : 0);
+    PK_CHECK((S + 63) / 64 <= CH_MAX_Y, PK_ERR_UNSUPPORTED, "gemm chain8: %d rows", S);
+    const bool vec = (ldx & 3) == 0 && I % (16 / (int)sizeof(TW)) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
+    const int64_t ot = (O + CT_TILE - 1) / CT_TILE, rt = (S + CT_TILE - 1) / CT_TILE;
+    if (vec && S > 32 && 8 * ot * rt >= 5 * (int64_t)pk_device_cus()) {
+        hipLaunchKernelGGL(k_gemm_chain8_tile<TW>, dim3((unsigned)ot, (unsigned)rt), dim3(256), 0, st, X, ldx, W,
+                           rscale, bias, out, ldo, S, I, O, add_res ? 1 : 0);
+        PK_HIP(hipGetLastError());
+        return PK_OK;
+    }
+    const int tiles = S <= 2 ? 1 : (S + 15) / 16;
+    const dim3 grid((O + CH_OUTS - 1) / CH_OUTS, std::min(tiles, CH_MAX_Y), (tiles + CH_MAX_Y - 1) / CH_MAX_Y);
+#define PK_CH8(V, M, N)                                                                                             \
+    hipLaunchKernelGGL((k_gemm_chain8<TW, V, M, N>), grid, dim3(CH_THREADS), 0, st, X, ldx, W, rscale, bias, out, ldo, \
+                       S, I, O, add_res ? 1 : 0)
+    if (S == 1) {
+        if (vec) PK_CH8(true, false, 1); else PK_CH8(false, false, 1);
+    } else if (S == 2) {
+        if (vec) PK_CH8(true, false, 2); else PK_CH8(false, false, 2);
+    } else {
+        if (vec) PK_CH8(true, true, 0); else PK_CH8(false, true, 0);
+    }
+#undef PK_CH8
     PK_HIP(hipGetLastError());
     return PK_OK;
+}
+
+int pk_launch_gemm_chain8(const float *X, int64_t ldx, const float *W, const float *bias, float *out, int64_t ldo,
+                          int S, int I, int O, bool add_res, hipStream_t st) {
+    return launch_chain8<float>(X, ldx, W, nullptr, bias, out, ldo, S, I, O, add_res, st);
 }
 
 int pk_launch_gemm_chain8_q8(const float *X, const int8_t *W, const float *scale, float *out, int S, int I, int O,
                              hipStream_t st) {
     PK_CHECK(S > 0 && I > 0 && O > 0 && scale, PK_ERR_ARG, "gemm chain8 q8: bad argument");
-    PK_CHECK((S + CH_ROWS - 1) / CH_ROWS <= 65535, PK_ERR_UNSUPPORTED, "gemm chain8: %d rows", S);
-    hipLaunchKernelGGL((k_gemm_chain8<int8_t, false>), dim3((O + CH_OUTS - 1) / CH_OUTS, (S + CH_ROWS - 1) / CH_ROWS),
-                       dim3(256), 0, st, X, (int64_t)I, W, scale, nullptr, out, (int64_t)O, S, I, O, 0);
-    PK_HIP(hipGetLastError());
-    return PK_OK;
+    // a wave per 64 outputs, once that gives every SIMD a wave (16,000 outputs,
+    // 250 waves: 32 against 23 us in k_gemm_chain8)
+    if (S <= 4 && (I & 15) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0 &&
+        (O + 63) / 64 >= 4 * pk_device_cus()) {
+        const dim3 grid((O + 63) / 64);
+        if (S == 1) hipLaunchKernelGGL(k_gemv_chain8_q8<1>, grid, dim3(64), 0, st, X, W, scale, out, S, I, O);
+        else if (S == 2) hipLaunchKernelGGL(k_gemv_chain8_q8<2>, grid, dim3(64), 0, st, X, W, scale, out, S, I, O);
+        else hipLaunchKernelGGL(k_gemv_chain8_q8<4>, grid, dim3(64), 0, st, X, W, scale, out, S, I, O);
+        PK_HIP(hipGetLastError());
+        return PK_OK;
+    }
+    return launch_chain8<int8_t>(X, I, W, scale, nullptr, out, O, S, I, O, false, st);
 }
 
 int pk_launch_attn_rows_exact(int pos_base, int n, const float *qkv, int64_t qkv_stride, const float *Kl,
