@@ -1025,7 +1025,7 @@ int pk_attention_rows(pk_engine *e, int l, const pk_dstate *st, int pos_base, in
         const int last = pos_base + n - 1;
         int span = (last < c->ctx_len ? last : c->ctx_len - 1) + 1;
         if (sliding && span > c->sliding_window) span = c->sliding_window;
-        if (span <= 16384) {
+        if (span <= PK_ATT_EXACT_SPAN) {
             PK_TRY(pk_launch_attn_rows_exact(pos_base, n, qkv, qkv_dim, Kl, Vl, H, KVH, hd, c->ctx_len, sliding,
                                              c->sliding_window, d.sinks, att, e->stream));
             PK_TRY(pk_launch_gemm_chain8(att, (int64_t)H * hd, d.wo, d.bo, h, D, n, H * hd, D, true, e->stream));

@@ -151,6 +151,7 @@ struct pk_engine {
     bool dot_tiles_off = false;                   // PK_DOT_TILES=0: one launch item per pair
     // prompt-chunk scratch for up to p_cap positions (pk_prefill.hip)
     int p_cap = 0;
+    int p_part_cap = 0;                       // rows of p_part
     float *p_H = nullptr, *p_XN = nullptr, *p_qkv = nullptr, *p_att = nullptr, *p_part = nullptr;
     int32_t *p_ids = nullptr;
     // batched decode (pk_decode_batch): logits [n_seq][vocab], token ring
@@ -266,6 +267,7 @@ int pk_launch_gemm_chain8(const float *X, int64_t ldx, const float *W, const flo
                           int S, int I, int O, bool add_res, hipStream_t st);
 int pk_launch_gemm_chain8_q8(const float *X, const int8_t *W, const float *scale, float *out, int S, int I, int O,
                              hipStream_t st);
+constexpr int PK_ATT_EXACT_SPAN = 16384;      // positions of a window that its LDS holds
 int pk_launch_attn_rows_exact(int pos_base, int n, const float *qkv, int64_t qkv_stride, const float *Kl,
                               const float *Vl, int H, int KVH, int hd, int ctx, int sliding, int window,
                               const float *sinks, float *att, hipStream_t st);

@@ -505,87 +505,93 @@ __global__ __launch_bounds__(128) void k_router_seq(const float *__restrict__ X,
     if (live) logits[(int64_t)s * E + e] = acc;
 }
 
-// The same sums with 16-byte loads (D % 4 == 0, aligned rows; 4 <= E <= 128):
-// the next 64 columns of the router rows and of the block's input rows load
-// into registers (at most 20 per thread, so that the load counter can wait
-// for them in order) while the current ones are multiplied; in LDS each
-// router row's chunk is contiguous, so a thread reads its 64 weights and
-// its row's 64 inputs as float4, 32 at a time, before the dependent adds.
+// The same sums with 16-byte loads (D % 4 == 0, aligned rows): one wave per
+// block of EB experts and 64 / EB rows, lane t taking expert t % EB of row t /
+// EB. What bounds it is the chain of dependent adds (2880 x 1.6 ns, each
+// after its product) and the latency of the router rows: a 64-column chunk is
+// multiplied in ~0.3 us, so RQ_PF chunks' loads are in flight in registers.
+// A chunk passes through the wave's own LDS (rows 4 mod 64 floats apart, read
+// as float4): several waves of one workgroup would share the loads but are
+// bound by their LDS reads. 64 rows x 32 experts x 2880: 35 us; 38 with four
+// waves per workgroup, 70 with two and one chunk in flight.
 constexpr int RQ_P = RS_KC + 4;          // padded LDS row (floats)
-__global__ __launch_bounds__(128) void k_router_seq4(const float *__restrict__ X, const float *__restrict__ R,
-                                                     const float *__restrict__ bias, int S, int D, int E,
-                                                     float *logits) {
-    extern __shared__ float lds_rs[];
-    const int rows = 128 / E;
-    float *wt = lds_rs;                   // [E][RQ_P]
-    float *xt = lds_rs + E * RQ_P;        // [rows][RQ_P]
-    const int tid = threadIdx.x;
-    const int e = tid % E, rr = tid / E;
-    const int s = blockIdx.x * rows + rr;
-    const bool live = rr < rows && s < S;
-    float acc = live ? bias[e] : 0.0f;
-    constexpr int WN = 16, XN = 4;        // float4 per thread: E * 16 / 128 and rows * 16 / 128
-    const int nw4 = E * (RS_KC / 4), nx4 = rows * (RS_KC / 4);
-    float4 wv[WN], xv[XN];
-    auto load = [&](int c0) {
-        const int nc4 = min(RS_KC, D - c0) / 4;
+constexpr int RQ_PF = 4;                 // chunks in flight
+template <int EB>
+__global__ __launch_bounds__(64) void k_router_seq4(const float *__restrict__ X, const float *__restrict__ R,
+                                                    const float *__restrict__ bias, int S, int D, int E,
+                                                    float *logits) {
+    constexpr int ROWS = 64 / EB, C4 = RS_KC / 4;
+    constexpr int WN = EB * C4 / 64, XN = (ROWS * C4 + 63) / 64;     // 16-byte loads per lane and chunk
+    __shared__ __attribute__((aligned(16))) float lds[2][(EB + ROWS) * RQ_P];
+    const int lane = threadIdx.x;
+    const int e0 = blockIdx.y * EB, s0 = blockIdx.x * ROWS;
+    const int e = e0 + lane % EB, s = s0 + lane / EB;
+    float acc = bias[min(e, E - 1)];
+    const int chunks = (D + RS_KC - 1) / RS_KC;
+    struct stage {
+        pk_f32x4 w[WN], x[XN];
+    };
+    // (rows and columns past the end repeat the last ones; they are not used)
+    auto load = [&](stage &st, int n) {
+        const int c0 = min(n, chunks - 1) * RS_KC, last = min(RS_KC, D - c0) / 4 - 1;
 #pragma unroll
         for (int u = 0; u < WN; ++u) {
-            const int q = min(tid + 128 * u, nw4 - 1), ee = q / (RS_KC / 4), c4 = q - ee * (RS_KC / 4);
-            const float4 v = *reinterpret_cast<const float4 *>(R + (int64_t)ee * D + c0 + 4 * min(c4, nc4 - 1));
-            wv[u] = c4 < nc4 ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+            const int q = lane + 64 * u;
+            st.w[u] = *reinterpret_cast<const pk_f32x4 *>(R + (int64_t)min(e0 + q / C4, E - 1) * D + c0 +
+                                                          4 * min(q % C4, last));
         }
 #pragma unroll
         for (int u = 0; u < XN; ++u) {
-            const int q = min(tid + 128 * u, nx4 - 1), r2 = q / (RS_KC / 4), c4 = q - r2 * (RS_KC / 4);
-            const int s2 = min(blockIdx.x * rows + r2, S - 1);
-            const float4 v = *reinterpret_cast<const float4 *>(X + (int64_t)s2 * D + c0 + 4 * min(c4, nc4 - 1));
-            xv[u] = c4 < nc4 ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+            const int q = min(lane + 64 * u, ROWS * C4 - 1);
+            st.x[u] = *reinterpret_cast<const pk_f32x4 *>(X + (int64_t)min(s0 + q / C4, S - 1) * D + c0 +
+                                                          4 * min(q % C4, last));
         }
     };
-    load(0);
+    stage st[RQ_PF];
+#pragma unroll
+    for (int u = 0; u < RQ_PF; ++u) load(st[u], u);
     // (the bias is waited for here: inside the loop the compiler would wait
     // for every outstanding load before the first add)
     asm volatile("" ::"v"(acc));
-    for (int c0 = 0; c0 < D; c0 += RS_KC) {
-        const int nc = min(RS_KC, D - c0);
-        __syncthreads();                  // the previous chunk's reads are done
+    for (int n0 = 0; n0 < chunks; n0 += RQ_PF) {
 #pragma unroll
-        for (int u = 0; u < WN; ++u) {
-            const int q = tid + 128 * u, ee = q / (RS_KC / 4), c4 = q - ee * (RS_KC / 4);
-            if (q < nw4) *reinterpret_cast<float4 *>(wt + ee * RQ_P + 4 * c4) = wv[u];
-        }
+        for (int v = 0; v < RQ_PF; ++v) {
+            const int n = n0 + v;
+            if (n < chunks) {
+                float *wt = lds[v & 1], *xt = wt + EB * RQ_P;
 #pragma unroll
-        for (int u = 0; u < XN; ++u) {
-            const int q = tid + 128 * u, r2 = q / (RS_KC / 4), c4 = q - r2 * (RS_KC / 4);
-            if (q < nx4) *reinterpret_cast<float4 *>(xt + r2 * RQ_P + 4 * c4) = xv[u];
-        }
-        __syncthreads();
-        if (c0 + RS_KC < D) load(c0 + RS_KC);
-        if (live) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                float4 xa[8], wa[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    xa[j] = *reinterpret_cast<const float4 *>(xt + rr * RQ_P + 32 * h + 4 * j);
-                    wa[j] = *reinterpret_cast<const float4 *>(wt + e * RQ_P + 32 * h + 4 * j);
+                for (int u = 0; u < WN; ++u) {
+                    const int q = lane + 64 * u;
+                    *reinterpret_cast<pk_f32x4 *>(wt + q / C4 * RQ_P + 4 * (q % C4)) = st[v].w[u];
                 }
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float xs[4] = {xa[j].x, xa[j].y, xa[j].z, xa[j].w};
-                    const float ws[4] = {wa[j].x, wa[j].y, wa[j].z, wa[j].w};
+                for (int u = 0; u < XN; ++u) {
+                    const int q = lane + 64 * u;
+                    if (q < ROWS * C4) *reinterpret_cast<pk_f32x4 *>(xt + q / C4 * RQ_P + 4 * (q % C4)) = st[v].x[u];
+                }
+                load(st[v], n + RQ_PF);
+                __syncthreads();                  // (one wave: orders the LDS writes and reads)
+                const int nc4 = min(RS_KC, D - n * RS_KC) / 4;
+                const float *wp = wt + lane % EB * RQ_P, *xp = xt + lane / EB * RQ_P;
+                auto add4 = [&](int j) {
+                    const pk_f32x4 w = *reinterpret_cast<const pk_f32x4 *>(wp + 4 * j);
+                    const pk_f32x4 x = *reinterpret_cast<const pk_f32x4 *>(xp + 4 * j);
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if (32 * h + 4 * j + k < nc) {
-                            const float p = xs[k] * ws[k];
-                            acc = acc + p;
-                        }
+                    for (int k = 0; k < 4; ++k) {
+                        const float p = x[k] * w[k];
+                        acc = acc + p;
+                    }
+                };
+                if (nc4 == C4) {
+#pragma unroll
+                    for (int j = 0; j < C4; ++j) add4(j);
+                } else {
+                    for (int j = 0; j < nc4; ++j) add4(j);
                 }
             }
         }
     }
-    if (live) logits[(int64_t)s * E + e] = acc;
+    if (e < E && s < S) logits[(int64_t)s * E + e] = acc;
 }
 
 }  // namespace
@@ -663,11 +669,12 @@ int pk_launch_attn_rows_exact(int pos_base, int n, const float *qkv, int64_t qkv
 int pk_launch_router_seq(const float *X, const float *R, const float *bias, int S, int D, int E, float *logits,
                          hipStream_t st) {
     PK_CHECK(S > 0 && D > 0 && E > 0 && E <= 128, PK_ERR_ARG, "router: bad shape");
-    if (E >= 4 && (D & 3) == 0 && (((uintptr_t)X | (uintptr_t)R) & 15) == 0) {
-        const int rows = 128 / E;
-        const size_t lds = ((size_t)E + rows) * RQ_P * 4;
-        hipLaunchKernelGGL(k_router_seq4, dim3((S + rows - 1) / rows), dim3(128), lds, st, X, R, bias, S, D, E,
-                           logits);
+    if ((D & 3) == 0 && (((uintptr_t)X | (uintptr_t)R) & 15) == 0) {
+        if (E <= 8)
+            hipLaunchKernelGGL(k_router_seq4<8>, dim3((S + 7) / 8), dim3(64), 0, st, X, R, bias, S, D, E, logits);
+        else
+            hipLaunchKernelGGL(k_router_seq4<32>, dim3((S + 1) / 2, (E + 31) / 32), dim3(64), 0, st, X, R, bias, S, D,
+                               E, logits);
         PK_HIP(hipGetLastError());
         return PK_OK;
     }

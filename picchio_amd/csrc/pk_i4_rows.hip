@@ -129,6 +129,24 @@ __device__ __forceinline__ void rw_group(const rw_stage<NS> &st, f32x4 (&p)[NS])
         }
 }
 
+// Results of input rows j (v0) and j + 1 (v1) of the tile at weight row
+// `row`: the SwiGLU of two input rows at once (even lanes finish the first's
+// pair of rows (row, row + 1), odd lanes the second's), or both values.
+template <int EPI, typename PAIR>
+__device__ __forceinline__ void rw_put2(const pk_i4_items &it, PAIR pair_of, int j, int cnt, int row, int O, float v0,
+                                        float v1, float lim, float alpha) {
+    if constexpr (EPI == PK_EPI_SWIGLU) {
+        const bool even = (row & 1) == 0;
+        const float other = __shfl_xor(even ? v1 : v0, 1, 64);
+        const float v = pk_swiglu(even ? v0 : other, even ? other : v1, lim, alpha);
+        const int jj = even ? j : j + 1;
+        if (jj < cnt && (row | 1) < O) it.y[(int64_t)pair_of(jj) * it.y_stride + (row >> 1)] = v;
+    } else if (row < O) {
+        if (j < cnt) it.y[(int64_t)pair_of(j) * it.y_stride + row] = v0;
+        if (j + 1 < cnt) it.y[(int64_t)pair_of(j + 1) * it.y_stride + row] = v1;
+    }
+}
+
 template <int NS, int EPI>
 __device__ __forceinline__ void rw_body(const pk_i4_items &it, const int32_t *pairs, int beg, int cnt,
                                         const uint8_t *base, int rb, int O, int NG, float lim, float alpha,
@@ -202,18 +220,7 @@ __device__ __forceinline__ void rw_body(const pk_i4_items &it, const int32_t *pa
     if (j >= cnt) return;
     float a0 = accs[j][lane], a1 = accs[j + 1][lane];
     if (it.off_bias >= 0 && row < O) { a0 = a0 + bias; a1 = a1 + bias; }
-    if constexpr (EPI == PK_EPI_SWIGLU) {
-        // even lanes finish the first input row's (gate, up) pair of matrix
-        // rows (row, row + 1), odd lanes the second's
-        const bool even = (lane & 1) == 0;
-        const float other = __shfl_xor(even ? a1 : a0, 1, 64);
-        const float v = pk_swiglu(even ? a0 : other, even ? other : a1, lim, alpha);
-        const int jj = even ? j : j + 1;
-        if (jj < cnt && (row | 1) < O) it.y[(int64_t)pair_of(jj) * it.y_stride + (row >> 1)] = v;
-    } else if (row < O) {
-        it.y[(int64_t)pair_of(j) * it.y_stride + row] = a0;
-        if (j + 1 < cnt) it.y[(int64_t)pair_of(j + 1) * it.y_stride + row] = a1;
-    }
+    rw_put2<EPI>(it, pair_of, j, cnt, row, O, a0, a1, lim, alpha);
 }
 
 // grid (RB, tiles): workgroup (rb, t) is row block rb of tile t, its waves
@@ -239,6 +246,196 @@ __global__ __launch_bounds__(RW_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2
     else rw_body<1, EPI>(it, tl.pairs, beg, cnt, base, rb, O, NG, lim, alpha, accs);
 }
 
+// ───────────────────── tiles of 16 rows ─────────────────────
+// Many pairs per expert: a wave walks all groups of one row block and folds
+// them as it goes. More than 8 rows of a tile run on
+// v_mfma_f32_16x16x1_4b_f32, its four blocks being the row block's quarters
+// (operand B, lane = weight row) times 16 input rows at one column, broadcast
+// to the blocks (cbsz = 2): 14.2 ns per 64 x 16 products against 15.5 on the
+// 4 x 4 form, and each decode serves 16 rows. Register 4 q + i of lane l is
+// weight row 16 q + l % 16, input row 4 (l / 16) + i.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <int D, int J>
+__device__ __forceinline__ void rw16_column(float q, const float4 (&x)[4], f32x16 (&c)[8]) {
+    constexpr f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    c[J] = __builtin_amdgcn_mfma_f32_16x16x1f32(rw_comp(x[D >> 1], J & 3), q, D == 0 ? zero : c[J], 2,
+                                                2 * (D & 1) + (J >> 2), 0);
+}
+
+template <int D>
+__device__ __forceinline__ void rw16_dword(const float (&q)[8], const float4 (&x)[4], f32x16 (&c)[8]) {
+    rw16_column<D, 0>(q[0], x, c);
+    rw16_column<D, 1>(q[1], x, c);
+    rw16_column<D, 2>(q[2], x, c);
+    rw16_column<D, 3>(q[3], x, c);
+    rw16_column<D, 4>(q[4], x, c);
+    rw16_column<D, 5>(q[5], x, c);
+    rw16_column<D, 6>(q[6], x, c);
+    rw16_column<D, 7>(q[7], x, c);
+}
+
+struct rw16_stage {
+    uint4 wa, wb;
+    float s[4];
+    float4 x[4];
+};
+
+__device__ __forceinline__ void rw16_group(const rw16_stage &st, f32x16 &acc) {
+    f32x16 c[8];
+    float q[4][8];
+    rw_decode(st.wa.x, q[0]);
+    rw_decode(st.wa.y, q[1]);
+    rw_decode(st.wa.z, q[2]);
+    rw_decode(st.wa.w, q[3]);
+    __builtin_amdgcn_sched_barrier(0);
+    rw16_dword<0>(q[0], st.x, c);
+    rw16_dword<1>(q[1], st.x, c);
+    rw16_dword<2>(q[2], st.x, c);
+    rw16_dword<3>(q[3], st.x, c);
+    __builtin_amdgcn_sched_barrier(0);
+    rw_decode(st.wb.x, q[0]);
+    rw_decode(st.wb.y, q[1]);
+    rw_decode(st.wb.z, q[2]);
+    rw_decode(st.wb.w, q[3]);
+    __builtin_amdgcn_sched_barrier(0);
+    rw16_dword<4>(q[0], st.x, c);
+    rw16_dword<5>(q[1], st.x, c);
+    rw16_dword<6>(q[2], st.x, c);
+    rw16_dword<7>(q[3], st.x, c);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const float b0 = c[0][i] + c[4][i], b1 = c[1][i] + c[5][i];
+        const float b2 = c[2][i] + c[6][i], b3 = c[3][i] + c[7][i];
+        acc[i] = __builtin_fmaf((b0 + b2) + (b1 + b3), st.s[i >> 2], acc[i]);
+    }
+}
+
+constexpr int RW16_PF = 2;
+
+template <int EPI>
+__device__ __forceinline__ void rw16_body(const pk_i4_items &it, const int32_t *pairs, int beg, int cnt,
+                                          const uint8_t *base, int rb, int O, int NG, float lim, float alpha) {
+    const int lane = threadIdx.x & 63;
+    const uint4 *tiles =
+        reinterpret_cast<const uint4 *>(base + it.off_tiles) + (int64_t)rb * NG * (PK_TILE_BYTES / 16);
+    const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64;
+    auto pair_of = [&](int j) { return pairs ? pairs[beg + j] : beg + j; };
+    // lane l loads input row l % 16, columns 4 (l / 16) .. + 3 of each 16
+    const float *xp = it.x + (int64_t)(pair_of(min(lane & 15, cnt - 1)) / it.x_div) * it.x_stride + 4 * (lane >> 4);
+    rw16_stage st[RW16_PF];
+    auto load = [&](rw16_stage &d, int g) {
+        d.wa = pk_load_nt(&tiles[g * 128 + lane]);
+        d.wb = pk_load_nt(&tiles[g * 128 + 64 + lane]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d.s[q] = sc[g * 64 + 16 * q + (lane & 15)];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) d.x[m] = *reinterpret_cast<const float4 *>(xp + g * 64 + 16 * m);
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+    for (int u = 0; u < RW16_PF; ++u) load(st[u], min(u, NG - 1));
+    for (int g = 0; g < NG; g += RW16_PF) {
+#pragma unroll
+        for (int u = 0; u < RW16_PF; ++u) {
+            if (g + u < NG) rw16_group(st[u], acc);
+            load(st[u], min(g + u + RW16_PF, NG - 1));
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int row = rb * 64 + 16 * q + (lane & 15);
+        if (it.off_bias >= 0 && row < O) {
+            const float bias = reinterpret_cast<const float *>(base + it.off_bias)[row];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[4 * q + i] = acc[4 * q + i] + bias;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i += 2)
+            rw_put2<EPI>(it, pair_of, 4 * (lane >> 4) + i, cnt, row, O, acc[4 * q + i], acc[4 * q + i + 1], lim, alpha);
+    }
+}
+
+// The same walk for up to 8 rows on the 4 x 4 form.
+template <int NS, int EPI>
+__device__ __forceinline__ void rw_walk(const pk_i4_items &it, const int32_t *pairs, int beg, int cnt,
+                                        const uint8_t *base, int rb, int O, int NG, float lim, float alpha) {
+    const int lane = threadIdx.x & 63;
+    const uint4 *tiles =
+        reinterpret_cast<const uint4 *>(base + it.off_tiles) + (int64_t)rb * NG * (PK_TILE_BYTES / 16);
+    const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64;
+    auto pair_of = [&](int j) { return pairs ? pairs[beg + j] : beg + j; };
+    const float *xp[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+        xp[s] = it.x + (int64_t)(pair_of(min(4 * s + (lane & 3), cnt - 1)) / it.x_div) * it.x_stride + 4 * (lane >> 2);
+    rw_stage<NS> st[RW16_PF];
+    auto load = [&](rw_stage<NS> &d, int g) {
+        d.wa = pk_load_nt(&tiles[g * 128 + lane]);
+        d.wb = pk_load_nt(&tiles[g * 128 + 64 + lane]);
+        d.s = sc[g * 64 + lane];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) d.x[s] = *reinterpret_cast<const float4 *>(xp[s] + g * 64);
+    };
+    f32x4 acc[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < RW16_PF; ++u) load(st[u], min(u, NG - 1));
+    for (int g = 0; g < NG; g += RW16_PF) {
+#pragma unroll
+        for (int u = 0; u < RW16_PF; ++u) {
+            if (g + u < NG) {
+                f32x4 p[NS];
+                rw_group<NS>(st[u], p);
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[s][i] = __builtin_fmaf(p[s][i], st[u].s, acc[s][i]);
+            }
+            load(st[u], min(g + u + RW16_PF, NG - 1));
+        }
+    }
+    const int row = rb * 64 + lane;
+    const float bias = it.off_bias >= 0 && row < O ? reinterpret_cast<const float *>(base + it.off_bias)[row] : 0.0f;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        if (it.off_bias >= 0 && row < O) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[s][i] = acc[s][i] + bias;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i += 2)
+            rw_put2<EPI>(it, pair_of, 4 * s + i, cnt, row, O, acc[s][i], acc[s][i + 1], lim, alpha);
+    }
+}
+
+// grid (ceil(RB / 4), tiles): wave w of a workgroup takes row block 4 x + w of
+// tile y (at most 16 rows).
+template <int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_i4_rows16(
+    pk_i4_items it, pk_i4_tiles tl, int O, int NG, int RB, float lim, float alpha) {
+    const int rb = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.y;
+    if (rb >= RB) return;
+    int beg, cnt, slot = it.slot_base;
+    if (tl.pairs) {
+        if (t >= *tl.n_tiles) return;
+        beg = tl.tile_beg[t];
+        cnt = tl.tile_cnt[t];
+        slot += tl.tile_exp[t];
+    } else {
+        beg = t * 16;
+        cnt = min(16, it.n_items - beg);
+    }
+    const uint8_t *base = it.base + (int64_t)slot * it.slot_stride;
+    if (cnt > 8) rw16_body<EPI>(it, tl.pairs, beg, cnt, base, rb, O, NG, lim, alpha);
+    else if (cnt > 4) rw_walk<2, EPI>(it, tl.pairs, beg, cnt, base, rb, O, NG, lim, alpha);
+    else rw_walk<1, EPI>(it, tl.pairs, beg, cnt, base, rb, O, NG, lim, alpha);
+}
+
 }  // namespace
 
 bool pk_i4_rows_ok(const pk_i4_items &it, int epilogue) {
@@ -246,18 +443,30 @@ bool pk_i4_rows_ok(const pk_i4_items &it, int epilogue) {
 }
 
 int pk_launch_i4_rows(const pk_i4_items &it, const pk_i4_tiles *tl, const pk_i4_shape &sh, int epilogue, float lim,
-                      float alpha, int max_tiles, hipStream_t st) {
+                      float alpha, int max_tiles, hipStream_t st, int tile_rows) {
     PK_CHECK(pk_i4_rows_ok(it, epilogue), PK_ERR_ARG, "i4 rows: inputs not 16-byte aligned, or not the fp32 chains");
     PK_CHECK(sh.NG > 0 && sh.RB > 0 && it.n_items > 0 && it.x_div > 0, PK_ERR_ARG, "i4 rows: empty shape");
     PK_CHECK(!tl || (tl->pairs && tl->tile_exp && tl->tile_beg && tl->tile_cnt && tl->n_tiles), PK_ERR_ARG,
              "i4 rows: missing tiles");
+    PK_CHECK(tile_rows == 8 || tile_rows == 16, PK_ERR_ARG, "i4 rows: tiles of %d", tile_rows);
     // one matrix: tiles of 8 rows, but of 4 where tiles of 8 would leave CUs
     // without a workgroup (5760 x 2880, 8 rows: 9.5 against 13.6 us)
-    int tile = RW_M;
-    if (!tl && (int64_t)sh.RB * ((it.n_items + RW_M - 1) / RW_M) <= pk_device_cus()) tile = 4;
+    int tile = tile_rows;
+    if (!tl && tile == 8 && (int64_t)sh.RB * ((it.n_items + 7) / 8) <= pk_device_cus()) tile = 4;
     const int tiles = tl ? max_tiles : (it.n_items + tile - 1) / tile;
     PK_CHECK(tiles > 0 && tiles <= 65535, PK_ERR_UNSUPPORTED, "i4 rows: %d tiles", tiles);
     const pk_i4_tiles none{};
+    if (tile == 16) {
+        const dim3 grid((sh.RB + 3) / 4, tiles);
+        if (epilogue == PK_EPI_SWIGLU)
+            hipLaunchKernelGGL(k_i4_rows16<PK_EPI_SWIGLU>, grid, dim3(256), 0, st, it, tl ? *tl : none, sh.O, sh.NG,
+                               sh.RB, lim, alpha);
+        else
+            hipLaunchKernelGGL(k_i4_rows16<PK_EPI_PLAIN>, grid, dim3(256), 0, st, it, tl ? *tl : none, sh.O, sh.NG,
+                               sh.RB, lim, alpha);
+        PK_HIP(hipGetLastError());
+        return PK_OK;
+    }
     const dim3 grid(sh.RB, tiles);
     if (epilogue == PK_EPI_SWIGLU)
         hipLaunchKernelGGL(k_i4_rows<PK_EPI_SWIGLU>, grid, dim3(RW_WAVES * 64), 0, st, it, tl ? *tl : none, tile, sh.O,

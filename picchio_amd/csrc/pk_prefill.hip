@@ -32,12 +32,17 @@ __global__ __launch_bounds__(256) void k_embed_rows(const int32_t *ids, const fl
 // forward_prefill's expert order (picchio.c:1846-1852, :1885-1902): experts are
 // ranked by first request, scanning positions, then k; each token adds its
 // experts in rank order. perm[p][j] = k of the token's j-th expert. One
-// workgroup: first request of each expert by atomic min, rank = number of
-// experts requested earlier, then each token orders its k by rank.
+// workgroup per chunk of `chunk` tokens (each with its own ranks): first
+// request of each expert by atomic min, rank = number of experts requested
+// earlier, then each token orders its k by rank.
 constexpr int UP_LDS = 16384;           // routing entries staged in LDS (all loads in flight at once)
-__global__ __launch_bounds__(1024) void k_uniq_perm(const int32_t *sel, int n, int K, int E, int32_t *perm) {
+__global__ __launch_bounds__(1024) void k_uniq_perm(const int32_t *sel, int n, int K, int E, int32_t *perm,
+                                                   int chunk) {
     __shared__ int first[128], rank[128];
     __shared__ int s_sel[UP_LDS];
+    sel += (int64_t)blockIdx.x * chunk * K;
+    perm += (int64_t)blockIdx.x * chunk * K;
+    n = min(chunk, n - (int)blockIdx.x * chunk);
     const int P = n * K;
     const bool staged = P <= UP_LDS && (int)blockDim.x * 16 >= UP_LDS;
     for (int e = threadIdx.x; e < E; e += blockDim.x) first[e] = 0x7fffffff;
@@ -220,14 +225,19 @@ static int route_rows(pk_engine *e, const rows_scratch &sc, int layer, const flo
 // (20B layer, 3 tokens 135.6 us either way, 6 tokens 164 against 158 us; 128
 // experts, 3 tokens 142 against 149).
 constexpr int ROWS_MIN_PAIRS = 24;
+// Pairs per expert from which the tiles hold 16 rows instead of 8 (32
+// experts: 128 tokens 455 against 428 us, 256 tokens 740 against 746, 512
+// tokens 1252 against 1350).
+constexpr int ROWS16_PAIRS = 32;
 
 // The MoE of forward_prefill (picchio.c:1829-1916) for T tokens x [T][D]:
 // out[t] = (residual ? residual[t] : 0) + sum over the token's experts, in the
 // batch's expert order, of (w_k * routed_scale) * expert_k(x[t]). With
 // decode_order the sum runs in routing order instead, as moe_forward adds
-// (picchio.c:1445-1454): T independent decode tokens.
+// (picchio.c:1445-1454): T independent decode tokens. chunk: the T rows are
+// consecutive batches of that many tokens, each with its own expert order.
 static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const float *x, int T, float *out,
-                       const float *residual, bool decode_order) {
+                       const float *residual, bool decode_order, int chunk) {
     const pk_cfg *c = &e->c;
     const int D = c->hidden, E = c->n_experts, K = c->topk, half = c->moe_inter / 2;
     // the integer-dot option: records of the token rows (written by the top-k
@@ -237,7 +247,8 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
     const int64_t xq_row = (int64_t)(D / 32) * PK_XQ_INTS, aq_row = (int64_t)e->ex.gu.RB * PK_XQ_INTS;
     PK_TRY(route_rows(e, sc, layer, x, T, !decode_order, dot ? sc.xq : nullptr));
     if (!decode_order) {
-        hipLaunchKernelGGL(k_uniq_perm, dim3(1), dim3(1024), 0, e->stream, sc.sel, T, K, E, sc.perm);
+        hipLaunchKernelGGL(k_uniq_perm, dim3((T + chunk - 1) / chunk), dim3(1024), 0, e->stream, sc.sel, T, K, E,
+                           sc.perm, chunk);
         PK_HIP(hipGetLastError());
     }
     pk_i4_items gu = pk_expert_items(e, layer, false);
@@ -257,7 +268,7 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
     pk_i4_tiles tl{sc.pairs, sc.tiles, sc.tiles + mt, sc.tiles + 2 * mt, sc.tiles + 3 * mt};
     const bool tiled = dot && !e->dot_tiles_off && e->ex.gu.NG <= 64 && e->ex.dn.NG <= 64 && E <= 128;
     const bool rows = !dot && E <= 128 && P >= ROWS_MIN_PAIRS && pk_i4_rows_ok(gu, PK_EPI_SWIGLU);
-    const int tile = tiled ? 4 : PK_ROWS_TILE, max_tiles = P / tile + 1 + E;
+    const int tile = tiled ? 4 : P >= ROWS16_PAIRS * E ? 16 : PK_ROWS_TILE, max_tiles = P / tile + 1 + E;
     if (tiled || rows)
         PK_TRY(pk_launch_group_pairs(sc.sel, P, E, sc.pairs, sc.tiles, sc.tiles + mt,
                                      sc.tiles + 2 * mt, sc.tiles + 3 * mt, e->stream, tile));
@@ -267,7 +278,7 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
                                       e->stream));
     else if (rows)
         PK_TRY(pk_launch_i4_rows(gu, &tl, e->ex.gu, PK_EPI_SWIGLU, c->swiglu_limit, c->swiglu_alpha, max_tiles,
-                                 e->stream));
+                                 e->stream, tile));
     else
         PK_TRY(pk_launch_i4_gemv(gu, e->ex.gu, PK_EPI_SWIGLU, c->swiglu_limit, c->swiglu_alpha, nullptr,
                                  e->stream));
@@ -284,7 +295,7 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
     if (tiled)
         PK_TRY(pk_launch_i4_dot_tiles(dn, tl, e->ex.dn, PK_EPI_PLAIN, 0.f, 0.f, max_tiles, e->stream));
     else if (rows)
-        PK_TRY(pk_launch_i4_rows(dn, &tl, e->ex.dn, PK_EPI_PLAIN, 0.f, 0.f, max_tiles, e->stream));
+        PK_TRY(pk_launch_i4_rows(dn, &tl, e->ex.dn, PK_EPI_PLAIN, 0.f, 0.f, max_tiles, e->stream, tile));
     else
         PK_TRY(pk_launch_i4_gemv(dn, e->ex.dn, PK_EPI_PLAIN, 0.f, 0.f, nullptr, e->stream));
     PK_TRY(pk_prof_end(e, ps));
@@ -292,9 +303,9 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
 }
 
 static int moe_rows(pk_engine *e, int layer, const float *x, int T, float *out, const float *residual,
-                    bool decode_order = false) {
+                    bool decode_order = false, int chunk = 0) {
     PK_TRY(batch_reserve(e, T));
-    return moe_rows_on(e, engine_rows_scratch(e), layer, x, T, out, residual, decode_order);
+    return moe_rows_on(e, engine_rows_scratch(e), layer, x, T, out, residual, decode_order, chunk > 0 ? chunk : T);
 }
 
 static int grouped_reserve(pk_engine *e, int T) {
@@ -338,7 +349,7 @@ static int moe_rows_mfma(pk_engine *e, int layer, const float *x, int T, float *
         PK_TRY(route_rows(e, engine_rows_scratch(e), layer, x, T, !decode_order));
     }
     if (!decode_order) {
-        hipLaunchKernelGGL(k_uniq_perm, dim3(1), dim3(1024), 0, e->stream, e->b_sel, T, K, E, e->b_perm);
+        hipLaunchKernelGGL(k_uniq_perm, dim3(1), dim3(1024), 0, e->stream, e->b_sel, T, K, E, e->b_perm, T);
         PK_HIP(hipGetLastError());
     }
     const bool f16 = e->grouped_f16;
@@ -485,7 +496,7 @@ extern "C" int pk_moe_forward_batch_noalloc(pk_engine *e, int layer, const float
              "moe_forward_batch_noalloc: %d tokens need %lld bytes of scratch, the fixed array holds %lld", T,
              (long long)need, (long long)PK_NOALLOC_SCRATCH_BYTES);
     rows_scratch_carve(e, T, e->noalloc_scratch, &sc);
-    PK_TRY(moe_rows_on(e, sc, layer, x_dev, T, out_dev, nullptr, false));
+    PK_TRY(moe_rows_on(e, sc, layer, x_dev, T, out_dev, nullptr, false, T));
     const int K = e->c.topk;
     if (sel_dev)
         PK_HIP(hipMemcpyAsync(sel_dev, sc.sel, (size_t)T * K * 4, hipMemcpyDeviceToDevice, e->stream));
@@ -494,33 +505,47 @@ extern "C" int pk_moe_forward_batch_noalloc(pk_engine *e, int layer, const float
     return PK_OK;
 }
 
-static int prefill_reserve(pk_engine *e, int B) {
+// Prompt rows: B rows of hidden states, QKV and attention; part_rows of the
+// split attention's partials (the lockstep decode, and windows past what
+// k_attn_rows_exact holds).
+static int prefill_reserve(pk_engine *e, int B, int part_rows) {
+    const pk_cfg *c = &e->c;
+    if (part_rows > e->p_part_cap) {
+        PK_HIP(hipStreamSynchronize(e->stream));
+        pk_dev_free(e, e->p_part);
+        e->p_part = nullptr;
+        e->p_part_cap = 0;
+        const int max_chunks = (c->ctx_len + 127) / 128;
+        PK_TRY(pk_dev_alloc(e, (void **)&e->p_part,
+                            (int64_t)part_rows * c->n_heads * max_chunks * (c->head_dim + 2) * 4));
+        e->p_part_cap = part_rows;
+    }
     if (B <= e->p_cap) return PK_OK;
     PK_HIP(hipStreamSynchronize(e->stream));
-    void *ptrs[] = {e->p_H, e->p_XN, e->p_qkv, e->p_att, e->p_part, e->p_ids};
+    void *ptrs[] = {e->p_H, e->p_XN, e->p_qkv, e->p_att, e->p_ids};
     for (void *p : ptrs) pk_dev_free(e, p);
-    e->p_H = e->p_XN = e->p_qkv = e->p_att = e->p_part = nullptr;
+    e->p_H = e->p_XN = e->p_qkv = e->p_att = nullptr;
     e->p_ids = nullptr;
     e->p_cap = 0;
-    const pk_cfg *c = &e->c;
     const int64_t qkv_dim = (int64_t)(c->n_heads + 2 * c->n_kv_heads) * c->head_dim;
-    const int max_chunks = (c->ctx_len + 127) / 128;
     PK_TRY(pk_dev_alloc(e, (void **)&e->p_H, (int64_t)B * c->hidden * 4));
     PK_TRY(pk_dev_alloc(e, (void **)&e->p_XN, (int64_t)B * c->hidden * 4));
     PK_TRY(pk_dev_alloc(e, (void **)&e->p_qkv, B * qkv_dim * 4));
     PK_TRY(pk_dev_alloc(e, (void **)&e->p_att, (int64_t)B * c->n_heads * c->head_dim * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->p_part,
-                        (int64_t)B * c->n_heads * max_chunks * (c->head_dim + 2) * 4));
     PK_TRY(pk_dev_alloc(e, (void **)&e->p_ids, (int64_t)c->ctx_len * 4));
     e->p_cap = B;
     return PK_OK;
 }
 
 // forward_prefill (picchio.c:1795-1932) of ids_dev[0..n) at positions
-// pos_base..pos_base+n-1; the greedy next token goes to the decode state
-// (and to out_toks when given).
-static int prefill_chunk(pk_engine *e, int seq, const int32_t *ids_dev, int last_tok, int n, int pos_base,
-                         int32_t *out_toks, int out_cap, bool mfma) {
+// pos_base..pos_base+n-1, in chunks of B: every layer runs on all n rows at
+// once (a row's arithmetic does not depend on the rows beside it, but for the
+// MoE's expert order, which stays each chunk's own). A chunk ends with a draw
+// (picchio.c:1750); the greedy token of any but the prompt's last chunk is
+// overwritten unread, so without sampling only `last` asks for it. The next
+// token goes to the decode state (and to out_toks when given).
+static int prefill_rows(pk_engine *e, int seq, const int32_t *ids, const int32_t *ids_dev, int n, int B, int pos_base,
+                        int32_t *out_toks, int out_cap, bool mfma, bool last) {
     const pk_cfg *c = &e->c;
     const int D = c->hidden;
     hipLaunchKernelGGL(k_embed_rows, dim3(n), dim3(256), 0, e->stream, ids_dev, e->embed, c->vocab, e->p_H, D);
@@ -533,12 +558,25 @@ static int prefill_chunk(pk_engine *e, int seq, const int32_t *ids_dev, int last
         if (mfma)
             PK_TRY(moe_rows_mfma(e, l, e->p_XN, n, e->p_H, e->p_H, nullptr, nullptr));
         else
-            PK_TRY(moe_rows(e, l, e->p_XN, n, e->p_H, e->p_H));
+            PK_TRY(moe_rows(e, l, e->p_XN, n, e->p_H, e->p_H, false, B));
     }
-    PK_TRY(pk_launch_rmsnorm(e->hn, e->p_H + (int64_t)(n - 1) * D, e->final_norm, D, c->eps, 1, e->stream));
-    PK_TRY(pk_set_state(e, last_tok, pos_base + n - 1));
-    return pk_lm_head_step(e, e->hn, nullptr, out_toks, out_cap);
+    for (int off = 0; off < n; off += B) {
+        const int end = std::min(off + B, n) - 1;
+        if (!e->samp_on && !(last && end == n - 1)) continue;
+        PK_TRY(pk_launch_rmsnorm(e->hn, e->p_H + (int64_t)end * D, e->final_norm, D, c->eps, 1, e->stream));
+        PK_TRY(pk_set_state(e, ids[end], pos_base + end));
+        PK_TRY(pk_lm_head_step(e, e->hn, nullptr, out_toks, out_cap));
+    }
+    return PK_OK;
 }
+
+// Rows that one pass over the layers takes: as many whole chunks as make up
+// PREFILL_ROWS, where nothing depends on the chunk (the matrix-core MoE and
+// the router trace keep one chunk per pass; so do windows that
+// k_attn_rows_exact does not hold). 512 tokens, four 20B layers: 17.7 ms
+// in chunks of 64 (each with its lm_head), 8.5 in one pass: full tiles of the
+// experts' rows, 512-row projections, one lm_head.
+constexpr int PREFILL_ROWS = 512;
 
 int pk_prefill_run(pk_engine *e, int seq, const int32_t *ids, int n, int pos_base, int32_t *out_toks,
                    int out_cap) {
@@ -555,15 +593,22 @@ int pk_prefill_run(pk_engine *e, int seq, const int32_t *ids, int n, int pos_bas
     // limbs with pk_set_grouped_f16 off)
     const char *mv = getenv("PK_PREFILL_MFMA");
     const bool mfma = mv && atoi(mv) != 0;
-    PK_TRY(prefill_reserve(e, B));
-    PK_TRY(batch_reserve(e, B));
+    int rows = B;
+    if (!mfma && !e->rtrace && B < PREFILL_ROWS) rows = std::min(PREFILL_ROWS / B * B, n);
+    if (prefill_reserve(e, rows, B) != PK_OK || batch_reserve(e, rows) != PK_OK) {
+        rows = B;                                      // little memory left: chunk by chunk
+        PK_TRY(prefill_reserve(e, B, B));
+        PK_TRY(batch_reserve(e, B));
+    }
     PK_HIP(hipMemcpyAsync(e->p_ids, ids, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
     // a repetition penalty counts the prompt itself (picchio.c:1960-1967)
     PK_TRY(pk_sample_seed_history(e, e->p_ids, n));
-    for (int off = 0; off < n; off += B) {
-        const int len = n - off < B ? n - off : B;
-        PK_TRY(prefill_chunk(e, seq, e->p_ids + off, ids[off + len - 1], len, pos_base + off, out_toks, out_cap,
-                             mfma));
+    for (int off = 0; off < n;) {
+        int len = std::min(rows, n - off);
+        if (pos_base + off + len > PK_ATT_EXACT_SPAN) len = std::min(B, n - off);
+        PK_TRY(prefill_rows(e, seq, ids + off, e->p_ids + off, len, B, pos_base + off, out_toks, out_cap, mfma,
+                            off + len == n));
+        off += len;
     }
     PK_HIP(hipStreamSynchronize(e->stream));           // ids is the caller's pageable memory
     return PK_OK;
@@ -720,7 +765,7 @@ extern "C" int pk_decode_batch(pk_engine *e, int n_seq, const int32_t *toks_host
     PK_TRY(pk_dense_tiles(e));
     const pk_cfg *c = &e->c;
     const int D = c->hidden, V = c->vocab;
-    PK_TRY(prefill_reserve(e, n_seq));
+    PK_TRY(prefill_reserve(e, n_seq, n_seq));
     PK_TRY(batch_reserve(e, n_seq));
     if (n_seq > e->bd_cap || n_steps + 1 > e->bd_steps) {
         PK_HIP(hipStreamSynchronize(e->stream));

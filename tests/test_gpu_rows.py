@@ -37,7 +37,7 @@ def test_i4_rows_matmul_bitexact(gpu, oracle, O, I, S, offset):
     assert bits_equal(y, y_ref), first_mismatch(y, y_ref)
 
 
-@pytest.mark.parametrize("T", [23, 24, 70])
+@pytest.mark.parametrize("T", [23, 24, 70, 255, 256, 300])
 def test_i4_rows_moe_matches_single_tokens(gpu, T):
     """With one expert per token the batch's expert order does not matter:
     every row of the grouped launch has the bits of the token's own call."""
