@@ -190,18 +190,21 @@ __global__ __launch_bounds__(CH_THREADS) void k_gemm_chain8(const float *__restr
         load(st[0], 0);
         load(st[1], min(1, chunks - 1) * KC);
     }
-    for (int n = 0; n < chunks; n += 2) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            if (n + u < chunks) {
-                float *wl = lds + u * BUF, *xl = wl + CH_OUTS * P;
-                store(st[u], wl, xl);
-                load(st[u], min(n + u + 2, chunks - 1) * KC);
-                __syncthreads();
-                multiply(wl, xl, min(KC, I8 - (n + u) * KC) / 8);
-            }
-        }
+    const auto chunk = [&](stage &sv, int n, float *wl, bool refill) {
+        float *xl = wl + CH_OUTS * P;
+        store(sv, wl, xl);
+        if (refill) load(sv, min(n + 2, chunks - 1) * KC);
+        __syncthreads();
+        multiply(wl, xl, min(KC, I8 - n * KC) / 8);
+    };
+    // pairs without guards (a guarded refill would make every wait one for all
+    // outstanding loads), then the last
+    int n = 0;
+    for (; n + 2 <= chunks; n += 2) {
+        chunk(st[0], n, lds, true);
+        chunk(st[1], n + 1, lds + BUF, true);
     }
+    if (n < chunks) chunk(st[0], n, lds, false);
     // hsum256: ((c0+c4)+(c2+c6))+((c1+c5)+(c3+c7)); wave 1 holds c4 .. c7
     __syncthreads();
     if (h == 1) {
@@ -364,30 +367,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         load(st[0], 0);
         load(st[1], min(1, chunks - 1) * CT_KC);
     }
-    for (int n = 0; n < chunks; n += 2) {
+    const auto chunk = [&](stage &sv, int n, float *wl, bool refill) {
+        float *xl = wl + CT_TILE * CT_P;
+        store(sv, wl, xl);
+        if (refill) load(sv, min(n + 2, chunks - 1) * CT_KC);
+        __syncthreads();
+        const int steps = min(CT_KC, I8 - n * CT_KC) / 8;
+        const float *wp = wl + (32 * p + r) * CT_P + 4 * b, *xp = xl + (32 * q + r) * CT_P + 4 * b;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            if (n + u < chunks) {
-                float *wl = lds + u * BUF, *xl = wl + CT_TILE * CT_P;
-                store(st[u], wl, xl);
-                load(st[u], min(n + u + 2, chunks - 1) * CT_KC);
-                __syncthreads();
-                const int steps = min(CT_KC, I8 - (n + u) * CT_KC) / 8;
-                const float *wp = wl + (32 * p + r) * CT_P + 4 * b, *xp = xl + (32 * q + r) * CT_P + 4 * b;
-#pragma unroll
-                for (int k = 0; k < CT_KC / 8; ++k) {
-                    if (k < steps) {
-                        const float4 w = *reinterpret_cast<const float4 *>(wp + 8 * k);
-                        const float4 x = *reinterpret_cast<const float4 *>(xp + 8 * k);
-                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.x, w.x, acc[0], 0, 0, 0);
-                        acc[1] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.y, w.y, acc[1], 0, 0, 0);
-                        acc[2] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.z, w.z, acc[2], 0, 0, 0);
-                        acc[3] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.w, w.w, acc[3], 0, 0, 0);
-                    }
-                }
+        for (int k = 0; k < CT_KC / 8; ++k) {
+            if (k < steps) {
+                const float4 w = *reinterpret_cast<const float4 *>(wp + 8 * k);
+                const float4 x = *reinterpret_cast<const float4 *>(xp + 8 * k);
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.x, w.x, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.y, w.y, acc[1], 0, 0, 0);
+                acc[2] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.z, w.z, acc[2], 0, 0, 0);
+                acc[3] = __builtin_amdgcn_mfma_f32_32x32x1f32(x.w, w.w, acc[3], 0, 0, 0);
             }
         }
+    };
+    // pairs without guards, then the last
+    int n = 0;
+    for (; n + 2 <= chunks; n += 2) {
+        chunk(st[0], n, lds, true);
+        chunk(st[1], n + 1, lds + BUF, true);
     }
+    if (n < chunks) chunk(st[0], n, lds, false);
     // registers k / 16 + k: block k / 16 (chains i, 4 + i), input row
     // 8 (k % 16 / 4) + 4 b + k % 4, output r
 #pragma unroll
@@ -553,44 +558,54 @@ __global__ __launch_bounds__(64) void k_router_seq4(const float *__restrict__ X,
     // (the bias is waited for here: inside the loop the compiler would wait
     // for every outstanding load before the first add)
     asm volatile("" ::"v"(acc));
-    for (int n0 = 0; n0 < chunks; n0 += RQ_PF) {
+    const auto chunk = [&](stage &sv, int n, float *wt, bool refill) {
+        float *xt = wt + EB * RQ_P;
 #pragma unroll
-        for (int v = 0; v < RQ_PF; ++v) {
-            const int n = n0 + v;
-            if (n < chunks) {
-                float *wt = lds[v & 1], *xt = wt + EB * RQ_P;
-#pragma unroll
-                for (int u = 0; u < WN; ++u) {
-                    const int q = lane + 64 * u;
-                    *reinterpret_cast<pk_f32x4 *>(wt + q / C4 * RQ_P + 4 * (q % C4)) = st[v].w[u];
-                }
-#pragma unroll
-                for (int u = 0; u < XN; ++u) {
-                    const int q = lane + 64 * u;
-                    if (q < ROWS * C4) *reinterpret_cast<pk_f32x4 *>(xt + q / C4 * RQ_P + 4 * (q % C4)) = st[v].x[u];
-                }
-                load(st[v], n + RQ_PF);
-                __syncthreads();                  // (one wave: orders the LDS writes and reads)
-                const int nc4 = min(RS_KC, D - n * RS_KC) / 4;
-                const float *wp = wt + lane % EB * RQ_P, *xp = xt + lane / EB * RQ_P;
-                auto add4 = [&](int j) {
-                    const pk_f32x4 w = *reinterpret_cast<const pk_f32x4 *>(wp + 4 * j);
-                    const pk_f32x4 x = *reinterpret_cast<const pk_f32x4 *>(xp + 4 * j);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const float p = x[k] * w[k];
-                        acc = acc + p;
-                    }
-                };
-                if (nc4 == C4) {
-#pragma unroll
-                    for (int j = 0; j < C4; ++j) add4(j);
-                } else {
-                    for (int j = 0; j < nc4; ++j) add4(j);
-                }
-            }
+        for (int u = 0; u < WN; ++u) {
+            const int q = lane + 64 * u;
+            *reinterpret_cast<pk_f32x4 *>(wt + q / C4 * RQ_P + 4 * (q % C4)) = sv.w[u];
         }
+#pragma unroll
+        for (int u = 0; u < XN; ++u) {
+            const int q = lane + 64 * u;
+            if (q < ROWS * C4) *reinterpret_cast<pk_f32x4 *>(xt + q / C4 * RQ_P + 4 * (q % C4)) = sv.x[u];
+        }
+        if (refill) load(sv, n + RQ_PF);
+        __syncthreads();                          // (one wave: orders the LDS writes and reads)
+        const int nc4 = min(RS_KC, D - n * RS_KC) / 4;
+        const float *wp = wt + lane % EB * RQ_P, *xp = xt + lane / EB * RQ_P;
+        const auto add4 = [&](const pk_f32x4 &w, const pk_f32x4 &x) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float p = x[k] * w[k];
+                acc = acc + p;
+            }
+        };
+        if (nc4 == C4) {
+            // every LDS read goes out before the first add
+            pk_f32x4 w[C4], x[C4];
+#pragma unroll
+            for (int j = 0; j < C4; ++j) {
+                w[j] = *reinterpret_cast<const pk_f32x4 *>(wp + 4 * j);
+                x[j] = *reinterpret_cast<const pk_f32x4 *>(xp + 4 * j);
+            }
+#pragma unroll
+            for (int j = 0; j < C4; ++j) add4(w[j], x[j]);
+        } else {
+            for (int j = 0; j < nc4; ++j)
+                add4(*reinterpret_cast<const pk_f32x4 *>(wp + 4 * j), *reinterpret_cast<const pk_f32x4 *>(xp + 4 * j));
+        }
+    };
+    // whole rounds without guards (a guarded refill would make every wait one
+    // for all outstanding loads), then the rest
+    int n = 0;
+    for (; n + RQ_PF <= chunks; n += RQ_PF) {
+#pragma unroll
+        for (int v = 0; v < RQ_PF; ++v) chunk(st[v], n + v, lds[v & 1], true);
     }
+#pragma unroll
+    for (int v = 0; v < RQ_PF; ++v)
+        if (n + v < chunks) chunk(st[v], n + v, lds[v & 1], false);
     if (e < E && s < S) logits[(int64_t)s * E + e] = acc;
 }
 
