@@ -173,6 +173,7 @@ struct pk_engine {
     int samp_cap = 0;
     float *samp_av = nullptr;
     int32_t *samp_ai = nullptr;
+    void *samp_ws = nullptr;                  // counts, candidates and sums of the draws over the device
 };
 
 // Fixed device array of pk_moe_forward_batch_noalloc (pk_prefill.hip): its
