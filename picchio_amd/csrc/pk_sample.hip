@@ -45,13 +45,15 @@ constexpr int NW = SNT / 64;              // its waves
 constexpr int U = 16;                     // loads in flight per lane in a pass
 constexpr int SMALL = 4096;               // kept entries handled in LDS in the reference's order
 constexpr int CAND = 4096;                // top-k candidates gathered into LDS after the first radix pass
+constexpr int RANK_N = 512;               // entries placed by counting instead of a bitonic network
 constexpr int FX_P = 62;                  // fixed-point bits for probabilities (sums <= ~1)
 
 // Scratch of the launches that spread a draw over the device (zeroed when
 // allocated; the counters are re-armed by the launch that reads them last).
 constexpr int SB_BINS = 4096;
 struct samp_ws {
-    uint32_t hist[SB_BINS], cur[SB_BINS + 1];
+    uint32_t hist[SB_BINS];
+    uint32_t cur[SB_BINS * 16];           // a bucket's cursor, 64 bytes apart: neighbours do not share a line
     int32_t n_cand;                       // top-k candidates in cv / ci (0: none gathered)
     uint32_t mx_key;                      // key of the largest scaled logit
     float sum;                            // the ordered sum of the launch before
@@ -233,6 +235,29 @@ __device__ __forceinline__ void bitonic(float *sv, int *si, int P) {
         }
 }
 
+// f(v) for v = p[0], p[1], .. until it returns true; the index it did so at,
+// or -1. LDS reads go out eight at a time ahead of the chain.
+template <class F>
+__device__ __forceinline__ int serial_scan(const float *p, int n, F f) {
+    int j = 0;
+    for (; j + 8 <= n; j += 8) {
+        float t[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) t[u] = p[j + u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (f(t[u])) return j + u;
+    }
+    for (; j < n; ++j)
+        if (f(p[j])) return j;
+    return -1;
+}
+__device__ __forceinline__ float serial_sum(const float *p, int n) {
+    float s = 0.0f;
+    (void)serial_scan(p, n, [&](float v) { s = s + v; return false; });
+    return s;
+}
+
 // Step 5 over kv / ki[0..n) in LDS (n <= SMALL), in the reference's order.
 // Returns (to thread 0) the position picked, or -1; *r_out the draw.
 __device__ __forceinline__ int finish_small(float *kv, int n, float top_p, pk_sampler_dev *sp, float *sv, int *si,
@@ -243,11 +268,7 @@ __device__ __forceinline__ int finish_small(float *kv, int n, float top_p, pk_sa
     mx = block_max(mx, s_red);
     for (int j = tid; j < n; j += SNT) kv[j] = expf(kv[j] - mx);
     __syncthreads();
-    if (tid == 0) {
-        float s = 0.0f;
-        for (int j = 0; j < n; ++j) s = s + kv[j];
-        *s_sum = s;
-    }
+    if (tid == 0) *s_sum = serial_sum(kv, n);
     __syncthreads();
     const float sum = *s_sum;
     for (int j = tid; j < n; j += SNT) kv[j] = kv[j] / sum;
@@ -264,31 +285,35 @@ __device__ __forceinline__ int finish_small(float *kv, int n, float top_p, pk_sa
         for (int w = 0; w < NW; ++w) na += s_redi[w];
         if (na > 1) {
             // sorting every entry puts the candidates (> 1e-10) first, in order
-            int P = 1;
-            while (P < n) P <<= 1;
-            for (int j = tid; j < P; j += SNT) {
-                sv[j] = j < n ? kv[j] : -INFINITY;
-                si[j] = j < n ? j : 0x7fffffff;
+            if (n <= RANK_N) {
+                // each entry's place by counting those before it
+                if (tid < n) {
+                    const float x = kv[tid];
+                    int at = 0;
+                    for (int i = 0; i < n; ++i) at += kv[i] > x || (kv[i] == x && i < tid) ? 1 : 0;
+                    sv[at] = x;
+                    si[at] = tid;
+                }
+                __syncthreads();
+            } else {
+                int P = 1;
+                while (P < n) P <<= 1;
+                for (int j = tid; j < P; j += SNT) {
+                    sv[j] = j < n ? kv[j] : -INFINITY;
+                    si[j] = j < n ? j : 0x7fffffff;
+                }
+                __syncthreads();
+                bitonic(sv, si, P);
             }
-            __syncthreads();
-            bitonic(sv, si, P);
             if (tid == 0) {
                 float cum = 0.0f;
-                int cut = na;
-                for (int j = 0; j < na; ++j) {
-                    cum = cum + sv[j];
-                    if (cum >= top_p) { cut = j + 1; break; }
-                }
-                *s_cut = cut;
+                const int at = serial_scan(sv, na, [&](float v) { cum = cum + v; return cum >= top_p; });
+                *s_cut = at < 0 ? na : at + 1;
             }
             __syncthreads();
             for (int j = *s_cut + tid; j < na; j += SNT) kv[si[j]] = 0.0f;
             __syncthreads();
-            if (tid == 0) {
-                float s = 0.0f;
-                for (int j = 0; j < n; ++j) s = s + kv[j];
-                *s_sum = s;
-            }
+            if (tid == 0) *s_sum = serial_sum(kv, n);
             __syncthreads();
             const float s2 = *s_sum;
             if (s2 > 0)
@@ -306,10 +331,7 @@ __device__ __forceinline__ int finish_small(float *kv, int n, float top_p, pk_sa
         const float r = (float)(x >> 33) / (float)(1ULL << 31);
         *r_out = r;
         float cum = 0.0f;
-        for (int j = 0; j < n; ++j) {
-            cum = cum + kv[j];
-            if (cum >= r) { pick = j; break; }
-        }
+        pick = serial_scan(kv, n, [&](float v) { cum = cum + v; return cum >= r; });
         if (pick < 0)
             for (int j = n - 1; j >= 0; --j)
                 if (kv[j] > 0) { pick = j; break; }
@@ -338,9 +360,30 @@ constexpr int OS_CHUNK = OS_E * SNT;
 constexpr int OS_BUF = OS_CHUNK + OS_CHUNK / OS_E;     // LDS floats (rows of 8 set 9 apart)
 constexpr uint32_t OS_BIG = 1u << 25;     // a move past the binade
 
-__device__ __forceinline__ uint2 os_then(uint2 a, uint2 b) {      // a's moves, then b's
-    return make_uint2(min(a.x + ((a.x & 1u) ? b.y : b.x), OS_BIG),
-                      min(a.y + ((a.y & 1u) ? b.x : b.y), OS_BIG));
+// a's moves, then b's (the callers clamp to OS_BIG before 32 bits could
+// overflow: 8 elements, 64 lanes, 16 waves)
+__device__ __forceinline__ uint2 os_then(uint2 a, uint2 b) {
+    return make_uint2(a.x + ((a.x & 1u) ? b.y : b.x), a.y + ((a.y & 1u) ? b.x : b.y));
+}
+__device__ __forceinline__ uint2 os_clamp(uint2 a) { return make_uint2(min(a.x, OS_BIG), min(a.y, OS_BIG)); }
+// a lane's pair moved by a DPP control (lanes without a source: no moves)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint2 os_dpp(uint2 a) {
+    return make_uint2((uint32_t)__builtin_amdgcn_update_dpp(0, (int)a.x, CTRL, ROWS, 0xf, false),
+                      (uint32_t)__builtin_amdgcn_update_dpp(0, (int)a.y, CTRL, ROWS, 0xf, false));
+}
+// Inclusive scan over the lanes of a row of 16, or of the wave.
+template <bool WAVE>
+__device__ __forceinline__ uint2 os_scan(uint2 a) {
+    a = os_then(os_dpp<0x111, 0xf>(a), a);                 // row shifts by 1, 2, 4, 8
+    a = os_then(os_dpp<0x112, 0xf>(a), a);
+    a = os_then(os_dpp<0x114, 0xf>(a), a);
+    a = os_then(os_dpp<0x118, 0xf>(a), a);
+    if constexpr (WAVE) {
+        a = os_then(os_dpp<0x142, 0xa>(a), a);             // lane 15 of rows 0, 2 to rows 1, 3
+        a = os_then(os_dpp<0x143, 0xc>(a), a);             // lane 31 to rows 2, 3
+    }
+    return a;
 }
 
 // find: stop at the first index whose running sum is >= r. Leaves the sum (up
@@ -354,13 +397,20 @@ __device__ __forceinline__ void order_sum(const float *src, int n, float *buf, b
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float s = 0.0f;
     int hit = -1;
-    for (int base = 0; base < n && hit < 0 && s == s; base += OS_CHUNK) {
+    float nx[OS_E];                       // the next chunk, in flight while this one is scanned
+    const auto fetch = [&](int b) {
+#pragma unroll
+        for (int k = 0; k < OS_E; ++k) nx[k] = src[min(b + tid + SNT * k, n - 1)];
+    };
+    if (n > 0) fetch(0);
+    for (int base = 0; base < n && hit < 0; base += OS_CHUNK) {
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < OS_E; ++k) {
             const int j = tid + SNT * k;
-            buf[j + j / OS_E] = base + j < n ? src[base + j] : 0.0f;      // (+ 0 leaves the sum as it is)
+            buf[j + j / OS_E] = base + j < n ? nx[k] : 0.0f;              // (+ 0 leaves the sum as it is)
         }
+        if (base + OS_CHUNK < n) fetch(base + OS_CHUNK);
         __syncthreads();
         float v[OS_E];
 #pragma unroll
@@ -373,39 +423,27 @@ __device__ __forceinline__ void order_sum(const float *src, int n, float *buf, b
             uint2 d = make_uint2(0u, 0u);                  // (x: from S even, y: from S odd)
 #pragma unroll
             for (int k = 0; k < OS_E; ++k) {
-                const float t = ldexpf(v[k], 150 - ex);
-                uint2 m;
-                if (!(t < 16777216.0f)) {                  // (NaN too)
-                    m = make_uint2(OS_BIG, OS_BIG);
-                } else {
-                    const float f = floorf(t), h = t - f;
-                    const uint32_t q = (uint32_t)f;
-                    m.x = q + (h > 0.5f || (h == 0.5f && (q & 1u)) ? 1u : 0u);
-                    m.y = q + (h > 0.5f || (h == 0.5f && !(q & 1u)) ? 1u : 0u);
-                }
-                if (OS_E * tid + k < start) m = make_uint2(0u, 0u);
-                d = os_then(d, m);
+                // (past the binade, infinite or NaN: OS_BIG)
+                const float t = fminf(ldexpf(v[k], 150 - ex), (float)OS_BIG);
+                const float q = rintf(t), h = t - q;       // a tie goes to even: the move for S even
+                const float qo = q + (fabsf(h) == 0.5f ? h + h : 0.0f);
+                d = os_then(d, make_uint2((uint32_t)q, (uint32_t)qo));
             }
-            uint2 inc = d;
-            for (int o = 1; o < 64; o <<= 1) {
-                uint2 t;
-                t.x = (uint32_t)__shfl_up((int)inc.x, o, 64);
-                t.y = (uint32_t)__shfl_up((int)inc.y, o, 64);
-                if (lane >= o) inc = os_then(t, inc);
-            }
+            d = os_clamp(d);
+            const uint2 inc = os_scan<true>(d);
             __syncthreads();                               // (s_wave, os_* of the last round are read)
-            if (lane == 63) s_wave[wave] = inc;
+            if (lane == 63) s_wave[wave] = os_clamp(inc);
             if (tid == 0) { os_start = OS_CHUNK; os_hit = 0x7fffffff; }
             __syncthreads();
-            uint2 pre = make_uint2(0u, 0u), all = make_uint2(0u, 0u);
-            for (int w = 0; w < NW; ++w) {
-                if (w == wave) pre = all;
-                all = os_then(all, s_wave[w]);
-            }
-            uint2 ex2;
-            ex2.x = (uint32_t)__shfl_up((int)inc.x, 1, 64);
-            ex2.y = (uint32_t)__shfl_up((int)inc.y, 1, 64);
-            if (lane > 0) pre = os_then(pre, ex2);
+            // lane l < 16: the waves up to l
+            const uint2 upto = os_scan<false>(lane < NW ? s_wave[lane & (NW - 1)] : make_uint2(0u, 0u));
+            const uint2 all = make_uint2((uint32_t)__builtin_amdgcn_readlane((int)upto.x, NW - 1),
+                                         (uint32_t)__builtin_amdgcn_readlane((int)upto.y, NW - 1));
+            const int before = __builtin_amdgcn_readfirstlane(max(wave - 1, 0));
+            uint2 pre = make_uint2((uint32_t)__builtin_amdgcn_readlane((int)upto.x, before),
+                                   (uint32_t)__builtin_amdgcn_readlane((int)upto.y, before));
+            if (wave == 0) pre = make_uint2(0u, 0u);
+            pre = os_then(pre, os_dpp<0x138, 0xf>(inc));   // and the wave's lanes before this one
             const bool odd = S & 1u;
             const uint32_t S0 = S + (odd ? pre.y : pre.x);             // before this thread's elements
             const uint32_t S1 = S0 + ((S0 & 1u) ? d.y : d.x);
@@ -417,7 +455,6 @@ __device__ __forceinline__ void order_sum(const float *src, int n, float *buf, b
                 float x = a0;
                 int at = -1;
                 for (int k = 0; k < OS_E; ++k) {
-                    if (OS_E * tid + k < start) continue;
                     x = x + v[k];
                     if (find && at < 0 && x >= r) {
                         at = OS_E * tid + k;
@@ -437,6 +474,10 @@ __device__ __forceinline__ void order_sum(const float *src, int n, float *buf, b
             if (start < OS_CHUNK || !(S + (odd ? all.y : all.x) < 0x1000000u)) s = os_s;
             else s = ldexpf((float)(S + (odd ? all.y : all.x)), ex - 150);
             if (!(s < INFINITY)) break;                    // NaN stays NaN, infinity stays (nothing later changes it)
+            if (OS_E * tid < start) {                      // (whole threads: in s)
+#pragma unroll
+                for (int k = 0; k < OS_E; ++k) v[k] = 0.0f;
+            }
         }
         if (!(s < INFINITY)) break;
     }
@@ -937,7 +978,22 @@ __global__ __launch_bounds__(SNT) void k_sample(float *lg, int V, pk_sampler_dev
             // current bucket fit in LDS they are gathered there and the rest runs on them
             bool in_lds = given > 0;
             int nc = given;
-            for (int shift = given > 0 ? 24 : 16; shift >= -8; shift -= 8) {
+            const bool few = given > 0 && given <= RANK_N;
+            if (few) {
+                // the K-th largest by counting: entries above it < K <= those not below it
+                if (tid < given) {
+                    const uint32_t k = key_of(cv[tid]);
+                    int above = 0, same = 0;
+                    for (int i = 0; i < given; ++i) {
+                        const uint32_t ki_ = key_of(cv[i]);
+                        above += ki_ > k ? 1 : 0;
+                        same += ki_ == k ? 1 : 0;
+                    }
+                    if (above < K && K <= above + same) s_prefix = k;      // (equal keys write the same)
+                }
+                __syncthreads();
+            }
+            for (int shift = few ? -16 : given > 0 ? 24 : 16; shift >= -8; shift -= 8) {
                 if (!in_lds && s_nc <= CAND) {
                     nc = s_nc;
                     const uint32_t top = s_prefix;
@@ -985,11 +1041,24 @@ __global__ __launch_bounds__(SNT) void k_sample(float *lg, int V, pk_sampler_dev
                     }
                 __syncthreads();
                 n = s_cnt;
-                int P = 1;
-                while (P < n) P <<= 1;
-                for (int j = n + tid; j < P; j += SNT) { kv[j] = 0.0f; ki[j] = 0x7fffffff; }
-                __syncthreads();
-                bitonic_by_index(kv, ki, P);
+                if (n <= RANK_N) {
+                    float x = 0.0f;
+                    int id = 0, at = 0;
+                    if (tid < n) {
+                        x = kv[tid];
+                        id = ki[tid];
+                        for (int i = 0; i < n; ++i) at += ki[i] < id ? 1 : 0;
+                    }
+                    __syncthreads();
+                    if (tid < n) { kv[at] = x; ki[at] = id; }
+                    __syncthreads();
+                } else {
+                    int P = 1;
+                    while (P < n) P <<= 1;
+                    for (int j = n + tid; j < P; j += SNT) { kv[j] = 0.0f; ki[j] = 0x7fffffff; }
+                    __syncthreads();
+                    bitonic_by_index(kv, ki, P);
+                }
                 direct = true;
             } else {
                 n = compact(lg, V, [inv_t, thr](float v) { return !(v * inv_t < thr); }, scaled, av, ai, s_w);
@@ -1202,8 +1271,8 @@ __global__ __launch_bounds__(SH_T) void k_samp_gather(float *lg, int V, const pk
 // its own workgroup (equal values need no order: a sum does not tell them
 // apart, and the cut takes ties by index). Where a bucket exceeds SORT_CAP
 // different values, one workgroup takes the list chunk by chunk instead.
-// Measured, 201,088 entries of a peaked distribution, top-p 0.95: NUC us
-// per draw against 6,000 in one workgroup.
+// Measured, 201,088 entries of a peaked distribution, top-p 0.95: 400 us
+// per draw against 5,000 to 6,000 in one workgroup.
 constexpr int SORT_CAP = 4096;
 constexpr uint32_t P_MIN = 0x2edbe6ffu;   // bits of 1e-10f
 constexpr int P_SHIFT = 17;
@@ -1314,7 +1383,7 @@ __global__ __launch_bounds__(SNT) void k_samp_offsets(samp_ws *ws) {
     uint32_t off = inc - sum;
 #pragma unroll
     for (int i = 0; i < B; ++i) {
-        ws->cur[B * tid + i] = off;
+        ws->cur[(B * tid + i) * 16] = off;
         off += c[i];
     }
     if (tid == SNT - 1) {
@@ -1332,7 +1401,7 @@ __global__ __launch_bounds__(SH_T) void k_samp_place(const float *lg, int V, sam
     for (int k = 0; k < SH_E; ++k) v[k] = lg[min(j0 + SH_T * k, V - 1)];
 #pragma unroll
     for (int k = 0; k < SH_E; ++k)
-        if (j0 + SH_T * k < V && v[k] > 1e-10f) sorted[atomicAdd(&ws->cur[p_bin(v[k])], 1u)] = v[k];
+        if (j0 + SH_T * k < V && v[k] > 1e-10f) sorted[atomicAdd(&ws->cur[p_bin(v[k]) * 16], 1u)] = v[k];
 }
 
 // bucket blockIdx.x, descending (cur[b] is its end once everything is placed);
@@ -1347,7 +1416,7 @@ __global__ __launch_bounds__(SH_T) void k_samp_sort(samp_ws *ws, float *sorted) 
         s_diff = 0;
     }
     if (n <= 1 || ws->m <= 1) return;
-    float *p = sorted + (int)ws->cur[b] - n;
+    float *p = sorted + (int)ws->cur[b * 16] - n;
     __syncthreads();
     if (n > SORT_CAP) {
         const float first = p[0];
