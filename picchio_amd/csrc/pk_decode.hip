@@ -642,13 +642,13 @@ __global__ __launch_bounds__(ATT_THREADS) void k_attn_part(const pk_dstate *st, 
                          gridDim.y, nullptr, 0);
 }
 
-// y[o] += (W[o] . x + b[o])  — attention output projection + residual
-// (picchio.c:615-616, :1690). One workgroup per 4 outputs (one per wave);
-// grid.y = row of a batch (x [rows][I], y [rows][O]).
+// y[o] = res[o] + (W[o] . x + b[o])  — attention output projection + residual
+// (picchio.c:615-616, :1690; res = y: added in place, null: 0). One workgroup
+// per 4 outputs (one per wave); grid.y = row of a batch (x [rows][I], y [rows][O]).
 constexpr int RES_U = 16;              // float4 per lane loaded up front (4096 columns)
 constexpr int ATT_RPW = 2;             // k_attn_oproj: output rows per wave
 
-__global__ __launch_bounds__(256) void k_gemv_res(float *y, const float *__restrict__ x,
+__global__ __launch_bounds__(256) void k_gemv_res(float *y, const float *res, const float *__restrict__ x,
                                                   const float *__restrict__ W,
                                                   const float *__restrict__ b, int I, int O) {
     const int lane = threadIdx.x & 63;
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(256) void k_gemv_res(float *y, const float *__restr
     // past the row read as zero and are not used)
     const pk_buf_t wr = pk_buf(w4, (uint32_t)n4 * 16u), xr = pk_buf(x4, (uint32_t)n4 * 16u);
     // the residual and the bias at entry (at the end each would cost a round trip)
-    const float yo = y[o], bo = b[o];
+    const float yo = res ? res[(int64_t)blockIdx.y * O + o] : 0.0f, bo = b[o];
     pk_f32x4 wv[RES_U];
     float4 xv[RES_U];
 #pragma unroll
@@ -981,7 +981,7 @@ extern "C" int pk_kv_layout(int ctx, int KVH, int hd, int64_t *k_off, int64_t n_
 // and adds the output projection into h [n][D] (residual).
 int pk_attention_rows(pk_engine *e, int l, const pk_dstate *st, int pos_base, int pos_step, int seq0,
                       int seq_step, int n, const float *xn, float *qkv, float *part, float *att, float *h,
-                      const float *norm_w, bool exact) {
+                      const float *norm_w, bool exact, bool residual) {
     const pk_cfg *c = &e->c;
     const pk_layer_dev &d = e->L[l];
     const int H = c->n_heads, KVH = c->n_kv_heads, hd = c->head_dim, D = c->hidden;
@@ -1093,8 +1093,8 @@ int pk_attention_rows(pk_engine *e, int l, const pk_dstate *st, int pos_base, in
                                          e->skinny_ws ? PK_SKINNY_WS : 0, nullptr,
                                          pk_tiles_current(e) ? d.wo_t : nullptr));
     } else {
-        hipLaunchKernelGGL(k_gemv_res, dim3((D + 3) / 4, n), dim3(256), 0, e->stream, h, att, d.wo, d.bo,
-                           H * hd, D);
+        hipLaunchKernelGGL(k_gemv_res, dim3((D + 3) / 4, n), dim3(256), 0, e->stream, h, residual ? h : nullptr, att,
+                           d.wo, d.bo, H * hd, D);
         PK_HIP(hipGetLastError());
     }
     return pk_prof_end(e, ps);
@@ -1182,13 +1182,17 @@ extern "C" int pk_gqa_attention(pk_engine *e, int layer, const float *x_dev, int
     PK_CHECK(pos < c->ctx_len, PK_ERR_CONTEXT_FULL, "pos %d >= context %d", pos, c->ctx_len);
     PK_CHECK(!e->capturing, PK_ERR_ARG, "gqa_attention: host position; not available while capturing");
     PK_TRY(pk_decode_reserve(e));
-    PK_TRY(pk_set_state(e, 0, pos));
-    PK_HIP(hipMemcpyAsync(e->hn, x_dev, (size_t)c->hidden * 4, hipMemcpyDeviceToDevice, e->stream));
-    PK_HIP(hipMemsetAsync(e->h, 0, (size_t)c->hidden * 4, e->stream));
+    // straight from x_dev (read by the first launch only) into out_dev, the
+    // position as a launch argument: four launches and no copies around them
+    // (a sliding-window and a full layer at 4096 positions 127 -> 102 us)
+    const float *x = x_dev;
+    if ((uintptr_t)x_dev & 15) {
+        PK_HIP(hipMemcpyAsync(e->hn, x_dev, (size_t)c->hidden * 4, hipMemcpyDeviceToDevice, e->stream));
+        x = e->hn;
+    }
     att_cap_scope cap(e, pos);
-    PK_TRY(pk_attention_rows(e, layer, e->dstate, 0, 0, 0, 0, 1, e->hn, e->qkv, e->attn_part, e->att,
-                             e->h));                // h = 0 + attn(x)
-    PK_HIP(hipMemcpyAsync(out_dev, e->h, (size_t)c->hidden * 4, hipMemcpyDeviceToDevice, e->stream));
+    PK_TRY(pk_attention_rows(e, layer, nullptr, pos, 0, 0, 0, 1, x, e->qkv, e->attn_part, e->att, out_dev, nullptr,
+                             false, false));               // out = 0 + attn(x)
     PK_HIP(hipStreamSynchronize(e->stream));
     return PK_OK;
 }

@@ -262,7 +262,7 @@ int pk_set_state(pk_engine *e, int tok, int pos);
 // exact: the prompt rows in the reference's operation order (pk_exact.hip).
 int pk_attention_rows(pk_engine *e, int l, const pk_dstate *st, int pos_base, int pos_step, int seq0,
                       int seq_step, int n, const float *xn, float *qkv, float *part, float *att, float *h,
-                      const float *norm_w = nullptr, bool exact = false);
+                      const float *norm_w = nullptr, bool exact = false, bool residual = true);
 // the prompt path's dense steps in the reference's order (pk_exact.hip)
 int pk_launch_gemm_chain8(const float *X, int64_t ldx, const float *W, const float *bias, float *out, int64_t ldo,
                           int S, int I, int O, bool add_res, hipStream_t st);

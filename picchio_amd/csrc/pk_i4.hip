@@ -148,6 +148,91 @@ __global__ __launch_bounds__(NW * 64) void k_i4_gemv(pk_i4_items it, int O, int 
         if (rt.logits && rb == 0 && item == 0) pk_wave_route_publish(rt);
 }
 
+// ───────────── GEMV of few row blocks ─────────────
+// k_i4_gemv's values where its workgroups would leave CUs idle: a workgroup
+// takes R = 16 or 32 rows of a row block, its waves 64 / R groups at a time
+// (lane = R gq + r: row r, group g0 + gq), GPW times. With 90 or 45 workgroups
+// on 256 CUs the three group dots of a wave's 64 rows, four waves to a SIMD,
+// take ~4 us of the launch; here a lane has one or two. The inputs, no longer
+// one group per wave, are read from LDS (groups 68 floats apart, so that the
+// groups' 16-byte reads meet distinct banks). One 20B expert's gate_up and
+// down: see pk_launch_i4_gemv.
+constexpr int PR_NW = 12, PR_XP = 68;
+template <int EPI, int R, int GPW>
+__global__ __launch_bounds__(PR_NW * 64) void k_i4_gemv_part(pk_i4_items it, int O, int NG, float lim, float alpha) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];     // xs[NG][68], part[NG][R], scl[NG][R]
+    constexpr int GQ = 64 / R, PARTS = 64 / R;
+    float *xs = lds, *part = lds + NG * PR_XP, *scl = part + NG * R;
+    const int lane = threadIdx.x & 63, r = lane % R, gq = lane / R;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rb = blockIdx.x / PARTS, r0 = R * (blockIdx.x % PARTS), item = blockIdx.y;
+    const int slot = it.slot_base + (it.slots ? it.slots[item] : 0);
+    const uint8_t *base = it.base + (int64_t)slot * it.slot_stride;
+    const uint4 *tiles =
+        reinterpret_cast<const uint4 *>(base + it.off_tiles) + (int64_t)rb * NG * (PK_TILE_BYTES / 16) + r0 + r;
+    const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64 + r0 + r;
+    const float *__restrict__ x = it.x + (int64_t)(item / it.x_div) * it.x_stride;
+    const int row = rb * 64 + r0 + r;
+    uint4 wa[GPW], wb[GPW];
+    float s[GPW];
+    const auto load = [&](int g0) {
+#pragma unroll
+        for (int u = 0; u < GPW; ++u) {
+            const int g = min(g0 + u * PR_NW * GQ + gq, NG - 1);
+            wa[u] = pk_load_nt(&tiles[g * 128]);
+            wb[u] = pk_load_nt(&tiles[g * 128 + 64]);
+            s[u] = sc[g * 64];
+        }
+    };
+    load(GQ * wave);
+    const float bias = wave == 0 && it.off_bias >= 0
+                           ? reinterpret_cast<const float *>(base + it.off_bias)[min(row, O - 1)] : 0.0f;
+    for (int i = threadIdx.x; i < NG * 64; i += PR_NW * 64) xs[(i >> 6) * PR_XP + (i & 63)] = x[i];
+    __syncthreads();
+    for (int g0 = GQ * wave; g0 < NG; g0 += GPW * PR_NW * GQ) {
+#pragma unroll
+        for (int u = 0; u < GPW; ++u) {
+            const int g = g0 + u * PR_NW * GQ + gq;
+            if (g < NG) {
+                float xr[64];
+                const float4 *x4 = reinterpret_cast<const float4 *>(xs + g * PR_XP);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const float4 t = x4[i];
+                    xr[4 * i] = t.x; xr[4 * i + 1] = t.y; xr[4 * i + 2] = t.z; xr[4 * i + 3] = t.w;
+                }
+                part[g * R + r] = pk_group_dot(wa[u], wb[u], (const float *)xr);
+                scl[g * R + r] = s[u];
+            }
+        }
+        if (g0 + GPW * PR_NW * GQ < NG) load(g0 + GPW * PR_NW * GQ);
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float acc = 0.0f;
+    constexpr int C = 15;
+    for (int b = 0; b < NG; b += C) {
+        float p[C], v[C];
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            p[j] = part[min(b + j, NG - 1) * R + r];
+            v[j] = scl[min(b + j, NG - 1) * R + r];
+        }
+#pragma unroll
+        for (int j = 0; j < C; ++j)
+            if (b + j < NG) acc = __builtin_fmaf(p[j], v[j], acc);
+    }
+    if (it.off_bias >= 0 && row < O) acc = acc + bias;
+    float *y = it.y + (int64_t)item * it.y_stride;
+    if constexpr (EPI == PK_EPI_SWIGLU) {
+        const float up = __shfl_down(acc, 1, 64);
+        const float a = pk_swiglu(acc, up, lim, alpha);
+        if (lane < R && (lane & 1) == 0 && row + 1 < O) y[row >> 1] = a;
+    } else {
+        if (lane < R && row < O) y[row] = acc;
+    }
+}
+
 // ───────────── persistent streaming GEMV (launches of many row blocks) ─────────────
 // The k_i4_gemv body for launches whose tasks (n_items x RB row blocks) are
 // well above the CUs: one 16-wave workgroup per CU walks tasks blockIdx.x,
@@ -446,6 +531,27 @@ int pk_launch_i4_gemv(const pk_i4_items &it, const pk_i4_shape &sh, int epilogue
             if (dot) PK_I4_STREAM(PK_EPI_PLAIN, true); else PK_I4_STREAM(PK_EPI_PLAIN, false);
         }
 #undef PK_I4_STREAM
+        PK_HIP(hipGetLastError());
+        return PK_OK;
+    }
+    // few row blocks: halves or quarters of them, as long as every CU gets one
+    // workgroup at most (20B widths: 1 expert's gate_up, 90 row blocks, 7.7
+    // against 9.2 us, its down, 45, 5.9 against 8.8; with two workgroups per
+    // CU no better than whole row blocks: 3 experts 393 against 380 us, 250
+    // row blocks 10.8 against 7.8)
+    const int64_t blocks = (int64_t)it.n_items * sh.RB;
+    if (!route && !it.xq && epilogue != PK_EPI_COMBINE && 2 * blocks <= n_cu) {
+        const bool quarter = 4 * blocks <= n_cu;
+        const dim3 grid((quarter ? 4 : 2) * sh.RB, it.n_items);
+        const size_t lds = (size_t)sh.NG * (PR_XP + (quarter ? 32 : 64)) * sizeof(float);
+#define PK_I4_PART(E, R, G)                                                                                          \
+    hipLaunchKernelGGL((k_i4_gemv_part<E, R, G>), grid, dim3(PR_NW * 64), lds, st, it, sh.O, sh.NG, lim, alpha)
+        if (epilogue == PK_EPI_SWIGLU) {
+            if (quarter) PK_I4_PART(PK_EPI_SWIGLU, 16, 1); else PK_I4_PART(PK_EPI_SWIGLU, 32, 2);
+        } else {
+            if (quarter) PK_I4_PART(PK_EPI_PLAIN, 16, 1); else PK_I4_PART(PK_EPI_PLAIN, 32, 2);
+        }
+#undef PK_I4_PART
         PK_HIP(hipGetLastError());
         return PK_OK;
     }

@@ -54,3 +54,24 @@ def test_i4_rows_moe_matches_single_tokens(gpu, T):
             eng.moe_forward_batch(0, xd[t:t + 1], one[t:t + 1])
         a, b = eng.to_host(out), eng.to_host(one)
     assert bits_equal(a, b), first_mismatch(a, b)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_i4_few_row_blocks_match_many(gpu, n):
+    """gate_up and down of a few experts (halves and quarters of row blocks:
+    k_i4_gemv_part) against the same experts among 32 in one launch."""
+    import picchio_amd as pa
+    import torch
+    cfg = pa.gptoss_cfg(n_layers=1, n_experts=32, ctx_len=16, vocab=64)
+    half = cfg.moe_inter // 2
+    with pa.Engine(cfg) as eng:
+        eng.build_synthetic(11, 1)
+        xd = eng.to_dev(_rand((cfg.hidden,), 3))
+        got = []
+        for ids in (np.arange(n, dtype=np.int32), np.arange(32, dtype=np.int32)):
+            act, eo = eng.empty((len(ids), half), torch.float32), eng.empty((len(ids), cfg.hidden), torch.float32)
+            eng.expert_gate_up(0, eng.to_dev(ids), xd, act)
+            eng.expert_down(0, eng.to_dev(ids), act, eo)
+            got.append((eng.to_host(act)[:n], eng.to_host(eo)[:n]))
+    for a, b in zip(*got):
+        assert bits_equal(a, b), first_mismatch(a, b)
