@@ -567,13 +567,14 @@ static int check_i4_host(const pk_qt_host *t, int O, int I, int gs, const char *
 // host ref layout -> staging -> tiles in the slot
 static int upload_i4(pk_engine *e, const pk_qt_host *t, uint8_t *tiles, float *sc16) {
     const int64_t qbytes = (int64_t)t->O * ((t->I + 1) / 2);
-    const int64_t sbytes = (int64_t)t->O * (t->I / PK_GS) * 4;
+    const bool row_scale = t->block_size <= 0;
+    const int64_t sbytes = (int64_t)t->O * (row_scale ? 1 : t->I / PK_GS) * 4;
     PK_TRY(pk_stage_reserve(e, pk_align256(qbytes) + sbytes));
     uint8_t *dq = e->stage;
     float *ds = (float *)(e->stage + pk_align256(qbytes));
     PK_HIP(hipMemcpyAsync(dq, t->data, qbytes, hipMemcpyHostToDevice, e->stream));
     PK_HIP(hipMemcpyAsync(ds, t->s, sbytes, hipMemcpyHostToDevice, e->stream));
-    PK_TRY(pk_launch_i4_repack(dq, ds, t->O, t->I, tiles, sc16, e->stream));
+    PK_TRY(pk_launch_i4_repack(dq, ds, t->O, t->I, tiles, sc16, e->stream, row_scale));
     return PK_OK;
 }
 
@@ -820,7 +821,9 @@ extern "C" int pk_qt_upload(pk_engine *e, const pk_qt_host *h, pk_qt **out) {
         const int gs = h->block_size;
         const int64_t nsc = gs > 0 ? (int64_t)h->O * ((h->I + gs - 1) / gs) : h->O;
         if (!h->s) rc = PK_ERR_ARG;
-        else if (gs == PK_GS && h->I % PK_GS == 0) {
+        else if (h->I % PK_GS == 0 && (gs == PK_GS || (gs <= 0 && h->I <= 128 * PK_GS))) {
+            // (a scale per row: the same tiles, the scale stored for each group;
+            // sum over groups of (scale x group sum), not scale x sum)
             t->tiled = 1;
             t->sh = pk_i4_make_shape(h->O, h->I);
             rc = pk_dev_alloc(e, &t->data, t->sh.tile_bytes);
@@ -871,8 +874,6 @@ extern "C" int pk_matmul_qt(pk_engine *e, float *y, const float *x, const pk_qt 
     case PK_FMT_INT8:   // quant.h:152-186, likewise
         return pk_launch_gemm_chain8_q8(x, (const int8_t *)w->data, w->s, y, S, w->I, w->O, e->stream);
     case PK_FMT_INT4:
-        if (w->gs <= 0)
-            return pk_launch_i4_rowscale_gemv(y, x, (const uint8_t *)w->data, w->s, S, w->I, w->O, e->stream);
         if (w->tiled) {
             pk_i4_items it{};
             it.base = (const uint8_t *)w->data;
@@ -891,6 +892,8 @@ extern "C" int pk_matmul_qt(pk_engine *e, float *y, const float *x, const pk_qt 
                 return pk_launch_i4_rows(it, nullptr, w->sh, PK_EPI_PLAIN, 0.f, 0.f, 0, e->stream);
             return pk_launch_i4_gemv(it, w->sh, PK_EPI_PLAIN, 0.f, 0.f, nullptr, e->stream);
         }
+        if (w->gs <= 0)
+            return pk_launch_i4_rowscale_gemv(y, x, (const uint8_t *)w->data, w->s, S, w->I, w->O, e->stream);
         return pk_launch_i4_gemv_ref(y, x, (const uint8_t *)w->data, w->s, S, w->I, w->O, w->gs, e->stream);
     default:
         pk_set_error("matmul_qt: format %d not supported", w->fmt);

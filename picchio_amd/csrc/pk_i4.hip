@@ -893,9 +893,10 @@ int pk_launch_i4_gemv_ref(float *y, const float *x, const uint8_t *q4, const flo
 
 // ───────────────────────── repack ─────────────────────────
 // Reference layout (q4 [O][I/2], s [O][I/64]) -> tiles + 16*scale.
-// One thread per (row of the padded block, group).
+// One thread per (row of the padded block, group). sng: scales per row in s
+// (NG, or 1: a row scale, stored for every group).
 __global__ void k_i4_repack(const uint8_t *q4, const float *s, int O, int I, int RB, int NG,
-                            uint8_t *tiles, float *sc16) {
+                            uint8_t *tiles, float *sc16, int sng) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (int64_t)RB * 64 * NG) return;
     const int g = (int)(t % NG);
@@ -910,7 +911,7 @@ __global__ void k_i4_repack(const uint8_t *q4, const float *s, int O, int I, int
         for (int k = 0; k < 8; ++k) v[k] = src[k] ^ 0x88888888u;
         lo = make_uint4(v[0], v[1], v[2], v[3]);
         hi = make_uint4(v[4], v[5], v[6], v[7]);
-        scv = 16.0f * s[(int64_t)row * NG + g];
+        scv = 16.0f * s[(int64_t)row * sng + (sng > 1 ? g : 0)];
     }
     uint4 *dst = reinterpret_cast<uint4 *>(tiles + ((int64_t)rb * NG + g) * PK_TILE_BYTES);
     dst[r] = lo;
@@ -919,13 +920,13 @@ __global__ void k_i4_repack(const uint8_t *q4, const float *s, int O, int I, int
 }
 
 int pk_launch_i4_repack(const uint8_t *q4, const float *s, int O, int I,
-                        uint8_t *tiles, float *sc16, hipStream_t st) {
+                        uint8_t *tiles, float *sc16, hipStream_t st, bool row_scale) {
     PK_CHECK(I % 64 == 0 && O > 0, PK_ERR_UNSUPPORTED, "repack: I=%d not a multiple of 64", I);
     PK_CHECK(((uintptr_t)q4 & 3) == 0, PK_ERR_ARG, "repack: q4 not 4-byte aligned");
     const pk_i4_shape sh = pk_i4_make_shape(O, I);
     const int64_t n = (int64_t)sh.RB * 64 * sh.NG;
     hipLaunchKernelGGL(k_i4_repack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                       q4, s, O, I, sh.RB, sh.NG, tiles, sc16);
+                       q4, s, O, I, sh.RB, sh.NG, tiles, sc16, row_scale ? 1 : sh.NG);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }

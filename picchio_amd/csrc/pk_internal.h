@@ -253,7 +253,7 @@ int pk_launch_i4_gemv_ref(float *y, const float *x, const uint8_t *q4, const flo
                           int S, int I, int O, int gs, hipStream_t st);
 
 int pk_launch_i4_repack(const uint8_t *q4, const float *s, int O, int I,
-                        uint8_t *tiles, float *sc16, hipStream_t st);
+                        uint8_t *tiles, float *sc16, hipStream_t st, bool row_scale = false);
 
 int pk_launch_quantize_i4(const float *w, int O, int I, int gs, uint8_t *packed,
                           float *scales, hipStream_t st);
