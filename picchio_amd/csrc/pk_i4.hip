@@ -97,7 +97,9 @@ __global__ __launch_bounds__(NW * 64) void k_i4_gemv(pk_i4_items it, int O, int 
     __syncthreads();
     if (wave != 0) return;
 
-    float acc = pk_fold_groups<DOT>(part, scl, NG);
+    float acc;
+    if constexpr (EPI == PK_EPI_ROW_SCALED) acc = pk_fold_row_scaled(part + lane, scl + lane, NG, 64);
+    else acc = pk_fold_groups<DOT>(part, scl, NG);
     if (it.off_bias >= 0 && row < O) acc = acc + bias;
     float *y = it.y + (int64_t)item * it.y_stride;
     if constexpr (EPI == PK_EPI_SWIGLU) {
@@ -211,7 +213,8 @@ __global__ __launch_bounds__(PR_NW * 64) void k_i4_gemv_part(pk_i4_items it, int
     if (wave != 0) return;
     float acc = 0.0f;
     constexpr int C = 15;
-    for (int b = 0; b < NG; b += C) {
+    if constexpr (EPI == PK_EPI_ROW_SCALED) acc = pk_fold_row_scaled(part + r, scl + r, NG, R);
+    else for (int b = 0; b < NG; b += C) {
         float p[C], v[C];
 #pragma unroll
         for (int j = 0; j < C; ++j) {
@@ -347,7 +350,11 @@ __global__ __launch_bounds__((ST_NW + 1) * 64) void k_i4_gemv_stream(pk_i4_items
         const float bias = it.off_bias >= 0 ? reinterpret_cast<const float *>(base + it.off_bias)[min(row, O - 1)]
                                             : 0.0f;
         st_wait(&cnt[b], ST_NW * ((k >> 1) + 1));
-        float acc = pk_fold_groups<DOT>(part + b * NG * 64, scl + b * NG * 64, NG);
+        float acc;
+        if constexpr (EPI == PK_EPI_ROW_SCALED)
+            acc = pk_fold_row_scaled(part + b * NG * 64 + lane, scl + b * NG * 64 + lane, NG, 64);
+        else
+            acc = pk_fold_groups<DOT>(part + b * NG * 64, scl + b * NG * 64, NG);
         st_signal(&cnt[2 + b]);
         if (it.off_bias >= 0 && row < O) acc = acc + bias;
         float *y = it.y + (int64_t)item * it.y_stride;
@@ -506,6 +513,7 @@ int pk_launch_i4_gemv(const pk_i4_items &it, const pk_i4_shape &sh, int epilogue
     PK_CHECK(sh.NG > 0 && sh.RB > 0 && it.n_items > 0, PK_ERR_ARG, "i4 gemv: empty shape");
     PK_CHECK(sh.NG <= 128, PK_ERR_UNSUPPORTED, "i4 gemv: I=%d above 8192", sh.I);
     PK_CHECK(!it.yq || epilogue == PK_EPI_SWIGLU, PK_ERR_ARG, "i4 gemv: output records need the SwiGLU epilogue");
+    PK_CHECK(epilogue != PK_EPI_ROW_SCALED || (!it.xq && !route), PK_ERR_ARG, "i4 gemv: row scales on the fp32 chains only");
     // many row blocks without routing: the persistent streaming kernel (one
     // workgroup per CU, the next row block's weights in flight meanwhile)
     const int n_cu = pk_device_cus();
@@ -527,6 +535,8 @@ int pk_launch_i4_gemv(const pk_i4_items &it, const pk_i4_shape &sh, int epilogue
                        sh.RB, lim, alpha)
         if (epilogue == PK_EPI_SWIGLU) {
             if (dot) PK_I4_STREAM(PK_EPI_SWIGLU, true); else PK_I4_STREAM(PK_EPI_SWIGLU, false);
+        } else if (epilogue == PK_EPI_ROW_SCALED) {
+            PK_I4_STREAM(PK_EPI_ROW_SCALED, false);
         } else {
             if (dot) PK_I4_STREAM(PK_EPI_PLAIN, true); else PK_I4_STREAM(PK_EPI_PLAIN, false);
         }
@@ -548,6 +558,8 @@ int pk_launch_i4_gemv(const pk_i4_items &it, const pk_i4_shape &sh, int epilogue
     hipLaunchKernelGGL((k_i4_gemv_part<E, R, G>), grid, dim3(PR_NW * 64), lds, st, it, sh.O, sh.NG, lim, alpha)
         if (epilogue == PK_EPI_SWIGLU) {
             if (quarter) PK_I4_PART(PK_EPI_SWIGLU, 16, 1); else PK_I4_PART(PK_EPI_SWIGLU, 32, 2);
+        } else if (epilogue == PK_EPI_ROW_SCALED) {
+            if (quarter) PK_I4_PART(PK_EPI_ROW_SCALED, 16, 1); else PK_I4_PART(PK_EPI_ROW_SCALED, 32, 2);
         } else {
             if (quarter) PK_I4_PART(PK_EPI_PLAIN, 16, 1); else PK_I4_PART(PK_EPI_PLAIN, 32, 2);
         }
@@ -567,6 +579,8 @@ int pk_launch_i4_gemv(const pk_i4_items &it, const pk_i4_shape &sh, int epilogue
         if (dot) PK_I4_LAUNCH(PK_EPI_SWIGLU, true); else PK_I4_LAUNCH(PK_EPI_SWIGLU, false);
     } else if (epilogue == PK_EPI_COMBINE) {
         if (dot) PK_I4_LAUNCH(PK_EPI_COMBINE, true); else PK_I4_LAUNCH(PK_EPI_COMBINE, false);
+    } else if (epilogue == PK_EPI_ROW_SCALED) {
+        PK_I4_LAUNCH(PK_EPI_ROW_SCALED, false);
     } else {
         if (dot) PK_I4_LAUNCH(PK_EPI_PLAIN, true); else PK_I4_LAUNCH(PK_EPI_PLAIN, false);
     }
@@ -893,10 +907,10 @@ int pk_launch_i4_gemv_ref(float *y, const float *x, const uint8_t *q4, const flo
 
 // ───────────────────────── repack ─────────────────────────
 // Reference layout (q4 [O][I/2], s [O][I/64]) -> tiles + 16*scale.
-// One thread per (row of the padded block, group). sng: scales per row in s
-// (NG, or 1: a row scale, stored for every group).
+// One thread per (row of the padded block, group). row_scale: s [O], stored as
+// it is for every group (16*s could overflow where scale x sum does not).
 __global__ void k_i4_repack(const uint8_t *q4, const float *s, int O, int I, int RB, int NG,
-                            uint8_t *tiles, float *sc16, int sng) {
+                            uint8_t *tiles, float *sc16, bool row_scale) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (int64_t)RB * 64 * NG) return;
     const int g = (int)(t % NG);
@@ -911,7 +925,7 @@ __global__ void k_i4_repack(const uint8_t *q4, const float *s, int O, int I, int
         for (int k = 0; k < 8; ++k) v[k] = src[k] ^ 0x88888888u;
         lo = make_uint4(v[0], v[1], v[2], v[3]);
         hi = make_uint4(v[4], v[5], v[6], v[7]);
-        scv = 16.0f * s[(int64_t)row * sng + (sng > 1 ? g : 0)];
+        scv = row_scale ? s[row] : 16.0f * s[(int64_t)row * NG + g];
     }
     uint4 *dst = reinterpret_cast<uint4 *>(tiles + ((int64_t)rb * NG + g) * PK_TILE_BYTES);
     dst[r] = lo;
@@ -926,7 +940,7 @@ int pk_launch_i4_repack(const uint8_t *q4, const float *s, int O, int I,
     const pk_i4_shape sh = pk_i4_make_shape(O, I);
     const int64_t n = (int64_t)sh.RB * 64 * sh.NG;
     hipLaunchKernelGGL(k_i4_repack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                       q4, s, O, I, sh.RB, sh.NG, tiles, sc16, row_scale ? 1 : sh.NG);
+                       q4, s, O, I, sh.RB, sh.NG, tiles, sc16, row_scale);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }

@@ -115,6 +115,27 @@ __device__ __forceinline__ float pk_fold_groups(const float *part, const float *
     return acc;
 }
 
+// The same partials where every group has the row's one scale (not multiplied
+// by 16) and no order is prescribed: scale x 16 p_g over four interleaved
+// chains, added pairwise. stride: values per group. (One chain's roundings
+// grow with the groups: 2880 columns 1.40e-7 relative against 64 bits; the
+// byte-per-lane kernel these launches replace 1.38e-7.)
+__device__ __forceinline__ float pk_fold_row_scaled(const float *part, const float *scl, int NG, int stride) {
+    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int g0 = 0; g0 < NG; g0 += 8) {
+        float p[8], q[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            p[j] = part[min(g0 + j, NG - 1) * stride];
+            q[j] = scl[min(g0 + j, NG - 1) * stride];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (g0 + j < NG) a[j & 3] = __builtin_fmaf(16.0f * p[j], q[j], a[j & 3]);
+    }
+    return (a[0] + a[1]) + (a[2] + a[3]);
+}
+
 // expf as the double exp rounded once to float: the correctly rounded value
 // (but for double rounding in about 2^-29 of inputs), which is glibc's expf
 // except where glibc's own result is not correctly rounded (~8e-5 of inputs).

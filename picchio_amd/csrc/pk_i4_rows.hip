@@ -175,7 +175,8 @@ __device__ __forceinline__ void rw_body(const pk_i4_items &it, const int32_t *pa
         for (int s = 0; s < NS; ++s) d.x[s] = *reinterpret_cast<const float4 *>(xp[s] + g * 64);
     };
     // the row's sum so far, handed from wave to wave (and span to span) in
-    // group order: a = fma(partial, scale, a)
+    // group order: a = fma(partial, scale, a). With a scale per row (no
+    // prescribed order) each wave's groups sum on their own and are added.
     f32x4 acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -193,20 +194,30 @@ __device__ __forceinline__ void rw_body(const pk_i4_items &it, const int32_t *pa
         }
         for (int w = 0; w < RW_WAVES; ++w) {
             if (w == wave) {
-                if (b0 + w > 0) {
+                f32x4 prev[NS];
 #pragma unroll
-                    for (int s = 0; s < NS; ++s)
+                for (int s = 0; s < NS; ++s)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[s][i] = accs[4 * s + i][lane];
-                }
+                    for (int i = 0; i < 4; ++i) {
+                        prev[s][i] = b0 + w > 0 ? accs[4 * s + i][lane] : 0.0f;
+                        acc[s][i] = EPI == PK_EPI_ROW_SCALED ? 0.0f : prev[s][i];
+                    }
 #pragma unroll
                 for (int u = 0; u < RW_GW; ++u)
                     if (g0 + u < NG) {
 #pragma unroll
                         for (int s = 0; s < NS; ++s)
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) acc[s][i] = __builtin_fmaf(p[u][s][i], sv[u], acc[s][i]);
+                            for (int i = 0; i < 4; ++i)
+                                acc[s][i] = __builtin_fmaf(
+                                    EPI == PK_EPI_ROW_SCALED ? 16.0f * p[u][s][i] : p[u][s][i], sv[u], acc[s][i]);
                     }
+                if constexpr (EPI == PK_EPI_ROW_SCALED) {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[s][i] = prev[s][i] + acc[s][i];
+                }
 #pragma unroll
                 for (int s = 0; s < NS; ++s)
 #pragma unroll
@@ -448,7 +459,8 @@ int pk_launch_i4_rows(const pk_i4_items &it, const pk_i4_tiles *tl, const pk_i4_
     PK_CHECK(sh.NG > 0 && sh.RB > 0 && it.n_items > 0 && it.x_div > 0, PK_ERR_ARG, "i4 rows: empty shape");
     PK_CHECK(!tl || (tl->pairs && tl->tile_exp && tl->tile_beg && tl->tile_cnt && tl->n_tiles), PK_ERR_ARG,
              "i4 rows: missing tiles");
-    PK_CHECK(tile_rows == 8 || tile_rows == 16, PK_ERR_ARG, "i4 rows: tiles of %d", tile_rows);
+    PK_CHECK(tile_rows == 8 || (tile_rows == 16 && epilogue != PK_EPI_ROW_SCALED), PK_ERR_ARG, "i4 rows: tiles of %d",
+             tile_rows);
     // one matrix: tiles of 8 rows, but of 4 where tiles of 8 would leave CUs
     // without a workgroup (5760 x 2880, 8 rows: 9.5 against 13.6 us)
     int tile = tile_rows;
@@ -471,6 +483,9 @@ int pk_launch_i4_rows(const pk_i4_items &it, const pk_i4_tiles *tl, const pk_i4_
     if (epilogue == PK_EPI_SWIGLU)
         hipLaunchKernelGGL(k_i4_rows<PK_EPI_SWIGLU>, grid, dim3(RW_WAVES * 64), 0, st, it, tl ? *tl : none, tile, sh.O,
                            sh.NG, lim, alpha);
+    else if (epilogue == PK_EPI_ROW_SCALED)
+        hipLaunchKernelGGL(k_i4_rows<PK_EPI_ROW_SCALED>, grid, dim3(RW_WAVES * 64), 0, st, it, none, tile, sh.O, sh.NG,
+                           lim, alpha);
     else
         hipLaunchKernelGGL(k_i4_rows<PK_EPI_PLAIN>, grid, dim3(RW_WAVES * 64), 0, st, it, tl ? *tl : none, tile, sh.O,
                            sh.NG, lim, alpha);

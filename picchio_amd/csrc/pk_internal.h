@@ -144,7 +144,8 @@ struct pk_i4_items {
 // (pk_i4_device.h: five digit planes of 4 dwords, the exponent, padding)
 constexpr int PK_XQ_INTS = 24;
 
-enum pk_i4_epilogue { PK_EPI_PLAIN = 0, PK_EPI_SWIGLU = 1, PK_EPI_COMBINE = 2 };
+// PK_EPI_ROW_SCALED: PLAIN of a tensor with one scale per row (pk_fold_row_scaled)
+enum pk_i4_epilogue { PK_EPI_PLAIN = 0, PK_EPI_SWIGLU = 1, PK_EPI_COMBINE = 2, PK_EPI_ROW_SCALED = 3 };
 
 struct pk_combine_args {
     const float *w;           // [n_items] routing weights (already * routed_scale), device

@@ -75,3 +75,36 @@ def test_i4_few_row_blocks_match_many(gpu, n):
             got.append((eng.to_host(act)[:n], eng.to_host(eo)[:n]))
     for a, b in zip(*got):
         assert bits_equal(a, b), first_mismatch(a, b)
+
+
+@pytest.mark.parametrize("O,I,S", [(130, 128, 1), (200, 3136, 3), (70, 6208, 131), (12000, 2880, 1), (33000, 192, 1),
+                                   (700, 8192, 33), (2880, 2880, 1), (5120, 2880, 17)])
+def test_i4_row_scales_in_tiles_bound(gpu, oracle, O, I, S):
+    """A scale per row in the tile layout (halves and quarters of row blocks,
+    whole ones, the streaming launch, several rows), against the exact sum
+    over the stored integers. The order is free: at most D roundings lie
+    between a product and its output, D = 8 in a group's chain + 3 in its
+    tree, ceil(NG / 4) in a fold chain or 12 + NG / 12 in the rows kernel, + 4
+    for the product, the last sums and the scale."""
+    import picchio_amd as pa
+    import torch
+    w = _rand((O, I), 7 + O + I, 0.02)
+    q4, s = oracle.quant_gs(w, 0)
+    s = np.asarray(s, np.float32).reshape(-1)
+    x = _rand((S, I), 13 + S)
+    s[0] = np.float32(2.0 ** 125)                 # 16 x the scale alone would overflow
+    x *= np.float32(2.0 ** -10)
+    b = np.asarray(q4).reshape(O, I // 2)
+    q = np.empty((O, I), np.float64)
+    q[:, 0::2], q[:, 1::2] = (b & 15).astype(np.float64) - 8, (b >> 4).astype(np.float64) - 8
+    with pa.Engine(pa.gptoss_cfg(n_layers=1, n_experts=4, ctx_len=16, vocab=64)) as eng:
+        qt = eng.qt_upload(pa.FMT_INT4, q4, s, O, I, 0)
+        yd = eng.empty((S, O), torch.float32)
+        eng.matmul_qt(yd, eng.to_dev(x), qt, S)
+        y = eng.to_host(yd).reshape(S, O).astype(np.float64)
+        eng.qt_free(qt)
+    sd, xd, ng = s.astype(np.float64), x.astype(np.float64), I // 64
+    exact = (xd @ q.T) * sd
+    depth = 8 + 3 + max(-(-ng // 4), 12 + ng // 12) + 4
+    bound = (np.abs(xd) @ np.abs(q).T) * sd * depth * 2.0 ** -24
+    assert (np.abs(y - exact) <= bound).all()
