@@ -2,9 +2,11 @@
 // picchio.c:1509-1649), so that a decode loop with temperature / top-k /
 // top-p / repetition penalty never leaves the GPU.
 //
-// One workgroup of 1024 threads per draw. For a pass over the vocabulary
-// wave w owns the w-th sixteenth, with 16 loads in flight per lane. Steps,
-// in the reference's order:
+// A draw over a large vocabulary is spread over the device (the launches after
+// k_sample below); greedy draws, small vocabularies, the exact-sum option and
+// a top-k beyond CAND run in k_sample alone: one workgroup of 1024 threads,
+// wave w owning the w-th sixteenth of the vocabulary in each pass, with 16
+// loads in flight per lane. Steps, in the reference's order:
 //   1. repetition penalty: once per history entry (a token that appears c
 //      times is divided / multiplied c times, as the reference's loop does);
 //   2. temperature below 1e-6: the first maximum (greedy), no draw;
@@ -18,16 +20,14 @@
 //   5. softmax, top-p over the probabilities > 1e-10, the draw.
 // A logit below the top-k threshold becomes -1e30 and then exactly 0 in the
 // reference, so its float sums equal the same sums over the kept entries in
-// index order, one term at a time. Every sum here is made in that order by
-// one lane: from LDS when at most SMALL entries are kept (every top-k up to
-// 4096), else from global memory staged through LDS by the other waves. The
-// top-p list is sorted descending with equal values by index (what glibc's
+// index order, one term at a time. Up to SMALL kept entries one lane makes
+// each sum in that order from LDS; beyond, a workgroup (order_sum) or, without
+// a top-k, the device (om_sum) scans to the same bits. The top-p list is sorted descending with equal values by index (what glibc's
 // merge sort leaves): in LDS for up to SMALL entries, beyond that chunk by
 // chunk (a radix select on 64-bit (key, ~index) finds each chunk's bound) with
 // the running sum carried across. The array left behind and the draw equal
 // the reference's up to the device expf's last ulp.
-// A serial sum over a 200k vocabulary costs about half a millisecond; the
-// opt-in fast_sums mode makes those sums exact instead (64-bit integers of
+// The opt-in fast_sums mode makes those sums exact instead (64-bit integers of
 // the values scaled by a power of two, rounded once), which any order gives:
 // the top-p cut is the shortest descending prefix whose exact sum reaches
 // top_p (a radix descent carrying counts and exact sums, ties by index) and
@@ -51,6 +51,7 @@ constexpr int FX_P = 62;                  // fixed-point bits for probabilities 
 // Scratch of the launches that spread a draw over the device (zeroed when
 // allocated; the counters are re-armed by the launch that reads them last).
 constexpr int SB_BINS = 4096;
+constexpr int SAMP_RUNS = 4096;
 struct samp_ws {
     uint32_t hist[SB_BINS];
     uint32_t cur[SB_BINS * 16];           // a bucket's cursor, 64 bytes apart: neighbours do not share a line
@@ -63,6 +64,9 @@ struct samp_ws {
     uint32_t unsorted;                    // 1: a bucket exceeds what a workgroup sorts
     float cv[CAND];
     int32_t ci[CAND];
+    float part[SAMP_RUNS];                // the ordered sum's runs: a plain sum,
+    uint2 mv[SAMP_RUNS];                  // the pair of moves in one binade,
+    int32_t mex[SAMP_RUNS];               // and that binade
 };
 
 __device__ __forceinline__ uint32_t key_of(float f) {
@@ -386,6 +390,20 @@ __device__ __forceinline__ uint2 os_scan(uint2 a) {
     return a;
 }
 
+// The pair of moves of a thread's OS_E elements in binade ex (s = S 2^(ex - 150)).
+__device__ __forceinline__ uint2 os_moves(const float (&v)[OS_E], int ex) {
+    uint2 d = make_uint2(0u, 0u);                          // (x: from S even, y: from S odd)
+#pragma unroll
+    for (int k = 0; k < OS_E; ++k) {
+        // (past the binade, infinite or NaN: OS_BIG)
+        const float t = fminf(ldexpf(v[k], 150 - ex), (float)OS_BIG);
+        const float q = rintf(t), h = t - q;               // a tie goes to even: the move for S even
+        const float qo = q + (fabsf(h) == 0.5f ? h + h : 0.0f);
+        d = os_then(d, make_uint2((uint32_t)q, (uint32_t)qo));
+    }
+    return os_clamp(d);
+}
+
 // find: stop at the first index whose running sum is >= r. Leaves the sum (up
 // to there) in *s_out and that index (or -1) in *hit_out; s0: where the sum
 // starts. Every thread of the workgroup calls it (buf: OS_BUF floats).
@@ -420,16 +438,7 @@ __device__ __forceinline__ void order_sum(const float *src, int n, float *buf, b
             const uint32_t sb = __float_as_uint(s);
             const int ex = max((int)(sb >> 23), 1);        // s = S 2^(ex - 150)
             const uint32_t S = (sb & 0x7fffffu) | ((sb >> 23) ? 0x800000u : 0u);
-            uint2 d = make_uint2(0u, 0u);                  // (x: from S even, y: from S odd)
-#pragma unroll
-            for (int k = 0; k < OS_E; ++k) {
-                // (past the binade, infinite or NaN: OS_BIG)
-                const float t = fminf(ldexpf(v[k], 150 - ex), (float)OS_BIG);
-                const float q = rintf(t), h = t - q;       // a tie goes to even: the move for S even
-                const float qo = q + (fabsf(h) == 0.5f ? h + h : 0.0f);
-                d = os_then(d, make_uint2((uint32_t)q, (uint32_t)qo));
-            }
-            d = os_clamp(d);
+            const uint2 d = os_moves(v, ex);
             const uint2 inc = os_scan<true>(d);
             __syncthreads();                               // (s_wave, os_* of the last round are read)
             if (lane == 63) s_wave[wave] = os_clamp(inc);
@@ -1264,15 +1273,16 @@ __global__ __launch_bounds__(SH_T) void k_samp_gather(float *lg, int V, const pk
 
 // ───────────── a draw over the device: no top-k ─────────────
 // The reference's steps as launches of their own: the elementwise ones on
-// every CU, the ordered float sums on one workgroup (order_sum). The top-p
+// every CU, the ordered float sums as runs (om_sum). The top-p
 // list is sorted by buckets: the candidates (> 1e-10) are counted by the
 // upper bits of their value (64 buckets per binade, at most 2131), placed
 // into their buckets, the largest first, and each bucket is sorted in LDS by
 // its own workgroup (equal values need no order: a sum does not tell them
 // apart, and the cut takes ties by index). Where a bucket exceeds SORT_CAP
 // different values, one workgroup takes the list chunk by chunk instead.
-// Measured, 201,088 entries of a peaked distribution, top-p 0.95: 400 us
-// per draw against 5,000 to 6,000 in one workgroup.
+// Measured, 201,088 entries of a peaked distribution, top-p 0.95: 252 us
+// per draw against 5,000 to 6,000 in one workgroup; 396 with each ordered sum
+// on one workgroup (100 us, 75 in the draw; 30 + 8 and 32 + 8 as runs).
 constexpr int SORT_CAP = 4096;
 constexpr uint32_t P_MIN = 0x2edbe6ffu;   // bits of 1e-10f
 constexpr int P_SHIFT = 17;
@@ -1320,15 +1330,161 @@ __global__ __launch_bounds__(SH_T) void k_samp_exp(float *lg, int V, const samp_
         if (j0 + SH_T * k < V) lg[j0 + SH_T * k] = expf(v[k] - mx);
 }
 
-// ws->sum = the ordered sum of src[0..n)
-__global__ __launch_bounds__(SNT) void k_samp_sum(const float *src, int n, samp_ws *ws) {
-    __shared__ __align__(16) float buf[OS_BUF];
-    __shared__ float s_sum;
-    __shared__ int s_hit;
+// The ordered sum over the device. order_sum walks the array with one
+// workgroup (201,088 entries: 25 chunks of 8192 and a round per binade, 2.3 us
+// each: 100 us). A run's pair of moves depends only on the binade of the sum
+// before it, so every wave composes its run's pair for the binade that a plain
+// float sum of the runs before it predicts (k_samp_part, k_samp_moves), and one
+// wave then scans the pairs, 64 runs at a time, in the exact sum. A run whose
+// prediction was wrong, or in which the sum passes a binade or the draw, is
+// added element by element from the array, as order_sum adds it: the
+// predictions decide what is fast, never the result.
+constexpr int OM_RUN = 64 * OS_E;         // elements of a wave's pass; a run is `per` of them
+static int om_per(int n) { return (n + OM_RUN * SAMP_RUNS - 1) / (OM_RUN * SAMP_RUNS); }
+static int om_runs(int n) { return (n + OM_RUN * om_per(n) - 1) / (OM_RUN * om_per(n)); }
+
+// part[c] = run c's sum, in any order
+__global__ __launch_bounds__(SH_T) void k_samp_part(const float *src, int n, int per, int runs, samp_ws *ws) {
+    const int lane = threadIdx.x & 63, c = blockIdx.x * (SH_T / 64) + (threadIdx.x >> 6);
+    if (c >= runs) return;
+    float sum = 0.0f;
+    for (int p = 0; p < per; ++p) {
+        const int64_t b = ((int64_t)c * per + p) * OM_RUN + lane;
+        float v[OS_E];
+#pragma unroll
+        for (int k = 0; k < OS_E; ++k) v[k] = src[min(b + 64 * k, (int64_t)n - 1)];
+#pragma unroll
+        for (int k = 0; k < OS_E; ++k) sum += b + 64 * k < n ? v[k] : 0.0f;
+    }
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if (lane == 0) ws->part[c] = sum;
+}
+
+// This lane's OS_E elements of the pass at b (zeros past n: + 0 leaves a sum as it is).
+__device__ __forceinline__ void om_load(const float *src, int n, int64_t b, float (&v)[OS_E]) {
+    const int64_t j = b + OS_E * (threadIdx.x & 63);
+    float t[OS_E];
+#pragma unroll
+    for (int k = 0; k < OS_E; ++k) t[k] = src[min(j + k, (int64_t)n - 1)];
+#pragma unroll
+    for (int k = 0; k < OS_E; ++k) v[k] = j + k < n ? t[k] : 0.0f;
+}
+
+// mv[c], mex[c] = run c's pair of moves, and the binade it holds in
+__global__ __launch_bounds__(SH_T) void k_samp_moves(const float *src, int n, int per, int runs, samp_ws *ws) {
+    const int lane = threadIdx.x & 63, c = blockIdx.x * (SH_T / 64) + (threadIdx.x >> 6);
+    if (c >= runs) return;
+    float v[OS_E];
+    om_load(src, n, (int64_t)c * per * OM_RUN, v);
+    float s = 0.0f;
+    for (int i = lane; i < c; i += 64) s += ws->part[i];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    const int ex = max((int)((__float_as_uint(s) >> 23) & 0xffu), 1);
+    uint2 all = make_uint2(0u, 0u);
+    for (int p = 0; p < per; ++p) {
+        if (p) om_load(src, n, ((int64_t)c * per + p) * OM_RUN, v);
+        const uint2 inc = os_scan<true>(os_moves(v, ex));
+        all = os_clamp(os_then(all, make_uint2((uint32_t)__builtin_amdgcn_readlane((int)inc.x, 63),
+                                               (uint32_t)__builtin_amdgcn_readlane((int)inc.y, 63))));
+    }
+    if (lane == 0) {
+        ws->mv[c] = all;
+        ws->mex[c] = ex;
+    }
+}
+
+// The sum of src[0..n) in index order on one wave, over the runs' moves; find:
+// stop at the first index whose running sum is >= r (-1: none).
+__device__ __forceinline__ float om_sum(const float *src, int n, int per, int runs, const samp_ws *ws, bool find,
+                                        float r, int &hit) {
+    __shared__ uint2 mv[SAMP_RUNS];
+    __shared__ int mex[SAMP_RUNS];
+    const int lane = threadIdx.x & 63;
+    for (int i = lane; i < runs; i += 64) {
+        mv[i] = ws->mv[i];
+        mex[i] = ws->mex[i];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    hit = -1;
+    float s = 0.0f;
+    for (int c = 0; c < runs;) {
+        {
+            const uint32_t sb = __float_as_uint(s);
+            const int ex = max((int)(sb >> 23), 1);
+            const uint32_t S = (sb & 0x7fffffu) | ((sb >> 23) ? 0x800000u : 0u);
+            const int i = min(c + lane, runs - 1);
+            const bool ok = c + lane < runs && mex[i] == ex;
+            const uint2 inc = os_scan<true>(ok ? mv[i] : make_uint2(OS_BIG, OS_BIG));
+            const uint32_t S1 = S + ((S & 1u) ? inc.y : inc.x);
+            const uint64_t bad =
+                __ballot(!ok || S1 >= 0x1000000u || (find && ldexpf((float)min(S1, OS_BIG), ex - 150) >= r));
+            const int f = bad ? __builtin_ctzll(bad) : 64;
+            if (f > 0) s = ldexpf((float)(uint32_t)__builtin_amdgcn_readlane((int)S1, f - 1), ex - 150);
+            c += f;
+            if (f == 64 || c >= runs) continue;
+        }
+        for (int p = 0; p < per; ++p) {
+            const int64_t base = ((int64_t)c * per + p) * OM_RUN;
+            if (base >= n) break;
+            float v[OS_E];
+            om_load(src, n, base, v);
+            for (int start = 0; start < OM_RUN;) {         // the pass's elements before it are in s
+                const uint32_t sb = __float_as_uint(s);
+                const int ex = max((int)(sb >> 23), 1);
+                const uint32_t S = (sb & 0x7fffffu) | ((sb >> 23) ? 0x800000u : 0u);
+                const uint2 d = os_moves(v, ex);
+                const uint2 inc = os_scan<true>(d), pre = os_dpp<0x138, 0xf>(inc);
+                const bool odd = S & 1u;
+                const uint32_t S0 = S + (odd ? pre.y : pre.x);         // before this lane's elements
+                const uint32_t S1 = S0 + ((S0 & 1u) ? d.y : d.x);
+                const float a0 = ldexpf((float)min(S0, OS_BIG), ex - 150);
+                const bool cross = S0 < 0x1000000u && S1 >= 0x1000000u;
+                const bool hits = find && S0 < 0x1000000u && !cross && ldexpf((float)S1, ex - 150) >= r &&
+                                  (!(a0 >= r) || OS_E * lane <= start);
+                float x = a0;
+                int at = -1;
+                if (cross || hits)
+#pragma unroll
+                    for (int k = 0; k < OS_E; ++k)
+                        if (at < 0) {
+                            x = x + v[k];
+                            if (find && x >= r) at = k;
+                        }
+                const uint64_t got = __ballot(at >= 0), over = __ballot(cross);
+                if (got) {
+                    const int f = __builtin_ctzll(got);
+                    hit = (int)base + OS_E * f + __builtin_amdgcn_readlane(at, f);
+                    return s;
+                }
+                if (over) {
+                    const int f = __builtin_ctzll(over);
+                    s = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), f));
+                    start = OS_E * (f + 1);
+                } else {
+                    s = ldexpf((float)(uint32_t)__builtin_amdgcn_readlane((int)S1, 63), ex - 150);
+                    start = OM_RUN;
+                }
+                if (!(s < INFINITY)) return s;             // NaN stays NaN, infinity stays
+                if (OS_E * lane < start) {                 // (whole lanes: in s)
+#pragma unroll
+                    for (int k = 0; k < OS_E; ++k) v[k] = 0.0f;
+                }
+            }
+        }
+        ++c;
+    }
+    return s;
+}
+
+// ws->sum = the ordered sum of src[0..n), after its k_samp_part and k_samp_moves
+__global__ __launch_bounds__(64) void k_samp_sum(const float *src, int n, int per, int runs, samp_ws *ws) {
     if (ws->cut == 2) return;
-    order_sum(src, n, buf, false, 0.0f, &s_sum, &s_hit);
+    int hit;
+    const float s = om_sum(src, n, per, runs, ws, false, 0.0f, hit);
     if (threadIdx.x == 0) {
-        ws->sum = s_sum;
+        ws->sum = s;
         ws->mx_key = 0;                               // (read; re-armed)
     }
 }
@@ -1520,10 +1676,9 @@ __global__ __launch_bounds__(SH_T) void k_samp_zero(float *lg, int V, const samp
 }
 
 // The draw: the first index whose ordered running sum reaches it.
-__global__ __launch_bounds__(SNT) void k_samp_draw(const float *lg, int V, pk_sampler_dev *sp, samp_ws *ws,
-                                                   pk_dstate *st, int32_t *out_toks, int out_cap) {
-    __shared__ __align__(16) float buf[OS_BUF];
-    __shared__ float s_sum, s_r;
+__global__ __launch_bounds__(SNT) void k_samp_draw(const float *lg, int V, int per, int runs, pk_sampler_dev *sp,
+                                                   samp_ws *ws, pk_dstate *st, int32_t *out_toks, int out_cap) {
+    __shared__ float s_r;
     __shared__ int s_hit, s_redi[NW];
     const int tid = threadIdx.x;
     if (tid == 0) {
@@ -1538,7 +1693,12 @@ __global__ __launch_bounds__(SNT) void k_samp_draw(const float *lg, int V, pk_sa
     }
     __syncthreads();
     const float r = s_r;
-    order_sum(lg, V, buf, true, r, &s_sum, &s_hit);
+    if (tid < 64) {
+        int hit;
+        (void)om_sum(lg, V, per, runs, ws, true, r, hit);
+        if (tid == 0) s_hit = hit;
+    }
+    __syncthreads();
     int pick = s_hit;
     if (pick < 0) {
         // nothing reached r: the last entry with probability > 0
@@ -1627,9 +1787,17 @@ int pk_launch_sample(pk_engine *e, float *logits, int vocab, pk_dstate *st, int3
     } while (0)
     if (kind == SAMP_NUCLEUS) {
         const bool cut = e->samp_params.top_p < 1.0f && e->samp_params.top_p > 0.0f;
+        const int per = om_per(vocab), runs = om_runs(vocab);
+        const dim3 waves((runs + SH_T / 64 - 1) / (SH_T / 64));
+#define PK_SUM()                                                               \
+    do {                                                                       \
+        PK_SAMP(k_samp_part, waves, SH_T, logits, vocab, per, runs, ws);       \
+        PK_SAMP(k_samp_moves, waves, SH_T, logits, vocab, per, runs, ws);      \
+    } while (0)
         PK_SAMP(k_samp_scale, grid, SH_T, logits, vocab, e->samp, ws);
         PK_SAMP(k_samp_exp, grid, SH_T, logits, vocab, ws);
-        PK_SAMP(k_samp_sum, 1, SNT, logits, vocab, ws);
+        PK_SUM();
+        PK_SAMP(k_samp_sum, 1, 64, logits, vocab, per, runs, ws);
         PK_SAMP(k_samp_div, grid, SH_T, logits, vocab, ws, cut ? 1 : 2);
         if (cut) {
             PK_SAMP(k_samp_offsets, 1, SNT, ws);
@@ -1637,10 +1805,13 @@ int pk_launch_sample(pk_engine *e, float *logits, int vocab, pk_dstate *st, int3
             PK_SAMP(k_samp_sort, P_BINS, SH_T, ws, e->samp_av);
             PK_SAMP(k_samp_cut, 1, SNT, logits, vocab, e->samp, ws, e->samp_av);
             PK_SAMP(k_samp_zero, grid, SH_T, logits, vocab, ws);
-            PK_SAMP(k_samp_sum, 1, SNT, logits, vocab, ws);
+            PK_SUM();
+            PK_SAMP(k_samp_sum, 1, 64, logits, vocab, per, runs, ws);
             PK_SAMP(k_samp_div, grid, SH_T, logits, vocab, ws, 0);
         }
-        PK_SAMP(k_samp_draw, 1, SNT, logits, vocab, e->samp, ws, st, out_toks, out_cap);
+        PK_SUM();
+        PK_SAMP(k_samp_draw, 1, SNT, logits, vocab, per, runs, e->samp, ws, st, out_toks, out_cap);
+#undef PK_SUM
         return PK_OK;
     }
     if (kind == SAMP_TOPK) {

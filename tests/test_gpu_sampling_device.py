@@ -63,3 +63,13 @@ def test_crowded_bucket(samp_eng, oracle):  # noqa: F811
     # descending order: nothing kept lies below anything dropped, but where
     # expf (an ulp off, 2^-23 near 1) and the division (2^-24) give one value
     assert x[got != 0].min() >= x[got == 0].max() - 2.0 ** -22
+
+
+@pytest.mark.parametrize("case", [(1.0, 1.0, 0, 1.0), (1.0, 0.9, 0, 1.0)], ids=["draw", "top-p"])
+@pytest.mark.parametrize("size", [16384, 33281, 524801, 2200003])
+def test_ordered_sum_runs(samp_eng, oracle, case, size):  # noqa: F811
+    """Runs of the ordered sum at their edges: whole, one entry over, more than
+    1024 of them, two passes per run. Equal logits: exp(0) = 1, so the device's
+    expf is exact."""
+    _check_draws(samp_eng, oracle, case, size, 2, lambda s: np.zeros(size, np.float32))
+    samp_eng.set_sampling(0.0, 1.0, 0, 1.0, 1)
