@@ -886,7 +886,7 @@ def measure_moe_layer(args):
         "gate_up_us": round(ffn_gu_ms * 1e3, 3), "down_us": round((ffn_ms - ffn_gu_ms) * 1e3, 3),
         "roofline": {"bound": "hbm", "achieved": round(ffn_gbps, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": round(ffn_gbps / HBM_PEAK_GBPS, 4), "traffic": FFN_TRAFFIC,
-                     "kernel": "k_i4_gemv<SWIGLU> (gate_up) then k_i4_gemv<PLAIN> (down), one expert, "
+                     "kernel": "k_i4_gemv_part<SWIGLU> (gate_up) then k_i4_gemv_part<PLAIN> (down), one expert, "
                                "fp32 chains (expert_apply's arithmetic, bit-exact with quant.h)",
                      "bytes_per_launch": FFN_BYTES, "mean_us": round(ffn_ms * 1e3, 3)},
         "cpu_baseline": cpu0,

@@ -416,8 +416,8 @@ int pk_sample_logits(pk_engine *e, float *logits_dev, int vocab, int32_t *tok_ho
  * exactly, as 64-bit integers of the values times a power of two, rounded to
  * float once, instead of one at a time in the reference's order; the top-p
  * cut is the shortest descending prefix whose exact sum reaches top_p and the
- * pick the first index whose exact running sum reaches the draw. About ten
- * times faster there; the probabilities differ from the reference's by its
+ * pick the first index whose exact running sum reaches the draw. About as
+ * fast as the ordered sums; the probabilities differ from the reference's by its
  * own float rounding (about 1e-5 relative at 200k entries), which over a
  * flat distribution moves a top-p cut or a pick now and then. Draws keeping
  * up to 4096 entries are unaffected. Default off. */

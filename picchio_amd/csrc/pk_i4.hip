@@ -247,9 +247,7 @@ __global__ __launch_bounds__(PR_NW * 64) void k_i4_gemv_part(pk_i4_items it, int
 // and writes its rows while the others move on. Two cumulative LDS counters
 // per buffer order them (partials in; fold done). The same per-row
 // arithmetic as k_i4_gemv, hence the same bits. Measured: 32 experts'
-// gate_up in one launch 4.3 -> 4.5 TB/s, the 512-token prompt of config 2
-// (its per-pair expert GEMVs) 0.43 -> 0.41 s; a ring of three slots was no
-// faster.
+// gate_up in one launch 4.3 -> 4.5 TB/s; a ring of three slots was no faster.
 constexpr int ST_NW = 15, ST_GPW = 3;     // load waves x groups per wave: NG <= 45
 
 __device__ __forceinline__ void st_signal(int *c) {

@@ -3,13 +3,16 @@
 //
 // A prompt runs in chunks of PREFILL_BATCH positions (64 unless the
 // environment says otherwise, read as picchio.c:1937-1938 reads it; 1 selects
-// the position-by-position path). Per chunk and layer, on n positions at once:
+// the position-by-position path); up to PREFILL_ROWS positions, as whole chunks,
+// take each layer together. Per layer, on n positions at once:
 //   RMSNorm -> QKV GEMV -> RoPE + KV store of every position -> causal /
 //   sliding attention of every position (each sees its own window) -> O
 //   projection + residual -> RMSNorm -> router logits -> top-k + softmax ->
-//   gate_up + SwiGLU and down over all n*K (token, expert) pairs, one launch
-//   each -> per-token sum in the chunk's expert order + residual.
-// Then the last position's final norm, lm_head and greedy argmax.
+//   gate_up + SwiGLU and down over all n*K (token, expert) pairs grouped by
+//   expert, one launch each -> per-token sum in the chunk's expert order +
+//   residual.
+// Then the last position's final norm, lm_head and greedy argmax (with sampling
+// on, each chunk's last position's).
 #include "pk_engine.h"
 
 #include <stdlib.h>
