@@ -77,7 +77,7 @@ def test_i4_few_row_blocks_match_many(gpu, n):
         assert bits_equal(a, b), first_mismatch(a, b)
 
 
-@pytest.mark.parametrize("O,I,S", [(130, 128, 1), (200, 3136, 3), (70, 6208, 131), (12000, 2880, 1), (33000, 192, 1),
+@pytest.mark.parametrize("O,I,S", [(130, 128, 1), (200, 3136, 3), (70, 6208, 131), (12000, 2880, 1), (33000, 192, 1), (5000, 8192, 1),
                                    (700, 8192, 33), (2880, 2880, 1), (5120, 2880, 17)])
 def test_i4_row_scales_in_tiles_bound(gpu, oracle, O, I, S):
     """A scale per row in the tile layout (halves and quarters of row blocks,
