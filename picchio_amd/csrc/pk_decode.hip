@@ -68,7 +68,10 @@ __device__ __forceinline__ void qkv_fma4(float &a, float4 x, pk_f32x4 w) {
     a = __builtin_fmaf(x.w, w.w, a);
 }
 
-__global__ __launch_bounds__(256) void k_qkv_rope_norm(const pk_dstate *st, const float *__restrict__ h,
+// NORM false: h is the input itself (one row at a host position), with the
+// bits of k_gemv_f32 + k_rope_kv: the same columns per lane, ascending.
+template <bool NORM>
+__global__ __launch_bounds__(256) void k_qkv_rope_norm(const pk_dstate *st, int host_pos, const float *__restrict__ h,
                                                        const float *__restrict__ nw, float eps,
                                                        const float *__restrict__ W, const float *__restrict__ b,
                                                        int D, int H, int KVH, int hd, int ctx, const float *rope,
@@ -106,23 +109,24 @@ __global__ __launch_bounds__(256) void k_qkv_rope_norm(const pk_dstate *st, cons
     // reads row 0 and writes nothing.
     float hv[12], nv[12];
     pk_rms_load(h, D, hv);
-    pk_rms_load(nw, D, nv);
+    if constexpr (NORM) pk_rms_load(nw, D, nv);
     const pk_buf_t wr = pk_buf(w4, (uint32_t)n4 * 16u);
     pk_f32x4 wf[QKV_U];
 #pragma unroll
     for (int u = 0; u < QKV_U; ++u) wf[u] = pk_buf_load4_nt(wr, (uint32_t)(lane + u * 64) * 16u);
-    const int pos = st->pos, kv_dim = KVH * hd;
+    const int pos = NORM ? st->pos : host_pos, kv_dim = KVH * hd;
     const float b0 = b[r0], b1 = b[r1];
     float cs = 0.0f, sn = 0.0f;
     if (pi < n_rot) {
         cs = rope[((int64_t)pos * half + j) * 2 + 0];
         sn = rope[((int64_t)pos * half + j) * 2 + 1];
     }
-    const float rn = pk_rms_finish(hv, h, D, eps, npart);
+    float rn = 1.0f;
+    if constexpr (NORM) rn = pk_rms_finish(hv, h, D, eps, npart);
     // (entries past the row are zeros on both sides: x = 0 * r * 0 in LDS,
     // w = 0 from the range check, so their products add nothing)
 #pragma unroll
-    for (int k = 0; k < 12; ++k) xn[threadIdx.x + 256 * k] = hv[k] * rn * nv[k];
+    for (int k = 0; k < 12; ++k) xn[threadIdx.x + 256 * k] = NORM ? hv[k] * rn * nv[k] : hv[k];
     __syncthreads();
     const float4 *xn4 = reinterpret_cast<const float4 *>(xn);
     float a = 0.0f;
@@ -137,7 +141,7 @@ __global__ __launch_bounds__(256) void k_qkv_rope_norm(const pk_dstate *st, cons
         for (int u = 0; u < 4; ++u) {
             const int i = i0 + u * 64;
             wv[u] = i < n4 ? __builtin_nontemporal_load(w4 + i) : pk_f32x4{0.f, 0.f, 0.f, 0.f};
-            xv[u] = i < n4 ? pk_norm4(h4[i], rn, n4w[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            xv[u] = i < n4 ? (NORM ? pk_norm4(h4[i], rn, n4w[i]) : h4[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) qkv_fma4(a, xv[u], wv[u]);
@@ -996,9 +1000,17 @@ int pk_attention_rows(pk_engine *e, int l, const pk_dstate *st, int pos_base, in
         PK_CHECK(((uintptr_t)xn & 15) == 0 && ((uintptr_t)norm_w & 15) == 0 && (D & 3) == 0,
                  PK_ERR_UNSUPPORTED, "qkv: needs 16-byte aligned rows");
         const int n_pairs = (H + 2 * KVH) * hd / 2;
-        hipLaunchKernelGGL(k_qkv_rope_norm, dim3((n_pairs + 1) / 2), dim3(256), 0, e->stream, st, xn, norm_w,
+        hipLaunchKernelGGL(k_qkv_rope_norm<true>, dim3((n_pairs + 1) / 2), dim3(256), 0, e->stream, st, 0, xn, norm_w,
                            c->eps, d.wqkv, d.bqkv, D, H, KVH, hd, c->ctx_len, e->rope, qkv, Kl, Vl,
                            e->counters + PK_CTR_ATT_EPOCH);
+        PK_HIP(hipGetLastError());
+    } else if (n == 1 && !st && !exact && qkv_dim > 2048 && hd % 2 == 0 && (D & 3) == 0 && d.bqkv &&
+               (((uintptr_t)xn | (uintptr_t)d.wqkv) & 15) == 0) {
+        // one row at a host position: QKV + bias + RoPE + KV store in one launch
+        // (2880 -> 5120: 12.0 us, 12.8 + 3.5 as two). Up to 2048 outputs a workgroup per row fills more CUs.
+        const int n_pairs = (H + 2 * KVH) * hd / 2;
+        hipLaunchKernelGGL(k_qkv_rope_norm<false>, dim3((n_pairs + 1) / 2), dim3(256), 0, e->stream, nullptr, pos_base,
+                           xn, nullptr, 0.0f, d.wqkv, d.bqkv, D, H, KVH, hd, c->ctx_len, e->rope, qkv, Kl, Vl, nullptr);
         PK_HIP(hipGetLastError());
     } else {
         // 4..32 rows with the workspace: the split sums + bias go into the RoPE launch
@@ -1183,8 +1195,9 @@ extern "C" int pk_gqa_attention(pk_engine *e, int layer, const float *x_dev, int
     PK_CHECK(!e->capturing, PK_ERR_ARG, "gqa_attention: host position; not available while capturing");
     PK_TRY(pk_decode_reserve(e));
     // straight from x_dev (read by the first launch only) into out_dev, the
-    // position as a launch argument: four launches and no copies around them
-    // (a sliding-window and a full layer at 4096 positions 127 -> 102 us)
+    // position as a launch argument: three launches and no copies around them
+    // (a sliding-window and a full layer at 4096 positions 127 -> 102 us; 95 with
+    // the rotation and KV store in the QKV launch)
     const float *x = x_dev;
     if ((uintptr_t)x_dev & 15) {
         PK_HIP(hipMemcpyAsync(e->hn, x_dev, (size_t)c->hidden * 4, hipMemcpyDeviceToDevice, e->stream));
