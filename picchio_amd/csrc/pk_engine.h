@@ -3,6 +3,10 @@
 
 #include "pk_internal.h"
 
+#include <atomic>
+#include <memory>
+#include <vector>
+
 struct pk_layer_dev {
     float *in_ln = nullptr, *post_ln = nullptr;
     float *wqkv = nullptr, *bqkv = nullptr;   // [(H + 2 KVH) hd][D], bias
@@ -106,6 +110,10 @@ struct pk_engine {
     uint64_t *att_t = nullptr;                // k_attn_oproj hand-over words: [heads x head_dim]
 
     bool capturing = false;                  // inside pk_capture_begin/end
+    // captured graphs (pk_graph) not yet destroyed, and the buffers outgrown
+    // while there were any: their kernels may address them (pk_regrow)
+    std::shared_ptr<std::atomic<int>> live_graphs = std::make_shared<std::atomic<int>>(0);
+    std::vector<void *> outgrown;
 
     // diagnostics (outside graph capture only): every MoE router launch
     // appends its logits [rows][E] to rtrace (pk_set_router_trace); with
@@ -184,6 +192,14 @@ int pk_noalloc_scratch_init(pk_engine *e);
 
 int pk_dev_alloc(pk_engine *e, void **p, int64_t bytes);
 void pk_dev_free(pk_engine *e, void *p);
+// Larger buffers in the place of *b[i].p (their contents are not kept). The
+// old ones are freed, or while a captured graph lives, kept for its kernels
+// until the next growth without one, or the engine's end.
+struct pk_buf_bytes {
+    void **p;
+    int64_t bytes;
+};
+int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n);
 int pk_stage_reserve(pk_engine *e, int64_t bytes);
 
 // kernels defined in pk_dense.hip / pk_attn.hip without a launcher above

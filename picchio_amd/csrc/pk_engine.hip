@@ -44,6 +44,22 @@ void pk_dev_free(pk_engine *e, void *p) {
     if (p) (void)hipFree(p);
 }
 
+int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n) {
+    PK_HIP(hipStreamSynchronize(e->stream));
+    const bool graphs = e->live_graphs->load() > 0;
+    if (!graphs) {
+        for (void *p : e->outgrown) pk_dev_free(e, p);
+        e->outgrown.clear();
+    }
+    for (int i = 0; i < n; ++i) {
+        if (graphs && *b[i].p) e->outgrown.push_back(*b[i].p);
+        else pk_dev_free(e, *b[i].p);
+        *b[i].p = nullptr;
+    }
+    for (int i = 0; i < n; ++i) PK_TRY(pk_dev_alloc(e, b[i].p, b[i].bytes));
+    return PK_OK;
+}
+
 int pk_stage_reserve(pk_engine *e, int64_t bytes) {
     if (bytes <= e->stage_bytes) return PK_OK;
     PK_CHECK(!e->capturing, PK_ERR_ARG, "uploads are not available while capturing a graph");
@@ -151,6 +167,7 @@ static void engine_free(pk_engine *e) {
                     e->lm_bval, e->lm_bidx, e->dstate, e->step_out, e->samp, e->samp_av, e->samp_ai, e->samp_ws, e->hn_q, e->act_q, e->b_xq, e->b_actq, e->b_pairs, e->b_tiles,
                     e->moe_act_t, e->moe_eo_t, e->moe_cont_t, e->att_t, e->skinny_ws, e->lm_t};
     for (void *p : ptrs) pk_dev_free(e, p);
+    for (void *p : e->outgrown) pk_dev_free(e, p);
     if (e->L) {
         for (int l = 0; l < e->c.n_layers; ++l) {
             pk_layer_dev &d = e->L[l];
@@ -510,6 +527,7 @@ extern "C" int pk_engine_stall(pk_engine *e, int usec) {
 struct pk_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    std::shared_ptr<std::atomic<int>> live;   // the engine's count (which may end before the graph)
 };
 
 extern "C" int pk_capture_begin(pk_engine *e) {
@@ -535,6 +553,8 @@ extern "C" int pk_capture_end(pk_engine *e, pk_graph **out) {
         delete g;
         return PK_ERR_HIP;
     }
+    g->live = e->live_graphs;
+    g->live->fetch_add(1);
     *out = g;
     return PK_OK;
 }
@@ -549,6 +569,7 @@ extern "C" int pk_graph_destroy(pk_graph *g) {
     if (!g) return PK_OK;
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
+    g->live->fetch_sub(1);
     delete g;
     return PK_OK;
 }

@@ -163,26 +163,23 @@ static int batch_reserve(pk_engine *e, int T) {
     const pk_cfg *c = &e->c;
     PK_CHECK((int64_t)T * c->topk <= 65535, PK_ERR_UNSUPPORTED, "batched MoE: %d tokens x top-%d", T,
              c->topk);
-    PK_HIP(hipStreamSynchronize(e->stream));
-    void *ptrs[] = {e->b_logits, e->b_w, e->b_act, e->b_eo, e->b_sel, e->b_perm, e->b_xq, e->b_actq,
-                    e->b_pairs, e->b_tiles};
-    for (void *p : ptrs) pk_dev_free(e, p);
-    e->b_logits = e->b_w = e->b_act = e->b_eo = nullptr;
-    e->b_sel = e->b_perm = e->b_xq = e->b_actq = e->b_pairs = e->b_tiles = nullptr;
     e->batch_cap = 0;
     const int64_t TK = (int64_t)T * c->topk;
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_logits, (int64_t)T * c->n_experts * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_w, TK * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_sel, TK * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_perm, TK * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_act, TK * (c->moe_inter / 2) * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_eo, TK * c->hidden * 4));
-    // integer-dot records: the token rows', each pair's SwiGLU outputs'
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_xq, (int64_t)T * ((c->hidden + 31) / 32) * PK_XQ_INTS * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_actq, TK * e->ex.gu.RB * PK_XQ_INTS * 4));
-    // pairs grouped by expert for the tiled integer-dot launches (tiles of 4)
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_pairs, TK * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->b_tiles, (3 * (TK / 4 + 1 + c->n_experts) + 1) * 4));
+    const pk_buf_bytes bufs[] = {
+        {(void **)&e->b_logits, (int64_t)T * c->n_experts * 4},
+        {(void **)&e->b_w, TK * 4},
+        {(void **)&e->b_sel, TK * 4},
+        {(void **)&e->b_perm, TK * 4},
+        {(void **)&e->b_act, TK * (c->moe_inter / 2) * 4},
+        {(void **)&e->b_eo, TK * c->hidden * 4},
+        // integer-dot records: the token rows', each pair's SwiGLU outputs'
+        {(void **)&e->b_xq, (int64_t)T * ((c->hidden + 31) / 32) * PK_XQ_INTS * 4},
+        {(void **)&e->b_actq, TK * e->ex.gu.RB * PK_XQ_INTS * 4},
+        // pairs grouped by expert (tiles of at least 4)
+        {(void **)&e->b_pairs, TK * 4},
+        {(void **)&e->b_tiles, (3 * (TK / 4 + 1 + c->n_experts) + 1) * 4},
+    };
+    PK_TRY(pk_regrow(e, bufs, sizeof(bufs) / sizeof(bufs[0])));
     if (!e->skinny_ws) PK_TRY(pk_dev_alloc(e, (void **)&e->skinny_ws, PK_SKINNY_WS * 4));
     e->batch_cap = T;
     return PK_OK;
@@ -316,18 +313,16 @@ static int grouped_reserve(pk_engine *e, int T) {
     const int64_t P = (int64_t)T * c->topk;
     if (P <= e->g_cap) return PK_OK;
     PK_CHECK(!e->capturing, PK_ERR_ARG, "grouped buffers must be sized before capturing a graph");
-    PK_HIP(hipStreamSynchronize(e->stream));
-    void *ptrs[] = {e->g_limbs, e->g_exps, e->g_pairs, e->g_tiles};
-    for (void *p : ptrs) pk_dev_free(e, p);
-    e->g_limbs = nullptr;
-    e->g_exps = e->g_pairs = e->g_tiles = nullptr;
     e->g_cap = 0;
     const int64_t plane = std::max((int64_t)T * c->hidden, P * (c->moe_inter / 2));
     const int64_t max_tiles = (P + 31) / 32 + c->n_experts;
-    PK_TRY(pk_dev_alloc(e, (void **)&e->g_limbs, 4 * plane));     // 3 int8 planes or 2 half planes
-    PK_TRY(pk_dev_alloc(e, (void **)&e->g_exps, std::max((int64_t)T, P) * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->g_pairs, P * 4));
-    PK_TRY(pk_dev_alloc(e, (void **)&e->g_tiles, (5 * max_tiles + 1) * 4));
+    const pk_buf_bytes bufs[] = {
+        {(void **)&e->g_limbs, 4 * plane},     // 3 int8 planes or 2 half planes
+        {(void **)&e->g_exps, std::max((int64_t)T, P) * 4},
+        {(void **)&e->g_pairs, P * 4},
+        {(void **)&e->g_tiles, (5 * max_tiles + 1) * 4},
+    };
+    PK_TRY(pk_regrow(e, bufs, sizeof(bufs) / sizeof(bufs[0])));
     e->g_cap = P;
     return PK_OK;
 }

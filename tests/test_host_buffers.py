@@ -1,0 +1,61 @@
+"""Device buffers over their life, on the host side alone (hip_host): what a
+captured graph addresses outlives the calls that need larger buffers."""
+import pytest
+
+from hip_host import run
+
+GROW = {
+    "prompt": "pa.check(prompt(h, 600))",
+    "batch": "pa.check(L.pk_moe_forward_batch(h, 1, x, 200, out, None, None))",
+    "grouped": "pa.check(L.pk_moe_forward_grouped(h, 1, x, 200, None, None, out, None, None))",
+    "decode_batch": """
+pa.check(L.pk_batch_reserve(h, 90))
+toks, res = np.zeros(90, np.int32), np.zeros(180, np.int32)
+pa.check(L.pk_decode_batch(h, 90, pa.ptr(toks), 0, 2, pa.ptr(res)))""",
+}
+
+
+@pytest.mark.parametrize("grow", sorted(GROW))
+@pytest.mark.parametrize("call", ["pk_moe_forward_batch(h, 0, x, 64, out, None, None)",
+                                  "pk_moe_forward_grouped(h, 0, x, 64, None, None, out, None, None)"],
+                         ids=["captured-batch", "captured-grouped"])
+def test_captured_buffers_outlive_growth(call, grow):
+    run(f"""
+h = engine(small(n_experts=8))
+x, out = dev(200 * 128), dev(200 * 128)
+pa.check(L.{call})                       # (sizes the buffers)
+pa.check(L.pk_capture_begin(h))
+pa.check(L.{call})
+g = vp()
+pa.check(L.pk_capture_end(h, C.byref(g)))
+{GROW[grow]}
+pa.check(L.pk_graph_launch(h, g))
+assert hh.hh_stale() == 0, hh.hh_stale()
+# given back: the growth after the last graph's end frees what it kept
+pa.check(L.pk_graph_destroy(g))
+used = hh.hh_in_use()
+big_x, big_out = dev(1000 * 128), dev(1000 * 128)
+pa.check(L.pk_moe_forward_grouped(h, 0, big_x, 1000, None, None, big_out, None, None))
+once = hh.hh_in_use()
+pa.check(L.pk_engine_destroy(h))
+assert hh.hh_in_use() == 4 * 128 * (200 + 200 + 1000 + 1000), hh.hh_in_use()
+# an engine that never captured holds as much
+h = engine(small(n_experts=8))
+{GROW[grow]}
+pa.check(L.pk_moe_forward_grouped(h, 0, big_x, 1000, None, None, big_out, None, None))
+assert hh.hh_in_use() == once, (hh.hh_in_use(), once)
+""")
+
+
+def test_graph_may_outlive_its_engine():
+    run("""
+h = engine(small())
+x, out = dev(64 * 128), dev(64 * 128)
+pa.check(L.pk_moe_forward_batch(h, 0, x, 64, out, None, None))
+pa.check(L.pk_capture_begin(h))
+pa.check(L.pk_moe_forward_batch(h, 0, x, 64, out, None, None))
+g = vp()
+pa.check(L.pk_capture_end(h, C.byref(g)))
+pa.check(L.pk_engine_destroy(h))
+pa.check(L.pk_graph_destroy(g))
+""")
