@@ -192,14 +192,17 @@ int pk_noalloc_scratch_init(pk_engine *e);
 
 int pk_dev_alloc(pk_engine *e, void **p, int64_t bytes);
 void pk_dev_free(pk_engine *e, void *p);
-// Larger buffers in the place of *b[i].p (their contents are not kept). The
-// old ones are freed, or while a captured graph lives, kept for its kernels
-// until the next growth without one, or the engine's end.
+// Larger buffers in the place of *b[i].p (their contents are not kept). Where
+// old and new do not fit together the old ones go first, unless the growth is
+// optional or a captured graph may address them: then, on an error, they stay
+// as they are (else null). Replaced ones are freed, or while a captured graph
+// lives, kept for its kernels until the next growth without one, or the
+// engine's end.
 struct pk_buf_bytes {
     void **p;
     int64_t bytes;
 };
-int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n);
+int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n, bool optional = false);
 int pk_stage_reserve(pk_engine *e, int64_t bytes);
 
 // kernels defined in pk_dense.hip / pk_attn.hip without a launcher above

@@ -44,19 +44,34 @@ void pk_dev_free(pk_engine *e, void *p) {
     if (p) (void)hipFree(p);
 }
 
-int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n) {
+int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n, bool optional) {
     PK_HIP(hipStreamSynchronize(e->stream));
     const bool graphs = e->live_graphs->load() > 0;
     if (!graphs) {
         for (void *p : e->outgrown) pk_dev_free(e, p);
         e->outgrown.clear();
     }
+    std::vector<void *> fresh(n, nullptr);
+    const auto alloc = [&]() {
+        int rc = PK_OK;
+        for (int i = 0; i < n && rc == PK_OK; ++i) rc = pk_dev_alloc(e, &fresh[i], b[i].bytes);
+        if (rc != PK_OK)
+            for (int i = 0; i < n; ++i) {
+                if (fresh[i]) e->device_bytes -= b[i].bytes;
+                pk_dev_free(e, fresh[i]);
+                fresh[i] = nullptr;
+            }
+        return rc;
+    };
+    int rc = alloc();
+    if (rc != PK_OK && (optional || graphs)) return rc;
     for (int i = 0; i < n; ++i) {
         if (graphs && *b[i].p) e->outgrown.push_back(*b[i].p);
         else pk_dev_free(e, *b[i].p);
         *b[i].p = nullptr;
     }
-    for (int i = 0; i < n; ++i) PK_TRY(pk_dev_alloc(e, b[i].p, b[i].bytes));
+    if (rc != PK_OK) PK_TRY(alloc());
+    for (int i = 0; i < n; ++i) *b[i].p = fresh[i];
     return PK_OK;
 }
 

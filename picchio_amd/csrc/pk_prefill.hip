@@ -157,13 +157,13 @@ static int launch_combine(pk_engine *e, float *out, const float *residual, const
     return PK_OK;
 }
 
-static int batch_reserve(pk_engine *e, int T) {
+// optional: on an error the buffers are as they were.
+static int batch_reserve(pk_engine *e, int T, bool optional = false) {
     if (T <= e->batch_cap) return PK_OK;
     PK_CHECK(!e->capturing, PK_ERR_ARG, "batch buffers must be sized before capturing a graph");
     const pk_cfg *c = &e->c;
     PK_CHECK((int64_t)T * c->topk <= 65535, PK_ERR_UNSUPPORTED, "batched MoE: %d tokens x top-%d", T,
              c->topk);
-    e->batch_cap = 0;
     const int64_t TK = (int64_t)T * c->topk;
     const pk_buf_bytes bufs[] = {
         {(void **)&e->b_logits, (int64_t)T * c->n_experts * 4},
@@ -179,8 +179,10 @@ static int batch_reserve(pk_engine *e, int T) {
         {(void **)&e->b_pairs, TK * 4},
         {(void **)&e->b_tiles, (3 * (TK / 4 + 1 + c->n_experts) + 1) * 4},
     };
-    PK_TRY(pk_regrow(e, bufs, sizeof(bufs) / sizeof(bufs[0])));
     if (!e->skinny_ws) PK_TRY(pk_dev_alloc(e, (void **)&e->skinny_ws, PK_SKINNY_WS * 4));
+    const int rc = pk_regrow(e, bufs, sizeof(bufs) / sizeof(bufs[0]), optional);
+    if (!e->b_logits) e->batch_cap = 0;
+    PK_TRY(rc);
     e->batch_cap = T;
     return PK_OK;
 }
@@ -313,7 +315,6 @@ static int grouped_reserve(pk_engine *e, int T) {
     const int64_t P = (int64_t)T * c->topk;
     if (P <= e->g_cap) return PK_OK;
     PK_CHECK(!e->capturing, PK_ERR_ARG, "grouped buffers must be sized before capturing a graph");
-    e->g_cap = 0;
     const int64_t plane = std::max((int64_t)T * c->hidden, P * (c->moe_inter / 2));
     const int64_t max_tiles = (P + 31) / 32 + c->n_experts;
     const pk_buf_bytes bufs[] = {
@@ -322,7 +323,9 @@ static int grouped_reserve(pk_engine *e, int T) {
         {(void **)&e->g_pairs, P * 4},
         {(void **)&e->g_tiles, (5 * max_tiles + 1) * 4},
     };
-    PK_TRY(pk_regrow(e, bufs, sizeof(bufs) / sizeof(bufs[0])));
+    const int rc = pk_regrow(e, bufs, sizeof(bufs) / sizeof(bufs[0]));
+    if (!e->g_limbs) e->g_cap = 0;
+    PK_TRY(rc);
     e->g_cap = P;
     return PK_OK;
 }
@@ -503,6 +506,15 @@ extern "C" int pk_moe_forward_batch_noalloc(pk_engine *e, int layer, const float
     return PK_OK;
 }
 
+static void prefill_free(pk_engine *e) {
+    (void)hipStreamSynchronize(e->stream);
+    void *ptrs[] = {e->p_H, e->p_XN, e->p_qkv, e->p_att, e->p_ids};
+    for (void *p : ptrs) pk_dev_free(e, p);
+    e->p_H = e->p_XN = e->p_qkv = e->p_att = nullptr;
+    e->p_ids = nullptr;
+    e->p_cap = 0;
+}
+
 // Prompt rows: B rows of hidden states, QKV and attention; part_rows of the
 // split attention's partials (the lockstep decode, and windows past what
 // k_attn_rows_exact holds).
@@ -519,12 +531,7 @@ static int prefill_reserve(pk_engine *e, int B, int part_rows) {
         e->p_part_cap = part_rows;
     }
     if (B <= e->p_cap) return PK_OK;
-    PK_HIP(hipStreamSynchronize(e->stream));
-    void *ptrs[] = {e->p_H, e->p_XN, e->p_qkv, e->p_att, e->p_ids};
-    for (void *p : ptrs) pk_dev_free(e, p);
-    e->p_H = e->p_XN = e->p_qkv = e->p_att = nullptr;
-    e->p_ids = nullptr;
-    e->p_cap = 0;
+    prefill_free(e);
     const int64_t qkv_dim = (int64_t)(c->n_heads + 2 * c->n_kv_heads) * c->head_dim;
     PK_TRY(pk_dev_alloc(e, (void **)&e->p_H, (int64_t)B * c->hidden * 4));
     PK_TRY(pk_dev_alloc(e, (void **)&e->p_XN, (int64_t)B * c->hidden * 4));
@@ -593,11 +600,12 @@ int pk_prefill_run(pk_engine *e, int seq, const int32_t *ids, int n, int pos_bas
     const bool mfma = mv && atoi(mv) != 0;
     int rows = B;
     if (!mfma && !e->rtrace && B < PREFILL_ROWS) rows = std::min(PREFILL_ROWS / B * B, n);
-    if (prefill_reserve(e, rows, B) != PK_OK || batch_reserve(e, rows) != PK_OK) {
-        rows = B;                                      // little memory left: chunk by chunk
-        PK_TRY(prefill_reserve(e, B, B));
-        PK_TRY(batch_reserve(e, B));
+    if (rows > B && (prefill_reserve(e, rows, B) != PK_OK || batch_reserve(e, rows, true) != PK_OK)) {
+        prefill_free(e);                               // little memory left: chunk by chunk
+        rows = B;
     }
+    PK_TRY(prefill_reserve(e, rows, B));
+    PK_TRY(batch_reserve(e, rows));
     PK_HIP(hipMemcpyAsync(e->p_ids, ids, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
     // a repetition penalty counts the prompt itself (picchio.c:1960-1967)
     PK_TRY(pk_sample_seed_history(e, e->p_ids, n));

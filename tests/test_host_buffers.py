@@ -59,3 +59,49 @@ pa.check(L.pk_capture_end(h, C.byref(g)))
 pa.check(L.pk_engine_destroy(h))
 pa.check(L.pk_graph_destroy(g))
 """)
+
+
+@pytest.mark.parametrize("sized", [0, 100])
+def test_prompt_in_the_memory_of_one_chunk(sized):
+    """Wherever the memory for a prompt chunk by chunk is there (the router
+    trace keeps one chunk of 64 per pass), the prompt runs, and buffers sized
+    for a capture are as they were after a pass of 512 rows did not fit."""
+    run(f"""
+T = {sized}
+def start():
+    h = engine(small(vocab=512))
+    if T:
+        pa.check(L.pk_moe_forward_batch(h, 0, x, T, x, None, None))
+    return h
+x, trace = dev(1 + T * 128), dev(16)
+h = start()
+base = hh.hh_in_use()
+pa.check(L.pk_set_router_trace(h, trace, 16))
+hh.hh_peak(1)
+pa.check(prompt(h, 600))
+need = hh.hh_peak(0)
+pa.check(L.pk_set_router_trace(h, None, 0))
+pa.check(prompt(h, 600))
+wide = hh.hh_peak(0)
+pa.check(L.pk_engine_destroy(h))
+assert need - base > 1 << 17 and wide - need > 1 << 20, (base, need, wide)
+for budget in range(need, wide + (1 << 16), (wide - need) // 60):
+    h = start()
+    if T:
+        pa.check(L.pk_capture_begin(h))
+        pa.check(L.pk_moe_forward_batch(h, 0, x, T, x, None, None))
+        g = vp()
+        pa.check(L.pk_capture_end(h, C.byref(g)))
+    hh.hh_budget(budget)
+    pa.check(prompt(h, 600))
+    if T:
+        pa.check(L.pk_graph_launch(h, g))
+        assert hh.hh_stale() == 0
+        pa.check(L.pk_graph_destroy(g))
+        pa.check(L.pk_capture_begin(h))
+        pa.check(L.pk_moe_forward_batch(h, 0, x, T, x, None, None))
+        pa.check(L.pk_capture_end(h, C.byref(g)))
+        pa.check(L.pk_graph_destroy(g))
+    pa.check(L.pk_engine_destroy(h))
+    hh.hh_budget(-1)
+""")
