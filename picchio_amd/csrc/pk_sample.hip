@@ -1746,6 +1746,11 @@ int pk_sample_reserve(pk_engine *e, int vocab) {
     if (vocab <= e->samp_cap) return PK_OK;
     PK_CHECK(!e->capturing, PK_ERR_ARG, "sampling: vocabulary %d beyond the scratch made before capture", vocab);
     PK_HIP(hipStreamSynchronize(e->stream));
+    if (e->step_exec) {                       // the captured step addresses the old scratch
+        (void)hipGraphExecDestroy(e->step_exec);
+        e->step_exec = nullptr;
+        e->step_cap = -1;
+    }
     pk_dev_free(e, e->samp_av);
     pk_dev_free(e, e->samp_ai);
     e->device_bytes -= (int64_t)e->samp_cap * 8;

@@ -105,3 +105,23 @@ for budget in range(need, wide + (1 << 16), (wide - need) // 60):
     pa.check(L.pk_engine_destroy(h))
     hh.hh_budget(-1)
 """)
+
+
+@pytest.mark.parametrize("case", [(1.0, 0.9, 0, 1.0), (1.0, 1.0, 50, 1.1), (1.0, 1.0, 0, 1.1)])
+def test_step_graph_after_a_larger_vocabulary(case):
+    """decode_replay keeps its captured step; a draw over a larger vocabulary
+    than the model's replaces the scratch that the step addresses."""
+    run(f"""
+h = engine(small())
+pa.check(L.pk_set_sampling(h, {case[0]}, {case[1]}, {case[2]}, {case[3]}, 5))
+out, lg, tok = np.zeros(8, np.int32), dev(70000), C.c_int32()
+pa.check(L.pk_decode_replay(h, 3, 0, 4, pa.ptr(out)))
+pa.check(L.pk_decode_replay(h, 3, 0, 4, pa.ptr(out)))
+assert hh.hh_instantiated() == 1
+pa.check(L.pk_sample_logits(h, lg, 70000, C.byref(tok)))
+assert hh.hh_execs() == 0                # (the step is gone with what it addressed)
+pa.check(L.pk_decode_replay(h, 3, 0, 4, pa.ptr(out)))
+assert hh.hh_stale() == 0, hh.hh_stale()
+pa.check(L.pk_sample_logits(h, lg, 70000, C.byref(tok)))
+assert hh.hh_execs() == 1 and hh.hh_instantiated() == 2
+""")
