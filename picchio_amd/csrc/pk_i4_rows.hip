@@ -457,6 +457,7 @@ int pk_launch_i4_rows(const pk_i4_items &it, const pk_i4_tiles *tl, const pk_i4_
                       float alpha, int max_tiles, hipStream_t st, int tile_rows) {
     PK_CHECK(pk_i4_rows_ok(it, epilogue), PK_ERR_ARG, "i4 rows: inputs not 16-byte aligned, or not the fp32 chains");
     PK_CHECK(sh.NG > 0 && sh.RB > 0 && it.n_items > 0 && it.x_div > 0, PK_ERR_ARG, "i4 rows: empty shape");
+    PK_CHECK(sh.NG <= 128, PK_ERR_UNSUPPORTED, "i4 rows: I=%d above 8192", sh.I);     // (as for one row)
     PK_CHECK(!tl || (tl->pairs && tl->tile_exp && tl->tile_beg && tl->tile_cnt && tl->n_tiles), PK_ERR_ARG,
              "i4 rows: missing tiles");
     PK_CHECK(tile_rows == 8 || (tile_rows == 16 && epilogue != PK_EPI_ROW_SCALED), PK_ERR_ARG, "i4 rows: tiles of %d",
