@@ -858,11 +858,12 @@ extern "C" int pk_qt_upload(pk_engine *e, const pk_qt_host *h, pk_qt **out) {
         const int64_t nsc = gs > 0 ? (int64_t)h->O * ((h->I + gs - 1) / gs) : h->O;
         if (!h->s) rc = PK_ERR_ARG;
         else if (h->I % PK_GS == 0 && (gs == PK_GS || (gs <= 0 && h->I > PK_GS && h->I <= 128 * PK_GS))) {
-            // (a scale per row: the same tiles, the scale stored for each group.
+            // (a scale per row: the same tiles, one scale per row of the blocks.
             // A 64-wide row has nothing to fold, and the lanes' tree over single
             // products is the more exact: 7.5e-8 against 7.6e-8 from 64 bits)
             t->tiled = 1;
             t->sh = pk_i4_make_shape(h->O, h->I);
+            if (gs <= 0) t->sh.scale_bytes = (int64_t)t->sh.RB * PK_TILE_ROWS * 4;
             rc = pk_dev_alloc(e, &t->data, t->sh.tile_bytes);
             if (rc == PK_OK) rc = pk_dev_alloc(e, (void **)&t->s, t->sh.scale_bytes);
             if (rc == PK_OK) {

@@ -52,14 +52,16 @@ __global__ __launch_bounds__(NW * 64) void k_i4_gemv(pk_i4_items it, int O, int 
     const uint8_t *base = it.base + (int64_t)slot * it.slot_stride;
     const uint4 *tiles = reinterpret_cast<const uint4 *>(base + it.off_tiles) +
                          (int64_t)rb * NG * (PK_TILE_BYTES / 16);
-    const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64;
+    constexpr bool RS = EPI == PK_EPI_ROW_SCALED;
+    const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * (RS ? 1 : NG) * 64;
     const float *__restrict__ x = it.x + (int64_t)(item / it.x_div) * it.x_stride;
     const int32_t *__restrict__ xq = DOT ? it.xq + (int64_t)(item / it.x_div) * it.xq_stride : nullptr;
     const int row = rb * 64 + lane;
     // the epilogue's operands go out with the weights, not after the fold
     // (a load issued there would put a memory round trip on the critical path)
-    float bias = 0.0f, res = 0.0f, cw[16];
+    float bias = 0.0f, res = 0.0f, rs = 0.0f, cw[16];
     if (wave == 0) {
+        if constexpr (RS) rs = sc[lane];
         if (it.off_bias >= 0) bias = reinterpret_cast<const float *>(base + it.off_bias)[min(row, O - 1)];
         if constexpr (EPI == PK_EPI_COMBINE) {
             if (cb.residual) res = cb.residual[min(row, O - 1)];
@@ -77,7 +79,7 @@ __global__ __launch_bounds__(NW * 64) void k_i4_gemv(pk_i4_items it, int O, int 
             if (g < NG) {
                 wa[u] = pk_load_nt(&tiles[g * 128 + lane]);
                 wb[u] = pk_load_nt(&tiles[g * 128 + 64 + lane]);
-                s[u] = sc[g * 64 + lane];
+                s[u] = RS ? 0.0f : sc[g * 64 + lane];
             }
         }
 #pragma unroll
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(NW * 64) void k_i4_gemv(pk_i4_items it, int O, int 
                                                        xq + (2 * g + 1) * PK_XQ_INTS, s[u]);
                 } else {
                     part[g * 64 + lane] = pk_group_dot(wa[u], wb[u], x + g * 64);
-                    scl[g * 64 + lane] = s[u];
+                    if constexpr (!RS) scl[g * 64 + lane] = s[u];
                 }
             }
         }
@@ -98,7 +100,7 @@ __global__ __launch_bounds__(NW * 64) void k_i4_gemv(pk_i4_items it, int O, int 
     if (wave != 0) return;
 
     float acc;
-    if constexpr (EPI == PK_EPI_ROW_SCALED) acc = pk_fold_row_scaled(part + lane, scl + lane, NG, 64);
+    if constexpr (RS) acc = pk_fold_row_scaled(part + lane, rs, NG, 64);
     else acc = pk_fold_groups<DOT>(part, scl, NG);
     if (it.off_bias >= 0 && row < O) acc = acc + bias;
     float *y = it.y + (int64_t)item * it.y_stride;
@@ -172,7 +174,9 @@ __global__ __launch_bounds__(PR_NW * 64) void k_i4_gemv_part(pk_i4_items it, int
     const uint8_t *base = it.base + (int64_t)slot * it.slot_stride;
     const uint4 *tiles =
         reinterpret_cast<const uint4 *>(base + it.off_tiles) + (int64_t)rb * NG * (PK_TILE_BYTES / 16) + r0 + r;
-    const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64 + r0 + r;
+    constexpr bool RS = EPI == PK_EPI_ROW_SCALED;
+    const float *sc =
+        reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * (RS ? 1 : NG) * 64 + r0 + r;
     const float *__restrict__ x = it.x + (int64_t)(item / it.x_div) * it.x_stride;
     const int row = rb * 64 + r0 + r;
     uint4 wa[GPW], wb[GPW];
@@ -183,10 +187,11 @@ __global__ __launch_bounds__(PR_NW * 64) void k_i4_gemv_part(pk_i4_items it, int
             const int g = min(g0 + u * PR_NW * GQ + gq, NG - 1);
             wa[u] = pk_load_nt(&tiles[g * 128]);
             wb[u] = pk_load_nt(&tiles[g * 128 + 64]);
-            s[u] = sc[g * 64];
+            s[u] = RS ? 0.0f : sc[g * 64];
         }
     };
     load(GQ * wave);
+    const float rs = RS && wave == 0 ? sc[0] : 0.0f;
     const float bias = wave == 0 && it.off_bias >= 0
                            ? reinterpret_cast<const float *>(base + it.off_bias)[min(row, O - 1)] : 0.0f;
     for (int i = threadIdx.x; i < NG * 64; i += PR_NW * 64) xs[(i >> 6) * PR_XP + (i & 63)] = x[i];
@@ -204,7 +209,7 @@ __global__ __launch_bounds__(PR_NW * 64) void k_i4_gemv_part(pk_i4_items it, int
                     xr[4 * i] = t.x; xr[4 * i + 1] = t.y; xr[4 * i + 2] = t.z; xr[4 * i + 3] = t.w;
                 }
                 part[g * R + r] = pk_group_dot(wa[u], wb[u], (const float *)xr);
-                scl[g * R + r] = s[u];
+                if constexpr (!RS) scl[g * R + r] = s[u];
             }
         }
         if (g0 + GPW * PR_NW * GQ < NG) load(g0 + GPW * PR_NW * GQ);
@@ -213,7 +218,7 @@ __global__ __launch_bounds__(PR_NW * 64) void k_i4_gemv_part(pk_i4_items it, int
     if (wave != 0) return;
     float acc = 0.0f;
     constexpr int C = 15;
-    if constexpr (EPI == PK_EPI_ROW_SCALED) acc = pk_fold_row_scaled(part + r, scl + r, NG, R);
+    if constexpr (RS) acc = pk_fold_row_scaled(part + r, rs, NG, R);
     else for (int b = 0; b < NG; b += C) {
         float p[C], v[C];
 #pragma unroll
@@ -260,6 +265,7 @@ __device__ __forceinline__ void st_wait(int *c, int target) {
 template <int EPI, bool DOT>
 __global__ __launch_bounds__((ST_NW + 1) * 64) void k_i4_gemv_stream(pk_i4_items it, int O, int NG, int RB,
                                                                      float lim, float alpha) {
+    constexpr bool RS = EPI == PK_EPI_ROW_SCALED;
     extern __shared__ float lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -289,14 +295,15 @@ __global__ __launch_bounds__((ST_NW + 1) * 64) void k_i4_gemv_stream(pk_i4_items
             const uint8_t *base = task(real ? k : 0, item, rb);
             const uint4 *tiles =
                 reinterpret_cast<const uint4 *>(base + it.off_tiles) + (int64_t)rb * NG * (PK_TILE_BYTES / 16);
-            const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64;
+            const float *sc =
+                reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * (RS ? 1 : NG) * 64;
             const int l = real ? lane : 0;
 #pragma unroll
             for (int u = 0; u < ST_GPW; ++u) {
                 const int g = min(wave + u * ST_NW, NG - 1);
                 wa[u] = pk_load_nt(&tiles[g * 128 + l]);
                 wb[u] = pk_load_nt(&tiles[g * 128 + 64 + l]);
-                s[u] = sc[g * 64 + l];
+                s[u] = RS ? 0.0f : sc[g * 64 + l];
             }
         };
         auto consume = [&](int k, const uint4 (&wa)[ST_GPW], const uint4 (&wb)[ST_GPW], const float (&s)[ST_GPW]) {
@@ -322,7 +329,7 @@ __global__ __launch_bounds__((ST_NW + 1) * 64) void k_i4_gemv_stream(pk_i4_items
                     const int g = wave + u * ST_NW;
                     if (g < NG) {
                         pb[g * 64 + lane] = pk_group_dot(wa[u], wb[u], x + g * 64);
-                        sb[g * 64 + lane] = s[u];
+                        if constexpr (!RS) sb[g * 64 + lane] = s[u];
                     }
                 }
             }
@@ -347,10 +354,11 @@ __global__ __launch_bounds__((ST_NW + 1) * 64) void k_i4_gemv_stream(pk_i4_items
         const int row = rb * 64 + lane;
         const float bias = it.off_bias >= 0 ? reinterpret_cast<const float *>(base + it.off_bias)[min(row, O - 1)]
                                             : 0.0f;
+        const float rs = RS ? reinterpret_cast<const float *>(base + it.off_scales)[row] : 0.0f;
         st_wait(&cnt[b], ST_NW * ((k >> 1) + 1));
         float acc;
-        if constexpr (EPI == PK_EPI_ROW_SCALED)
-            acc = pk_fold_row_scaled(part + b * NG * 64 + lane, scl + b * NG * 64 + lane, NG, 64);
+        if constexpr (RS)
+            acc = pk_fold_row_scaled(part + b * NG * 64 + lane, rs, NG, 64);
         else
             acc = pk_fold_groups<DOT>(part + b * NG * 64, scl + b * NG * 64, NG);
         st_signal(&cnt[2 + b]);
@@ -906,7 +914,7 @@ int pk_launch_i4_gemv_ref(float *y, const float *x, const uint8_t *q4, const flo
 // ───────────────────────── repack ─────────────────────────
 // Reference layout (q4 [O][I/2], s [O][I/64]) -> tiles + 16*scale.
 // One thread per (row of the padded block, group). row_scale: s [O], stored as
-// it is for every group (16*s could overflow where scale x sum does not).
+// it is, one per row of the padded blocks.
 __global__ void k_i4_repack(const uint8_t *q4, const float *s, int O, int I, int RB, int NG,
                             uint8_t *tiles, float *sc16, bool row_scale) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -928,7 +936,8 @@ __global__ void k_i4_repack(const uint8_t *q4, const float *s, int O, int I, int
     uint4 *dst = reinterpret_cast<uint4 *>(tiles + ((int64_t)rb * NG + g) * PK_TILE_BYTES);
     dst[r] = lo;
     dst[64 + r] = hi;
-    sc16[((int64_t)rb * NG + g) * 64 + r] = scv;
+    if (!row_scale) sc16[((int64_t)rb * NG + g) * 64 + r] = scv;
+    else if (g == 0) sc16[row] = scv;
 }
 
 int pk_launch_i4_repack(const uint8_t *q4, const float *s, int O, int I,

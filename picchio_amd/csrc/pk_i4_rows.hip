@@ -155,7 +155,8 @@ __device__ __forceinline__ void rw_body(const pk_i4_items &it, const int32_t *pa
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint4 *tiles =
         reinterpret_cast<const uint4 *>(base + it.off_tiles) + (int64_t)rb * NG * (PK_TILE_BYTES / 16);
-    const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64;
+    constexpr bool RS = EPI == PK_EPI_ROW_SCALED;
+    const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * (RS ? 1 : NG) * 64;
     auto pair_of = [&](int j) { return pairs ? pairs[beg + j] : beg + j; };
     // lane l loads input row l % 4 of each set, columns 4 (l / 4) .. + 3
     // (rows past the tile's last repeat it; their results are not stored)
@@ -166,17 +167,19 @@ __device__ __forceinline__ void rw_body(const pk_i4_items &it, const int32_t *pa
     const int row = rb * 64 + lane;
     const float bias =
         it.off_bias >= 0 ? reinterpret_cast<const float *>(base + it.off_bias)[min(row, O - 1)] : 0.0f;
+    const float rs = RS ? sc[lane] : 0.0f;
     rw_stage<NS> st[RW_PF];
     auto load = [&](rw_stage<NS> &d, int g) {
         d.wa = pk_load_nt(&tiles[g * 128 + lane]);
         d.wb = pk_load_nt(&tiles[g * 128 + 64 + lane]);
-        d.s = sc[g * 64 + lane];
+        d.s = RS ? 0.0f : sc[g * 64 + lane];
 #pragma unroll
         for (int s = 0; s < NS; ++s) d.x[s] = *reinterpret_cast<const float4 *>(xp[s] + g * 64);
     };
     // the row's sum so far, handed from wave to wave (and span to span) in
     // group order: a = fma(partial, scale, a). With a scale per row (no
-    // prescribed order) each wave's groups sum on their own and are added.
+    // prescribed order) each wave's groups are summed pairwise, unscaled, and
+    // added; the scale comes last.
     f32x4 acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -200,23 +203,31 @@ __device__ __forceinline__ void rw_body(const pk_i4_items &it, const int32_t *pa
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         prev[s][i] = b0 + w > 0 ? accs[4 * s + i][lane] : 0.0f;
-                        acc[s][i] = EPI == PK_EPI_ROW_SCALED ? 0.0f : prev[s][i];
+                        acc[s][i] = prev[s][i];
                     }
-#pragma unroll
-                for (int u = 0; u < RW_GW; ++u)
-                    if (g0 + u < NG) {
-#pragma unroll
-                        for (int s = 0; s < NS; ++s)
-#pragma unroll
-                            for (int i = 0; i < 4; ++i)
-                                acc[s][i] = __builtin_fmaf(
-                                    EPI == PK_EPI_ROW_SCALED ? 16.0f * p[u][s][i] : p[u][s][i], sv[u], acc[s][i]);
-                    }
-                if constexpr (EPI == PK_EPI_ROW_SCALED) {
+                if constexpr (RS) {
+                    // (pairwise, in eights and fours)
+                    static_assert(RW_GW == 12, "");
 #pragma unroll
                     for (int s = 0; s < NS; ++s)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[s][i] = prev[s][i] + acc[s][i];
+                        for (int i = 0; i < 4; ++i) {
+                            float v[RW_GW];
+#pragma unroll
+                            for (int u = 0; u < RW_GW; ++u) v[u] = g0 + u < NG ? p[u][s][i] : 0.0f;
+                            const float lo[8] = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+                            acc[s][i] = prev[s][i] + (pk_add8(lo) + ((v[8] + v[9]) + (v[10] + v[11])));
+                        }
+                } else {
+#pragma unroll
+                    for (int u = 0; u < RW_GW; ++u)
+                        if (g0 + u < NG) {
+#pragma unroll
+                            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    acc[s][i] = __builtin_fmaf(p[u][s][i], sv[u], acc[s][i]);
+                        }
                 }
 #pragma unroll
                 for (int s = 0; s < NS; ++s)
@@ -230,6 +241,10 @@ __device__ __forceinline__ void rw_body(const pk_i4_items &it, const int32_t *pa
     const int j = 2 * wave;
     if (j >= cnt) return;
     float a0 = accs[j][lane], a1 = accs[j + 1][lane];
+    if constexpr (RS) {
+        a0 = (float)(16.0 * (double)a0 * (double)rs);
+        a1 = (float)(16.0 * (double)a1 * (double)rs);
+    }
     if (it.off_bias >= 0 && row < O) { a0 = a0 + bias; a1 = a1 + bias; }
     rw_put2<EPI>(it, pair_of, j, cnt, row, O, a0, a1, lim, alpha);
 }

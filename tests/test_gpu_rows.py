@@ -108,3 +108,27 @@ def test_i4_row_scales_in_tiles_bound(gpu, oracle, O, I, S):
     depth = 8 + 3 + max(-(-ng // 4), 12 + ng // 12) + 4
     bound = (np.abs(xd) @ np.abs(q).T) * sd * depth * 2.0 ** -24
     assert (np.abs(y - exact) <= bound).all()
+
+
+@pytest.mark.parametrize("O,I,S", [(130, 128, 1), (5000, 8192, 1), (12000, 2880, 1), (33000, 192, 1), (700, 8192, 33)])
+def test_i4_row_scale_applies_to_the_whole_sum(gpu, O, I, S):
+    """Groups that would overflow times the row's scale but cancel (halves and
+    quarters of row blocks, whole ones, the streaming launch, several rows).
+    Every sum is a small integer over 16 and every scale a power of two, so the
+    result is exact."""
+    import picchio_amd as pa
+    import torch
+    q4 = np.full((O, I // 2), 0xff, np.uint8)          # every weight 7
+    s = np.full(O, 2.0 ** 125, np.float32)
+    s[1::3] = np.float32(2.0 ** -140)
+    x = np.zeros((S, I), np.float32)
+    x[:, :64], x[:, -64:] = 16.0, -16.0                # +-7168 per group, times 2^125
+    x[:, 5] += 0.125 * (1 + np.arange(S) % 8)
+    with pa.Engine(pa.gptoss_cfg(n_layers=1, n_experts=4, ctx_len=16, vocab=64)) as eng:
+        qt = eng.qt_upload(pa.FMT_INT4, q4, s, O, I, 0)
+        yd = eng.empty((S, O), torch.float32)
+        eng.matmul_qt(yd, eng.to_dev(x), qt, S)
+        y = eng.to_host(yd).reshape(S, O)
+        eng.qt_free(qt)
+    ref = (x.astype(np.float64).sum(1)[:, None] * 7 * s.astype(np.float64)).astype(np.float32)
+    assert bits_equal(y, ref), first_mismatch(y, ref)

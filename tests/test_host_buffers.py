@@ -125,3 +125,18 @@ assert hh.hh_stale() == 0, hh.hh_stale()
 pa.check(L.pk_sample_logits(h, lg, 70000, C.byref(tok)))
 assert hh.hh_execs() == 1 and hh.hh_instantiated() == 2
 """)
+
+
+def test_row_scaled_int4_holds_one_scale_per_row():
+    run("""
+h = engine(small(vocab=512), synthetic=False)
+O, I = 1000, 2880
+q, s = np.zeros((O, I // 2), np.uint8), np.ones(O, np.float32)
+t, qt = pa.PkQtHost(pa.FMT_INT4, q.ctypes.data, s.ctypes.data, O, I, 0), vp()
+pa.check(L.pk_qt_upload(h, C.byref(t), C.byref(qt)))
+pa.check(L.pk_qt_free(h, qt))                         # (the upload's staging stays)
+before = hh.hh_in_use()
+pa.check(L.pk_qt_upload(h, C.byref(t), C.byref(qt)))
+rows = (O + 63) // 64 * 64
+assert hh.hh_in_use() - before == rows * (I // 2 + 4), hh.hh_in_use() - before
+""")
