@@ -146,7 +146,15 @@ hipError_t hipMalloc(void **p, size_t n) {
     *p = nullptr;
     if (budget >= 0 && in_use + (int64_t)n > budget) return fail(hipErrorOutOfMemory);
     const size_t len = (n + 4095) & ~(size_t)4095;
-    void *m = mmap(nullptr, len, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    // low halves of the addresses: none that a small int (beside 32 bits of
+    // padding in a structure) could be taken for
+    constexpr uintptr_t LO = 0x10000000, HI = 0xf0000000;
+    if (len > HI - LO) return fail(hipErrorOutOfMemory);
+    static uintptr_t next = 0x5a0000000000ull + LO;
+    if ((next & 0xffffffffu) + len > HI) next = (next & ~(uintptr_t)0xffffffffu) + 0x100000000ull + LO;
+    void *m = mmap((void *)next, len, PROT_READ | PROT_WRITE,
+                   MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE | MAP_FIXED_NOREPLACE, -1, 0);
+    next += len;
     if (m == MAP_FAILED) return fail(hipErrorOutOfMemory);
     mem[(uintptr_t)m] = {(uintptr_t)m + n, true};
     in_use += (int64_t)n;
