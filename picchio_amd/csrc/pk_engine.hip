@@ -600,17 +600,26 @@ static int check_i4_host(const pk_qt_host *t, int O, int I, int gs, const char *
     return PK_OK;
 }
 
-// host ref layout -> staging -> tiles in the slot
+// host ref layout -> staging -> tiles in the slot, some row blocks at a time
+// (at most UPLOAD_STAGE bytes, or one row block, so that the staging stays
+// small beside a large tensor)
+constexpr int64_t UPLOAD_STAGE = 32ll << 20;
 static int upload_i4(pk_engine *e, const pk_qt_host *t, uint8_t *tiles, float *sc16) {
-    const int64_t qbytes = (int64_t)t->O * ((t->I + 1) / 2);
     const bool row_scale = t->block_size <= 0;
-    const int64_t sbytes = (int64_t)t->O * (row_scale ? 1 : t->I / PK_GS) * 4;
-    PK_TRY(pk_stage_reserve(e, pk_align256(qbytes) + sbytes));
+    const int NG = t->I / PK_GS, ns = row_scale ? 1 : NG;            // scales per row
+    const int64_t row_q = (t->I + 1) / 2, row_s = (int64_t)ns * 4;
+    const int64_t fit = std::max<int64_t>(UPLOAD_STAGE / (PK_TILE_ROWS * (row_q + row_s)), 1);
+    const int step = (int)std::min<int64_t>(fit * PK_TILE_ROWS, t->O);
+    PK_TRY(pk_stage_reserve(e, pk_align256(step * row_q) + step * row_s));
     uint8_t *dq = e->stage;
-    float *ds = (float *)(e->stage + pk_align256(qbytes));
-    PK_HIP(hipMemcpyAsync(dq, t->data, qbytes, hipMemcpyHostToDevice, e->stream));
-    PK_HIP(hipMemcpyAsync(ds, t->s, sbytes, hipMemcpyHostToDevice, e->stream));
-    PK_TRY(pk_launch_i4_repack(dq, ds, t->O, t->I, tiles, sc16, e->stream, row_scale));
+    float *ds = (float *)(e->stage + pk_align256(step * row_q));
+    for (int r0 = 0; r0 < t->O; r0 += step) {
+        const int n = std::min(step, t->O - r0), rb = r0 / PK_TILE_ROWS;
+        PK_HIP(hipMemcpyAsync(dq, (const uint8_t *)t->data + r0 * row_q, n * row_q, hipMemcpyHostToDevice, e->stream));
+        PK_HIP(hipMemcpyAsync(ds, t->s + (int64_t)r0 * ns, n * row_s, hipMemcpyHostToDevice, e->stream));
+        PK_TRY(pk_launch_i4_repack(dq, ds, n, t->I, tiles + (int64_t)rb * NG * PK_TILE_BYTES,
+                                   sc16 + (int64_t)rb * PK_TILE_ROWS * ns, e->stream, row_scale));
+    }
     return PK_OK;
 }
 

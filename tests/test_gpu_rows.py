@@ -132,3 +132,31 @@ def test_i4_row_scale_applies_to_the_whole_sum(gpu, O, I, S):
         eng.qt_free(qt)
     ref = (x.astype(np.float64).sum(1)[:, None] * 7 * s.astype(np.float64)).astype(np.float32)
     assert bits_equal(y, ref), first_mismatch(y, ref)
+
+
+def test_i4_upload_in_pieces(gpu, oracle):
+    """A tensor larger than the upload's staging (32 MiB: 113 row blocks of 8192
+    gs64 columns, 127 with a scale per row), the last piece ragged."""
+    import picchio_amd as pa
+    import torch
+    O, I = 9001, 8192
+    rng = np.random.default_rng(3)
+    q4 = rng.integers(0, 256, (O, I // 2)).astype(np.uint8)
+    x = rng.standard_normal((1, I)).astype(np.float32)
+    w = np.empty((O, I), np.float32)
+    w[:, 0::2], w[:, 1::2] = (q4 & 15).astype(np.float32) - 8, (q4 >> 4).astype(np.float32) - 8
+    sums = (w.astype(np.float64).reshape(O, I // 64, 64) * x[0].astype(np.float64).reshape(1, I // 64, 64)).sum(2)
+    size = (np.abs(w) * np.abs(x[0])).sum(1).astype(np.float64)
+    with pa.Engine(pa.gptoss_cfg(n_layers=1, n_experts=4, ctx_len=16, vocab=64)) as eng:
+        xd, yd = eng.to_dev(x), eng.empty((1, O), torch.float32)
+        for gs, ng in ((64, I // 64), (0, 1)):
+            s = (rng.random((O, ng)) + 0.5).astype(np.float32)
+            qt = eng.qt_upload(pa.FMT_INT4, q4, s, O, I, gs)
+            eng.matmul_qt(yd, xd, qt, 1)
+            y = eng.to_host(yd).reshape(O)
+            eng.qt_free(qt)
+            if gs:
+                ref = oracle.mm_i4_gs(x, q4, s, O, I, 64).reshape(O)
+                assert bits_equal(y, ref), first_mismatch(y, ref)
+            else:                                       # (20 roundings at most of sums of these terms)
+                assert (np.abs(y - sums.sum(1) * s[:, 0]) <= 20 * 2.0 ** -24 * size * s[:, 0]).all()

@@ -140,3 +140,20 @@ pa.check(L.pk_qt_upload(h, C.byref(t), C.byref(qt)))
 rows = (O + 63) // 64 * 64
 assert hh.hh_in_use() - before == rows * (I // 2 + 4), hh.hh_in_use() - before
 """)
+
+
+@pytest.mark.parametrize("gs", [0, 64])
+def test_int4_upload_needs_no_second_tensor(gs):
+    """The staging of an upload is bounded: a large tensor fits beside it."""
+    run(f"""
+h = engine(small(vocab=512), synthetic=False)
+O, I = 60000, 8192
+q, s = np.zeros((O, I // 2), np.uint8), np.ones(O * (1 if {gs} == 0 else I // 64), np.float32)
+t, qt = pa.PkQtHost(pa.FMT_INT4, q.ctypes.data, s.ctypes.data, O, I, {gs}), vp()
+before = hh.hh_in_use()
+hh.hh_peak(1)
+pa.check(L.pk_qt_upload(h, C.byref(t), C.byref(qt)))
+rows = (O + 63) // 64 * 64
+tensor = rows * (I // 2 + 4 * (1 if {gs} == 0 else I // 64))
+assert hh.hh_peak(0) - before <= tensor + (33 << 20), hh.hh_peak(0) - before - tensor
+""")
