@@ -911,7 +911,7 @@ __global__ __launch_bounds__(SNT) void k_sample(float *lg, int V, pk_sampler_dev
             };
             // candidates gathered by k_samp_gather: every entry at or above the
             // bucket of the K-th largest
-            const int given = pre ? pre->n_cand : 0;
+            const int given = pre ? min(pre->n_cand, CAND) : 0;
             if (given > 0) {
                 for (int i = tid; i < given; i += SNT) {
                     cv[i] = pre->cv[i];
@@ -1242,6 +1242,10 @@ __global__ __launch_bounds__(SH_T) void k_samp_gather(float *lg, int V, const pk
         if (lane >= o) inc += t;
     }
     if (lane == 63) s_w[wave] = inc;
+    if (tid == 0) {                                   // (no bin for top_k 0 or above V: k_sample takes the draw)
+        s_bin = 0;
+        s_cnt = CAND + 1;
+    }
     __syncthreads();
     for (int w = 0; w < wave; ++w) inc += s_w[w];
     if (inc >= K && inc - sum < K) {
@@ -1264,8 +1268,10 @@ __global__ __launch_bounds__(SH_T) void k_samp_gather(float *lg, int V, const pk
         const float x = v[k] * inv_t;
         if ((int)(key_of(x) >> 20) >= bin) {
             const int o = atomicAdd(&ws->n_cand, 1);
-            ws->cv[o] = x;                            // (o < s_cnt <= CAND)
-            ws->ci[o] = j;
+            if (o < CAND) {                           // (o < s_cnt)
+                ws->cv[o] = x;
+                ws->ci[o] = j;
+            }
         }
         if (write_back) lg[j] = 0.0f;
     }
