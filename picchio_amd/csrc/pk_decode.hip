@@ -1174,6 +1174,14 @@ int pk_lm_head_step(pk_engine *e, const float *hn, float *logits_dev, int32_t *o
     return pk_prof_end(e, ps);
 }
 
+void pk_drop_steps(pk_engine *e) {
+    for (auto &s : e->steps) {
+        if (s.exec) (void)hipGraphExecDestroy(s.exec);
+        s.exec = nullptr;
+        s.cap = -1;
+    }
+}
+
 // tok / pos (and n_out = 0) for position pos through its pinned staging slot
 int pk_set_state(pk_engine *e, int tok, int pos) {
     pk_dstate &s = e->pin_state[pos];
@@ -1299,16 +1307,17 @@ extern "C" int pk_decode_replay(pk_engine *e, int tok, int pos, int n_steps, int
     PK_CHECK(pos + n_steps <= e->c.ctx_len, PK_ERR_CONTEXT_FULL, "positions exceed context");
     PK_TRY(pk_check_model(e));
     PK_TRY(pk_decode_reserve(e));
-    // The graph's attention grids cover positions 0..step_cap: captured
+    // The graph's attention grids cover positions 0..step.cap: captured
     // again, with the bound doubled, when a call goes past it
+    auto &step = e->steps[e->step_key];
     const int need = pos + n_steps - 1;
-    if (e->step_exec && need > e->step_cap) {
+    if (step.exec && need > step.cap) {
         PK_HIP(hipStreamSynchronize(e->stream));
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
+        (void)hipGraphExecDestroy(step.exec);
+        step.exec = nullptr;
+        step.cap = -1;
     }
-    if (!e->step_exec) {
+    if (!step.exec) {
         if (!e->step_out) {
             int32_t *od = nullptr;
             PK_TRY(pk_dev_alloc(e, (void **)&od, (int64_t)e->c.ctx_len * 4));
@@ -1327,19 +1336,19 @@ extern "C" int pk_decode_replay(pk_engine *e, int tok, int pos, int n_steps, int
         }
         e->capturing = false;
         hipError_t hr = hipStreamEndCapture(e->stream, &g);
-        if (rc == PK_OK && hr == hipSuccess) hr = hipGraphInstantiate(&e->step_exec, g, nullptr, nullptr, 0);
+        if (rc == PK_OK && hr == hipSuccess) hr = hipGraphInstantiate(&step.exec, g, nullptr, nullptr, 0);
         if (g) (void)hipGraphDestroy(g);            // every exit path after the capture
         PK_TRY(rc);
         if (hr != hipSuccess) {
-            e->step_exec = nullptr;
-            e->step_cap = -1;
+            step.exec = nullptr;
+            step.cap = -1;
             pk_set_error("decode step capture failed: %s", hipGetErrorString(hr));
             return PK_ERR_HIP;
         }
-        e->step_cap = cap;
+        step.cap = cap;
     }
     PK_TRY(pk_set_state(e, tok, pos));
-    for (int i = 0; i < n_steps; ++i) PK_HIP(hipGraphLaunch(e->step_exec, e->stream));
+    for (int i = 0; i < n_steps; ++i) PK_HIP(hipGraphLaunch(step.exec, e->stream));
     PK_HIP(hipMemcpyAsync(out, e->step_out, (size_t)n_steps * 4, hipMemcpyDeviceToHost, e->stream));
     PK_HIP(hipStreamSynchronize(e->stream));
     bool redo = false;

@@ -48,6 +48,9 @@ constexpr int PK_CTR_ATTN = 4096;         // [rows x heads] attention chunk arri
 constexpr int PK_CTR_ATTN_N = 4096;
 constexpr int PK_CTR_N = PK_CTR_ATTN + PK_CTR_ATTN_N;
 
+// Sets of launches that a decode step's draw is made of (pk_step_key).
+constexpr int PK_STEPS = 8;
+
 struct pk_engine {
     pk_cfg c{};
     int device = 0;
@@ -128,8 +131,14 @@ struct pk_engine {
     pk_dstate *pin_state = nullptr;           // pinned host staging [ctx_len]
     float *lm_bval = nullptr;                 // lm_head block maxima
     int32_t *lm_bidx = nullptr;
-    hipGraphExec_t step_exec = nullptr;       // captured decode step (pk_decode_replay)
-    int step_cap = -1;                        // att_pos_cap the step graph was captured with
+    // captured decode steps (pk_decode_replay), one per set of launches that the
+    // sampling settings select (pk_step_key), and the att_pos_cap each was
+    // captured with
+    struct {
+        hipGraphExec_t exec = nullptr;
+        int cap = -1;
+    } steps[PK_STEPS];
+    int step_key = 0;
     // Decode attention from the device state: the grid covers positions
     // 0..att_pos_cap (-1: the whole context), set by the callers that know
     // the highest position a launch or a replayed graph will reach
@@ -274,6 +283,7 @@ inline bool pk_tiles_current(const pk_engine *e) { return e->tiles_ver == e->den
 // decode driver pieces (pk_decode.hip) reused by the prompt driver
 int pk_decode_reserve(pk_engine *e);
 int pk_check_model(pk_engine *e);
+void pk_drop_steps(pk_engine *e);          // after a change of what the captured steps run or address
 int pk_set_state(pk_engine *e, int tok, int pos);
 // Rows r = 0..n-1 at position (st ? st->pos : pos_base + r * pos_step) of
 // sequence seq0 + r * seq_step.

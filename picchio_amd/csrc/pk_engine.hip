@@ -193,7 +193,7 @@ static void engine_free(pk_engine *e) {
         delete[] e->L;
     }
     free(e->expert_ready);
-    if (e->step_exec) (void)hipGraphExecDestroy(e->step_exec);
+    pk_drop_steps(e);
     if (e->pin_state) (void)hipHostFree(e->pin_state);
     if (e->prof_ev) {
         for (int i = 0; i < 2 * pk_engine::PROF_CAP; ++i) (void)hipEventDestroy(e->prof_ev[i]);
@@ -328,11 +328,7 @@ int pk_wait_fallback(pk_engine *e, bool *redo) {
         pk_set_error("a device-side wait gave up with the one-launch forms off: results are invalid");
         return PK_ERR_HIP;
     }
-    if (e->step_exec) {
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
-    }
+    pk_drop_steps(e);
     e->moe_fused = 0;
     e->attn_fused = false;
     e->wait_fallbacks += 1;
@@ -1109,11 +1105,7 @@ int pk_moe_layer(pk_engine *e, int layer, const float *x_dev, float *out_dev,
 extern "C" int pk_set_i4_dot(pk_engine *e, int on) {
     PK_CHECK(e, PK_ERR_ARG, "engine is null");
     PK_CHECK(!e->capturing, PK_ERR_ARG, "set_i4_dot: not available while capturing");
-    if (e->i4_dot != (on != 0) && e->step_exec) {      // the captured step holds the other kernels
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
-    }
+    if (e->i4_dot != (on != 0)) pk_drop_steps(e);      // the captured step holds the other kernels
     e->i4_dot = on != 0;
     return PK_OK;
 }
@@ -1129,11 +1121,7 @@ extern "C" int pk_set_moe_fused(pk_engine *e, int mode) {
     PK_CHECK(e, PK_ERR_ARG, "engine is null");
     PK_CHECK(mode >= 0 && mode <= 2, PK_ERR_ARG, "set_moe_fused: mode %d (0, 1 or 2)", mode);
     PK_CHECK(!e->capturing, PK_ERR_ARG, "set_moe_fused: not available while capturing");
-    if (e->moe_fused != mode && e->step_exec) {   // the captured step holds the other kernels
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
-    }
+    if (e->moe_fused != mode) pk_drop_steps(e);      // the captured step holds the other kernels
     e->moe_fused = mode;
     return PK_OK;
 }
@@ -1141,11 +1129,7 @@ extern "C" int pk_set_moe_fused(pk_engine *e, int mode) {
 extern "C" int pk_set_attn_fused(pk_engine *e, int on) {
     PK_CHECK(e, PK_ERR_ARG, "engine is null");
     PK_CHECK(!e->capturing, PK_ERR_ARG, "set_attn_fused: not available while capturing");
-    if (e->attn_fused != (on != 0) && e->step_exec) {   // the captured step holds the other kernels
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
-    }
+    if (e->attn_fused != (on != 0)) pk_drop_steps(e);      // the captured step holds the other kernels
     e->attn_fused = on != 0;
     return PK_OK;
 }

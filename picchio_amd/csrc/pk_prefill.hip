@@ -703,11 +703,7 @@ extern "C" int pk_batch_reserve(pk_engine *e, int n_seq) {
     pk_dev_free(e, e->V);
     e->K = e->V = nullptr;
     e->device_bytes -= 2 * (int64_t)e->n_seq * e->seq_stride * 4;
-    if (e->step_exec) {                       // the captured step addresses the old cache
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
-    }
+    pk_drop_steps(e);                         // they address the old cache
     e->n_seq = 0;
     PK_TRY(pk_dev_alloc(e, (void **)&e->K, bytes));
     PK_TRY(pk_dev_alloc(e, (void **)&e->V, bytes));

@@ -1752,11 +1752,7 @@ int pk_sample_reserve(pk_engine *e, int vocab) {
     if (vocab <= e->samp_cap) return PK_OK;
     PK_CHECK(!e->capturing, PK_ERR_ARG, "sampling: vocabulary %d beyond the scratch made before capture", vocab);
     PK_HIP(hipStreamSynchronize(e->stream));
-    if (e->step_exec) {                       // the captured step addresses the old scratch
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
-    }
+    pk_drop_steps(e);                         // they address the old scratch
     pk_dev_free(e, e->samp_av);
     pk_dev_free(e, e->samp_ai);
     e->device_bytes -= (int64_t)e->samp_cap * 8;
@@ -1842,13 +1838,18 @@ int pk_sample_seed_history(pk_engine *e, const int32_t *ids_dev, int n) {
     return PK_OK;
 }
 
-// Whether two settings' draws are the same launches (a captured step's
-// kernels read the values on the device, but not which kernels run).
-static bool same_launches(const pk_sampler_dev &a, const pk_sampler_dev &b, int vocab) {
-    const auto cut = [](const pk_sampler_dev &p) { return p.top_p < 1.0f && p.top_p > 0.0f; };
-    const int k = samp_kind(a, vocab);
-    if (k != samp_kind(b, vocab)) return false;
-    return k == SAMP_ONE || ((a.rep_penalty > 1.0f) == (b.rep_penalty > 1.0f) && (k != SAMP_NUCLEUS || cut(a) == cut(b)));
+// Which of the captured steps serves these settings: a captured step's
+// kernels read the values on the device, but not which kernels run.
+static int step_key(const pk_sampler_dev &p, int vocab) {
+    const int pen = p.rep_penalty > 1.0f, cut = p.top_p < 1.0f && p.top_p > 0.0f;
+    // greedy without a penalty is the lm_head's own argmax (no draw, no history use)
+    if (!(p.temperature >= 1e-6f) && !pen) return 0;
+    static_assert(PK_STEPS == 8, "one workgroup, top-k, no top-k with and without a cut");
+    switch (samp_kind(p, vocab)) {
+    case SAMP_TOPK: return 2 + pen;
+    case SAMP_NUCLEUS: return 4 + pen + 2 * cut;
+    default: return 1;
+    }
 }
 
 // Parameters into the device state; rng and history replaced only on reset
@@ -1858,16 +1859,9 @@ static int put_params(pk_engine *e, const pk_sampler_dev &p, bool reset) {
     const size_t bytes = reset ? offsetof(pk_sampler_dev, history) : offsetof(pk_sampler_dev, rng);
     PK_HIP(hipMemcpyAsync(e->samp, &p, bytes, hipMemcpyHostToDevice, e->stream));
     PK_HIP(hipStreamSynchronize(e->stream));
-    const pk_sampler_dev was = e->samp_params;
     e->samp_params = p;
-    // greedy without a penalty is the lm_head's own argmax (no draw, no history use)
-    const bool on = p.temperature >= 1e-6f || p.rep_penalty > 1.0f;
-    if (e->step_exec && (on != e->samp_on || !same_launches(was, p, e->c.vocab))) {   // the captured step's launches
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
-    }
-    e->samp_on = on;
+    e->step_key = step_key(p, e->c.vocab);
+    e->samp_on = e->step_key != 0;
     return PK_OK;
 }
 
@@ -1890,14 +1884,8 @@ extern "C" int pk_set_sampling_fast_sums(pk_engine *e, int on) {
     PK_CHECK(e, PK_ERR_ARG, "null argument");
     PK_CHECK(!e->capturing, PK_ERR_ARG, "set_sampling_fast_sums: not available while capturing");
     PK_TRY(pk_sample_reserve(e, e->c.vocab > 0 ? e->c.vocab : 1));
-    const pk_sampler_dev was = e->samp_params;
     e->samp_params.fast_sums = on ? 1 : 0;
-    if (e->step_exec && !same_launches(was, e->samp_params, e->c.vocab)) {
-        (void)hipStreamSynchronize(e->stream);
-        (void)hipGraphExecDestroy(e->step_exec);
-        e->step_exec = nullptr;
-        e->step_cap = -1;
-    }
+    e->step_key = step_key(e->samp_params, e->c.vocab);
     PK_HIP(hipMemcpyAsync((char *)e->samp + offsetof(pk_sampler_dev, fast_sums), &e->samp_params.fast_sums, 4,
                           hipMemcpyHostToDevice, e->stream));
     PK_HIP(hipStreamSynchronize(e->stream));

@@ -34,6 +34,8 @@ for a, sa in enumerate(S):
             else:
                 pa.check(L.pk_set_sampling(h, *sb, 5))
             assert replay(h) == want[b], (sa, sb, turn)
+# each set of launches is captured once, however often the settings change
+assert hh.hh_instantiated() == len(S) + kinds, hh.hh_instantiated()
 pa.check(L.pk_set_sampling(h, 0.8, 0.9, 0, 1.0, 5))
 a = replay(h)
 pa.check(L.pk_set_sampling_fast_sums(h, 1))
