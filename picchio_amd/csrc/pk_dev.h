@@ -2,6 +2,15 @@
 #pragma once
 #include "pk_internal.h"
 
+// Orders a wave's LDS writes before it and reads after it, for values that its
+// own lanes exchange. (A wave's LDS accesses run in order, so this costs no
+// instruction; a wave barrier alone would leave the compiler free to move them.)
+__device__ __forceinline__ void pk_wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ───────────────────────── wave sums ─────────────────────────
 // Sum over the 64 lanes of a wave (all active), every lane getting it. The
 // tree is fixed: lane ^ 1, ^ 2, ^ 4, ^ 8 within each row of 16 lanes (own +

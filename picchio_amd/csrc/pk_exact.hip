@@ -22,6 +22,7 @@
 // expf is evaluated as the double exp rounded to float (pk_expf_cr), which
 // equals glibc's expf except where glibc's result is not the correctly
 // rounded one (about 8e-5 of inputs).
+#include "pk_dev.h"
 #include "pk_engine.h"
 #include "pk_i4_device.h"
 
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(64) void k_gemv_chain8_q8(const float *__restrict__
         const int c0 = n * GQ_KC;
 #pragma unroll
         for (int u = 0; u < 8; ++u) *reinterpret_cast<uint4 *>(wl + (8 * u + lr) * GQ_P + lc) = st[u];
-        __builtin_amdgcn_wave_barrier();
+        pk_wave_lds_order();
         load(min(n + 1, chunks - 1) * GQ_KC);
         const int pieces = min(GQ_KC, I - c0) / 16;
         for (int m = 0; m < pieces; ++m) {
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(64) void k_gemv_chain8_q8(const float *__restrict__
                     }
                 }
         }
-        __builtin_amdgcn_wave_barrier();
+        pk_wave_lds_order();
     }
 #pragma unroll
     for (int t = 0; t < NS; ++t) {

@@ -34,6 +34,7 @@
 // the pick the first index whose exact running sum reaches the draw. The
 // reference's float rounding (about sqrt(n) * 2^-24 relative) then separates
 // the two, so over a flat distribution a cut or a pick moves now and then.
+#include "pk_dev.h"
 #include "pk_engine.h"
 
 #include <cstddef>
@@ -1410,9 +1411,7 @@ __device__ __forceinline__ float om_sum(const float *src, int n, int per, int ru
         mv[i] = ws->mv[i];
         mex[i] = ws->mex[i];
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    pk_wave_lds_order();
     hit = -1;
     float s = 0.0f;
     for (int c = 0; c < runs;) {
