@@ -222,11 +222,15 @@ static int route_rows(pk_engine *e, const rows_scratch &sc, int layer, const flo
                                 e->stream);
 }
 
-// (token, expert) pairs from which the fp32 chains run on k_i4_rows: with
-// fewer, the pair grouping's launch costs more than the shared decodes give
-// (20B layer, 3 tokens 135.6 us either way, 6 tokens 164 against 158 us; 128
-// experts, 3 tokens 142 against 149).
+// (token, expert) pairs from which the fp32 chains run on k_i4_rows: 5 for 8
+// experts, and at least 24. With fewer, most experts have one pair, and the
+// pair grouping's launch costs more than the shared decodes give (a layer of
+// 2880 / 5760, top-4, per pair against grouped: 32 experts, 5 tokens 111 / 105
+// us, 8 tokens 140 / 129; 64 experts, 8 tokens 140 / 143, 10 tokens 163 / 158;
+// 128 experts, 10 tokens 163 / 172, 16 tokens 218 / 213, 20 tokens 258 / 258,
+// 24 tokens 292 / 274).
 constexpr int ROWS_MIN_PAIRS = 24;
+static bool rows_grouped(int P, int E) { return P >= ROWS_MIN_PAIRS && 8 * P >= 5 * E; }
 // Pairs per expert from which the tiles hold 16 rows instead of 8 (32
 // experts: 128 tokens 455 against 428 us, 256 tokens 740 against 746, 512
 // tokens 1252 against 1350).
@@ -269,7 +273,7 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
     const int mt = P / 4 + 1 + E;
     pk_i4_tiles tl{sc.pairs, sc.tiles, sc.tiles + mt, sc.tiles + 2 * mt, sc.tiles + 3 * mt};
     const bool tiled = dot && !e->dot_tiles_off && e->ex.gu.NG <= 64 && e->ex.dn.NG <= 64 && E <= 128;
-    const bool rows = !dot && E <= 128 && P >= ROWS_MIN_PAIRS && pk_i4_rows_ok(gu, PK_EPI_SWIGLU);
+    const bool rows = !dot && E <= 128 && rows_grouped(P, E) && pk_i4_rows_ok(gu, PK_EPI_SWIGLU);
     const int tile = tiled ? 4 : P >= ROWS16_PAIRS * E ? 16 : PK_ROWS_TILE, max_tiles = P / tile + 1 + E;
     if (tiled || rows)
         PK_TRY(pk_launch_group_pairs(sc.sel, P, E, sc.pairs, sc.tiles, sc.tiles + mt,
