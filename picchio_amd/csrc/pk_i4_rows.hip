@@ -347,7 +347,7 @@ __device__ __forceinline__ void rw16_body(const pk_i4_items &it, const int32_t *
     const uint4 *tiles =
         reinterpret_cast<const uint4 *>(base + it.off_tiles) + (int64_t)rb * NG * (PK_TILE_BYTES / 16);
     const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64;
-    auto pair_of = [&](int j) { return pairs ? pairs[beg + j] : beg + j; };
+    auto pair_of = [&](int j) { return pairs[beg + j]; };
     // lane l loads input row l % 16, columns 4 (l / 16) .. + 3 of each 16
     const float *xp = it.x + (int64_t)(pair_of(min(lane & 15, cnt - 1)) / it.x_div) * it.x_stride + 4 * (lane >> 4);
     rw16_stage st[RW16_PF];
@@ -393,7 +393,7 @@ __device__ __forceinline__ void rw_walk(const pk_i4_items &it, const int32_t *pa
     const uint4 *tiles =
         reinterpret_cast<const uint4 *>(base + it.off_tiles) + (int64_t)rb * NG * (PK_TILE_BYTES / 16);
     const float *sc = reinterpret_cast<const float *>(base + it.off_scales) + (int64_t)rb * NG * 64;
-    auto pair_of = [&](int j) { return pairs ? pairs[beg + j] : beg + j; };
+    auto pair_of = [&](int j) { return pairs[beg + j]; };
     const float *xp[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s)
@@ -440,22 +440,13 @@ __device__ __forceinline__ void rw_walk(const pk_i4_items &it, const int32_t *pa
 }
 
 // grid (ceil(RB / 4), tiles): wave w of a workgroup takes row block 4 x + w of
-// tile y (at most 16 rows).
+// tile y of tl (at most 16 pairs).
 template <int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_i4_rows16(
     pk_i4_items it, pk_i4_tiles tl, int O, int NG, int RB, float lim, float alpha) {
     const int rb = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.y;
-    if (rb >= RB) return;
-    int beg, cnt, slot = it.slot_base;
-    if (tl.pairs) {
-        if (t >= *tl.n_tiles) return;
-        beg = tl.tile_beg[t];
-        cnt = tl.tile_cnt[t];
-        slot += tl.tile_exp[t];
-    } else {
-        beg = t * 16;
-        cnt = min(16, it.n_items - beg);
-    }
+    if (rb >= RB || t >= *tl.n_tiles) return;
+    const int beg = tl.tile_beg[t], cnt = tl.tile_cnt[t], slot = it.slot_base + tl.tile_exp[t];
     const uint8_t *base = it.base + (int64_t)slot * it.slot_stride;
     if (cnt > 8) rw16_body<EPI>(it, tl.pairs, beg, cnt, base, rb, O, NG, lim, alpha);
     else if (cnt > 4) rw_walk<2, EPI>(it, tl.pairs, beg, cnt, base, rb, O, NG, lim, alpha);
@@ -475,8 +466,8 @@ int pk_launch_i4_rows(const pk_i4_items &it, const pk_i4_tiles *tl, const pk_i4_
     PK_CHECK(sh.NG <= 128, PK_ERR_UNSUPPORTED, "i4 rows: I=%d above 8192", sh.I);     // (as for one row)
     PK_CHECK(!tl || (tl->pairs && tl->tile_exp && tl->tile_beg && tl->tile_cnt && tl->n_tiles), PK_ERR_ARG,
              "i4 rows: missing tiles");
-    PK_CHECK(tile_rows == 8 || (tile_rows == 16 && epilogue != PK_EPI_ROW_SCALED), PK_ERR_ARG, "i4 rows: tiles of %d",
-             tile_rows);
+    PK_CHECK(tile_rows == 8 || (tile_rows == 16 && tl && epilogue != PK_EPI_ROW_SCALED), PK_ERR_ARG,
+             "i4 rows: tiles of %d", tile_rows);
     // one matrix: tiles of 8 rows, but of 4 where tiles of 8 would leave CUs
     // without a workgroup (5760 x 2880, 8 rows: 9.5 against 13.6 us)
     int tile = tile_rows;
@@ -487,11 +478,11 @@ int pk_launch_i4_rows(const pk_i4_items &it, const pk_i4_tiles *tl, const pk_i4_
     if (tile == 16) {
         const dim3 grid((sh.RB + 3) / 4, tiles);
         if (epilogue == PK_EPI_SWIGLU)
-            hipLaunchKernelGGL(k_i4_rows16<PK_EPI_SWIGLU>, grid, dim3(256), 0, st, it, tl ? *tl : none, sh.O, sh.NG,
-                               sh.RB, lim, alpha);
+            hipLaunchKernelGGL(k_i4_rows16<PK_EPI_SWIGLU>, grid, dim3(256), 0, st, it, *tl, sh.O, sh.NG, sh.RB, lim,
+                               alpha);
         else
-            hipLaunchKernelGGL(k_i4_rows16<PK_EPI_PLAIN>, grid, dim3(256), 0, st, it, tl ? *tl : none, sh.O, sh.NG,
-                               sh.RB, lim, alpha);
+            hipLaunchKernelGGL(k_i4_rows16<PK_EPI_PLAIN>, grid, dim3(256), 0, st, it, *tl, sh.O, sh.NG, sh.RB, lim,
+                               alpha);
         PK_HIP(hipGetLastError());
         return PK_OK;
     }

@@ -238,8 +238,8 @@ int pk_launch_i4_dot_tiles(const pk_i4_items &it, const pk_i4_tiles &tl, const p
 // The fp32-chain GEMV of several input rows on the matrix instructions
 // (pk_i4_rows.hip), the bits of pk_launch_i4_gemv: the pairs of tl's tiles (at
 // most tile_rows = 8 or 16 per tile, x and y indexed by pair) or, with tl
-// null, the it.n_items rows of the one matrix at slot_base. ok: 16-byte
-// aligned input rows, fp32 arithmetic, plain or SwiGLU epilogue.
+// null, the it.n_items rows of the one matrix at slot_base, 8 or 4 per tile.
+// ok: 16-byte aligned input rows, fp32 arithmetic, plain or SwiGLU epilogue.
 constexpr int PK_ROWS_TILE = 8;
 int pk_device_cus();               // compute units of the current device
 bool pk_i4_rows_ok(const pk_i4_items &it, int epilogue);
