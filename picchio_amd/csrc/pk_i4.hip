@@ -998,57 +998,68 @@ __global__ void k_quantize_i4(const float *w, int O, int I, int glen, int ng, in
 }
 
 // The same for a group length of 4 .. 256 that is a power of two: a wave takes
-// a row, V adjacent columns per lane and 64 V per step (V = 4 for 16-byte
-// aligned rows, else 1), with every step's loads of QZ_U steps in flight; a
-// group is GL / V adjacent lanes, whose maximum a few lane exchanges give. A
-// thread per group (above) reads 256 bytes apart from its neighbours: 5760 x
-// 2880 took 223 us there (with the launch), 23 here.
+// `per` spans of 64 V QZ_U columns of a row (whole groups), V adjacent columns
+// per lane and 64 V per step (V = 4 for 16-byte aligned rows, else 1), with a
+// span's loads in flight; a group is glen / V adjacent lanes, whose maximum a
+// few lane exchanges give. A thread per group (above) reads glen * 4 bytes
+// apart from its neighbours. Measured (us with the launch, above / here): 5760
+// x 2880, gs 64: 224 / 20.6; 32 x 100000, gs 64: 32 / 7 (216 with a wave per
+// row); 100000 x 64 as one row, gs 4: 17.5 / 9.2 (34 row by row).
 constexpr int QZ_U = 4;
+constexpr int64_t QZ_WAVES = 16384;       // (20000 x 2880, gs 64, 60000 spans: 57 us; 64 with a wave per span)
 template <int V>
-__global__ __launch_bounds__(256) void k_quantize_i4_rows(const float *__restrict__ w, int O, int I, int glen, int ng,
+__global__ __launch_bounds__(256) void k_quantize_i4_rows(const float *__restrict__ w, int O, int64_t I, int glen,
+                                                          int64_t ng, int spans, int per,
                                                           uint8_t *__restrict__ packed, float *__restrict__ scales) {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    constexpr int SPAN = 64 * V * QZ_U;
+    const int lane = threadIdx.x & 63, wpr = (spans + per - 1) / per;          // waves per row
+    const int64_t task = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = (int)(task / wpr), first = (int)(task - (int64_t)row * wpr) * per;
     if (row >= O) return;
     const float *wr = w + (int64_t)row * I;
     uint8_t *pr = packed + (int64_t)row * ((I + 1) / 2);
     float *sr = scales + (int64_t)row * ng;
     const int span = glen / V;                       // lanes per group
-    for (int base = 0; base < I; base += 64 * V * QZ_U) {
+    const int gsh = 31 - __clz(glen);
+    for (int sp = first; sp < min(first + per, spans); ++sp) {
+        const int64_t base = (int64_t)sp * SPAN;
+        const int n_in = (int)min((int64_t)SPAN, I - base);                    // columns of this span
+        const float *wb = wr + base;
         float v[QZ_U][V];
 #pragma unroll
         for (int u = 0; u < QZ_U; ++u) {
-            const int c = base + (u * 64 + lane) * V;
+            const int c = (u * 64 + lane) * V;
             if constexpr (V == 4) {
-                const float4 t = *reinterpret_cast<const float4 *>(wr + min(c, I - 4));
+                const float4 t = *reinterpret_cast<const float4 *>(wb + min(c, n_in - 4));
                 v[u][0] = t.x; v[u][1] = t.y; v[u][2] = t.z; v[u][3] = t.w;
             } else {
-                v[u][0] = wr[min(c, I - 1)];
+                v[u][0] = wb[min(c, n_in - 1)];
             }
         }
 #pragma unroll
         for (int u = 0; u < QZ_U; ++u) {
-            const int c = base + (u * 64 + lane) * V;
-            const bool in = c < I;
+            const int c = (u * 64 + lane) * V;
+            const bool in = c < n_in;
             float amax = 0.0f;
 #pragma unroll
             for (int k = 0; k < V; ++k) amax = fmaxf(amax, in ? fabsf(v[u][k]) : 0.0f);
             for (int o = 1; o < span; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
             const float s = amax > 1e-8f ? amax / 7.0f : 1e-8f;
-            if (in && (lane & (span - 1)) == 0) sr[c / glen] = s;
+            if (in && (lane & (span - 1)) == 0) sr[(base + c) >> gsh] = s;
             int n[V];
 #pragma unroll
             for (int k = 0; k < V; ++k) {
                 const float r = fminf(fmaxf(rintf(v[u][k] / s), -8.0f), 7.0f);
                 n[k] = in ? ((int)r + 8) & 15 : 0;
             }
+            uint8_t *pb = pr + ((base + c) >> 1);
             if constexpr (V == 4) {
                 const uint16_t b = (uint16_t)(n[0] | (n[1] << 4) | (n[2] << 8) | (n[3] << 12));
-                if (in) *reinterpret_cast<uint16_t *>(pr + (c >> 1)) = b;
+                if (in) *reinterpret_cast<uint16_t *>(pb) = b;
             } else {
                 // even lanes store the pair; the last column of an odd row keeps a zero high nibble
                 const int hi = __shfl_down(n[0], 1, 64);
-                if (in && (lane & 1) == 0) pr[c >> 1] = (uint8_t)(n[0] | (c + 1 < I ? hi << 4 : 0));
+                if (in && (lane & 1) == 0) *pb = (uint8_t)(n[0] | (c + 1 < n_in ? hi << 4 : 0));
             }
         }
     }
@@ -1062,12 +1073,26 @@ int pk_launch_quantize_i4(const float *w, int O, int I, int gs, uint8_t *packed,
     const int ng = per_row_scale ? 1 : (I + gs - 1) / gs;
     if (ng > 1 && glen >= 4 && glen <= 256 && (glen & (glen - 1)) == 0) {
         const bool v4 = (I & 3) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)packed & 1) == 0;
-        if (v4 || glen <= 64) {
-            const dim3 grid((O + 3) / 4);
+        // (unaligned rows: groups of 4 are 16 bytes apart already, 5760 x 2881 40
+        // us above, 44 here; of 8, 64 and 47)
+        if (v4 || (glen >= 8 && glen <= 64)) {
+            // rows of whole groups are one long row (neither values nor bytes nor
+            // scales lie between them)
+            const bool flat = v4 && I % glen == 0;
+            const int64_t cols = flat ? (int64_t)O * I : I, groups = flat ? (int64_t)O * ng : ng;
+            const int rows = flat ? 1 : O, step = 64 * QZ_U * (v4 ? 4 : 1);
+            const int64_t spans = (cols + step - 1) / step;
+            // a wave per span, several beyond QZ_WAVES
+            const int64_t per = std::min(std::max<int64_t>(rows * spans / QZ_WAVES, 1), spans);
+            const int64_t blocks = (rows * ((spans + per - 1) / per) + 3) / 4;
+            PK_CHECK(spans <= 0x7fffffff && blocks <= 0x7fffffff, PK_ERR_UNSUPPORTED, "quantize: %d x %d", O, I);
+            const dim3 grid((unsigned)blocks);
             if (v4)
-                hipLaunchKernelGGL(k_quantize_i4_rows<4>, grid, dim3(256), 0, st, w, O, I, glen, ng, packed, scales);
+                hipLaunchKernelGGL(k_quantize_i4_rows<4>, grid, dim3(256), 0, st, w, rows, cols, glen, groups,
+                                   (int)spans, (int)per, packed, scales);
             else
-                hipLaunchKernelGGL(k_quantize_i4_rows<1>, grid, dim3(256), 0, st, w, O, I, glen, ng, packed, scales);
+                hipLaunchKernelGGL(k_quantize_i4_rows<1>, grid, dim3(256), 0, st, w, rows, cols, glen, groups,
+                                   (int)spans, (int)per, packed, scales);
             PK_HIP(hipGetLastError());
             return PK_OK;
         }

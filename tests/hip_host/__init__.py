@@ -20,7 +20,7 @@ sys.path.insert(0, {root!r})
 import picchio_amd as pa
 L = pa.lib()
 hh.hh_name.restype = C.c_char_p
-hh.hh_in_use.restype = hh.hh_peak.restype = C.c_int64
+hh.hh_in_use.restype = hh.hh_peak.restype = hh.hh_groups.restype = C.c_int64
 hh.hh_budget.argtypes = [C.c_int64]
 vp = C.c_void_p
 

@@ -74,6 +74,7 @@ int hh_stale() { return stale; }
 int hh_execs() { return execs; }
 int hh_instantiated() { return instantiated; }
 int hh_launches() { return (int)log_.size(); }
+int64_t hh_groups(int i) { return (int64_t)log_[i].grid.x * log_[i].grid.y * log_[i].grid.z; }
 const char *hh_name(int i) { return log_[i].name.c_str(); }
 void hh_clear() { log_.clear(); }
 
