@@ -364,6 +364,12 @@ constexpr int OS_E = 8;                   // elements per thread
 constexpr int OS_CHUNK = OS_E * SNT;
 constexpr int OS_BUF = OS_CHUNK + OS_CHUNK / OS_E;     // LDS floats (rows of 8 set 9 apart)
 constexpr uint32_t OS_BIG = 1u << 25;     // a move past the binade
+// The first OS_HEAD elements are added by one thread (2.4 ns each): a sum's
+// first binades are short, and each costs a scan of the chunk (2.3 us). A draw
+// in one workgroup, no cut, 5000 flat entries: 62 us with every element on one
+// thread, 76 with the scan alone, 53 so (256 elements 55, 2048 60); 16000: 141,
+// 87 and 65.
+constexpr int OS_HEAD = 512;
 
 // a's moves, then b's (the callers clamp to OS_BIG before 32 bits could
 // overflow: 8 elements, 64 lanes, 16 waves)
@@ -413,6 +419,7 @@ __device__ __forceinline__ void order_sum(const float *src, int n, float *buf, b
     __shared__ uint2 s_wave[NW];
     __shared__ float os_s;
     __shared__ int os_start, os_hit;
+    static_assert(OS_HEAD % (4 * OS_E) == 0 && OS_HEAD <= OS_CHUNK, "four rows of elements at a time");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float s = 0.0f;
     int hit = -1;
@@ -435,6 +442,38 @@ __device__ __forceinline__ void order_sum(const float *src, int n, float *buf, b
 #pragma unroll
         for (int k = 0; k < OS_E; ++k) v[k] = buf[(OS_E + 1) * tid + k];
         int start = 0;                                     // the chunk's elements before it are in s
+        if (base == 0) {
+            if (tid == 0) {
+                float x = 0.0f;
+                int at = -1;
+                for (int row = 0; row < OS_HEAD / OS_E && at < 0; row += 4) {      // (zeros past n: + 0)
+                    float t[4 * OS_E];
+#pragma unroll
+                    for (int k = 0; k < 4 * OS_E; ++k) t[k] = buf[(OS_E + 1) * (row + k / OS_E) + k % OS_E];
+                    const float x0 = x;
+#pragma unroll
+                    for (int k = 0; k < 4 * OS_E; ++k) x = x + t[k];
+                    if (find && x >= r) {                  // (the sum only grows: the crossing is among these)
+                        x = x0;
+                        for (int k = 0; k < 4 * OS_E && at < 0; ++k) {
+                            x = x + buf[(OS_E + 1) * (row + k / OS_E) + k % OS_E];
+                            if (x >= r) at = OS_E * row + k;
+                        }
+                    }
+                }
+                os_s = x;
+                os_hit = at;
+            }
+            __syncthreads();
+            s = os_s;
+            hit = os_hit;
+            start = OS_HEAD;
+            if (OS_E * tid < start) {
+#pragma unroll
+                for (int k = 0; k < OS_E; ++k) v[k] = 0.0f;
+            }
+            if (hit >= 0 || !(s < INFINITY)) break;
+        }
         while (start < OS_CHUNK) {
             const uint32_t sb = __float_as_uint(s);
             const int ex = max((int)(sb >> 23), 1);        // s = S 2^(ex - 150)

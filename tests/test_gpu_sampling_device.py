@@ -73,3 +73,17 @@ def test_ordered_sum_runs(samp_eng, oracle, case, size):  # noqa: F811
     expf is exact."""
     _check_draws(samp_eng, oracle, case, size, 2, lambda s: np.zeros(size, np.float32))
     samp_eng.set_sampling(0.0, 1.0, 0, 1.0, 1)
+
+
+@pytest.mark.parametrize("kind", ["normal", "equal", "late", "inf"])
+@pytest.mark.parametrize("case", [(1.0, 1.0, 0, 1.0), (1.0, 0.9, 0, 1.0), (1.0, 1.0, 4500, 1.0)],
+                         ids=["draw", "top-p", "top-k"])
+@pytest.mark.parametrize("size", [4097, 5003, 12001])
+def test_one_workgroup_ordered_sums(samp_eng, oracle, size, case, kind):  # noqa: F811
+    """Ordered sums of one workgroup: picks and cuts in the part that one thread
+    adds, at its end and in the scan after it. (Not "steps": where every add is
+    half way, an ulp of the device's expf in each of n terms moves the sum by up
+    to n 2^-24 relative, past the 4e-6 that the arrays are held to.)"""
+    rng = np.random.default_rng(size)
+    _check_draws(samp_eng, oracle, case, size, 12, lambda s: _logits(kind, rng, size).astype(np.float32))
+    samp_eng.set_sampling(0.0, 1.0, 0, 1.0, 1)
