@@ -928,13 +928,10 @@ extern "C" int pk_matmul_qt(pk_engine *e, float *y, const float *x, const pk_qt 
             it.x = x; it.x_stride = w->I;
             it.y = y; it.y_stride = w->O;
             it.n_items = S;
-            // several rows, once a workgroup per (row block, row) exceeds the CUs: each
-            // weight decoded once per 4 rows (5760 x 2880: 2 rows 7.2 against 9.5 us,
-            // 3 rows 12.2 against 9.5, 64 rows 117 against 36)
             PK_CHECK(w->gs > 0 || S <= 65535, PK_ERR_ARG, "matmul_qt: INT4 row scales, S=%d", S);
             const int epi = w->gs > 0 ? PK_EPI_PLAIN : PK_EPI_ROW_SCALED;
             // (beyond 65535 tiles the grid ends: the per-row launch, as for one row)
-            if ((int64_t)S * w->sh.RB > pk_device_cus() && S >= 2 && S <= 65535 * PK_ROWS_TILE && pk_i4_rows_ok(it, epi))
+            if (S >= 2 && S <= 65535 * PK_ROWS_TILE && pk_i4_rows_pays(w->sh, S) && pk_i4_rows_ok(it, epi))
                 return pk_launch_i4_rows(it, nullptr, w->sh, epi, 0.f, 0.f, 0, e->stream);
             return pk_launch_i4_gemv(it, w->sh, epi, 0.f, 0.f, nullptr, e->stream);
         }

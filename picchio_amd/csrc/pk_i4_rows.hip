@@ -459,6 +459,22 @@ bool pk_i4_rows_ok(const pk_i4_items &it, int epilogue) {
     return !it.xq && !it.yq && epilogue != PK_EPI_COMBINE && (it.x_stride & 3) == 0 && ((uintptr_t)it.x & 15) == 0;
 }
 
+// A workgroup per (row block, row) takes as long as its groups while a CU has
+// at most two; beyond, each further one adds its time, and decoding a weight
+// once per 4 rows pays. Here a row block takes a span of 48 groups at a time,
+// whole spans' time whatever the last one holds, so that with one or two
+// workgroups per CU it pays for rows that fill 3/4 of their spans. Per row /
+// here, us: 1024 x 1024, 17 rows (272 workgroups) 6.4 / 9.8, 33 rows (528)
+// 11.3 / 9.7; 5760 x 576, 3 rows 5.8 / 8.4, 6 rows 10.0 / 8.6; 4096 x 4096, 8
+// rows (512) 15.4 / 16.6, 9 rows 20.3 / 16.8; 2048 x 2048, 9 rows 9.4 / 10.0;
+// 2880 x 2880, 6 rows (270) 13.0 / 10.1; 5760 x 2880, 3 rows 12.4 / 10.0; 2880 x
+// 5760, 6 rows 21.6 / 17.1; 2880 x 8192, 6 rows 28.5 / 24.0.
+bool pk_i4_rows_pays(const pk_i4_shape &sh, int64_t n) {
+    const int span = RW_WAVES * RW_GW, spans = (sh.NG + span - 1) / span;
+    const int64_t blocks = n * sh.RB, n_cu = pk_device_cus();
+    return blocks > 2 * n_cu || (blocks > n_cu && 4 * sh.NG >= 3 * span * spans);
+}
+
 int pk_launch_i4_rows(const pk_i4_items &it, const pk_i4_tiles *tl, const pk_i4_shape &sh, int epilogue, float lim,
                       float alpha, int max_tiles, hipStream_t st, int tile_rows) {
     PK_CHECK(pk_i4_rows_ok(it, epilogue), PK_ERR_ARG, "i4 rows: inputs not 16-byte aligned, or not the fp32 chains");

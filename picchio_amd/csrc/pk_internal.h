@@ -243,6 +243,7 @@ int pk_launch_i4_dot_tiles(const pk_i4_items &it, const pk_i4_tiles &tl, const p
 constexpr int PK_ROWS_TILE = 8;
 int pk_device_cus();               // compute units of the current device
 bool pk_i4_rows_ok(const pk_i4_items &it, int epilogue);
+bool pk_i4_rows_pays(const pk_i4_shape &sh, int64_t n);        // for n rows of one matrix
 int pk_launch_i4_rows(const pk_i4_items &it, const pk_i4_tiles *tl, const pk_i4_shape &sh, int epilogue, float lim,
                       float alpha, int max_tiles, hipStream_t st, int tile_rows = PK_ROWS_TILE);
 

@@ -160,3 +160,33 @@ def test_i4_upload_in_pieces(gpu, oracle):
                 assert bits_equal(y, ref), first_mismatch(y, ref)
             else:                                       # (20 roundings at most of sums of these terms)
                 assert (np.abs(y - sums.sum(1) * s[:, 0]) <= 20 * 2.0 ** -24 * size * s[:, 0]).all()
+
+
+@pytest.mark.parametrize("O,I,S", [(64, 64, 513), (130, 128, 175), (200, 3136, 129), (70, 6208, 257), (4000, 128, 9)])
+def test_i4_rows_edges_bitexact(gpu, oracle, O, I, S):
+    """The shapes above with rows enough for k_i4_rows whatever their groups
+    fill, and a scale per row beside (order free: against the exact sum)."""
+    import picchio_amd as pa
+    import torch
+    q4, s = oracle.quant_gs(_rand((O, I), 5 + O + I, 0.02), 64)
+    x = _rand((S, I), 9 + S)
+    y_ref = oracle.mm_i4_gs(x, q4, s, O, I, 64)
+    b = np.asarray(q4).reshape(O, I // 2)
+    q = np.empty((O, I), np.float64)
+    q[:, 0::2], q[:, 1::2] = (b & 15).astype(np.float64) - 8, (b >> 4).astype(np.float64) - 8
+    rs = (np.random.default_rng(1).random(O) + 0.5).astype(np.float32)
+    with pa.Engine(pa.gptoss_cfg(n_layers=1, n_experts=4, ctx_len=16, vocab=64)) as eng:
+        xd, yd = eng.to_dev(x), eng.empty((S, O), torch.float32)
+        got = []
+        for gs, sc in ((64, s), (0, rs)):
+            qt = eng.qt_upload(pa.FMT_INT4, q4, sc, O, I, gs)
+            eng.matmul_qt(yd, xd, qt, S)
+            got.append(eng.to_host(yd).copy())
+            eng.qt_free(qt)
+    assert bits_equal(got[0], y_ref), first_mismatch(got[0], y_ref)
+    # a product and its sum: 8 in a chain + 3 in its tree, 4 of a wave's 12
+    # groups pairwise, 4 waves per span, the scale
+    xd64, depth = x.astype(np.float64), 8 + 3 + 4 + 4 * (-(-I // 3072)) + 1
+    exact = (xd64 @ q.T) * rs
+    bound = (np.abs(xd64) @ np.abs(q).T) * rs * depth * 2.0 ** -24
+    assert (np.abs(got[1] - exact) <= bound).all()
