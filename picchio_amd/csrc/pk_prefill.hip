@@ -222,15 +222,20 @@ static int route_rows(pk_engine *e, const rows_scratch &sc, int layer, const flo
                                 e->stream);
 }
 
-// (token, expert) pairs from which the fp32 chains run on k_i4_rows: 5 for 8
-// experts, and at least 24. With fewer, most experts have one pair, and the
-// pair grouping's launch costs more than the shared decodes give (a layer of
-// 2880 / 5760, top-4, per pair against grouped: 32 experts, 5 tokens 111 / 105
-// us, 8 tokens 140 / 129; 64 experts, 8 tokens 140 / 143, 10 tokens 163 / 158;
-// 128 experts, 10 tokens 163 / 172, 16 tokens 218 / 213, 20 tokens 258 / 258,
-// 24 tokens 292 / 274).
-constexpr int ROWS_MIN_PAIRS = 24;
-static bool rows_grouped(int P, int E) { return P >= ROWS_MIN_PAIRS && 8 * P >= 5 * E; }
+// When the fp32 chains of P (token, expert) pairs run on k_i4_rows, grouped by
+// expert: from 5 pairs for 8 experts on (with fewer, nearly every pair has an
+// expert of its own and no decode is shared), and from 12 row blocks of the
+// pairs' gate_up and down per CU on (with fewer, the grouping's launch and the
+// long waves of its few tiles cost more than the decodes they share). A layer,
+// us, per pair / grouped: 2880 / 5760, top-4 of 32 experts, 5 tokens 110 / 101,
+// 6 tokens 122 / 118; of 64 experts, 8 tokens 140 / 143, 10 tokens 163 / 158; of
+// 128, 10 tokens 163 / 159 to 172, 20 tokens 257 / 237; 1024 / 2048, top-4 of 32,
+// 16 tokens (3072 row blocks) 66 / 69, 20 tokens 74 / 70; 640 / 1280 of 32, 24
+// tokens (2880) 57 / 59, 32 tokens 62 / 59; 256 / 512, top-2 of 8, 24 tokens (576)
+// 23 / 34, 128 tokens (3072) 40 / 42, 200 tokens 52 / 42.
+static bool rows_grouped(const pk_engine *e, int P) {
+    return 8 * P >= 5 * e->c.n_experts && (int64_t)P * (e->ex.gu.RB + e->ex.dn.RB) >= 12 * (int64_t)pk_device_cus();
+}
 // Pairs per expert from which the tiles hold 16 rows instead of 8 (32
 // experts: 128 tokens 455 against 428 us, 256 tokens 740 against 746, 512
 // tokens 1252 against 1350).
@@ -273,7 +278,7 @@ static int moe_rows_on(pk_engine *e, const rows_scratch &sc, int layer, const fl
     const int mt = P / 4 + 1 + E;
     pk_i4_tiles tl{sc.pairs, sc.tiles, sc.tiles + mt, sc.tiles + 2 * mt, sc.tiles + 3 * mt};
     const bool tiled = dot && !e->dot_tiles_off && e->ex.gu.NG <= 64 && e->ex.dn.NG <= 64 && E <= 128;
-    const bool rows = !dot && E <= 128 && rows_grouped(P, E) && pk_i4_rows_ok(gu, PK_EPI_SWIGLU);
+    const bool rows = !dot && E <= 128 && rows_grouped(e, P) && pk_i4_rows_ok(gu, PK_EPI_SWIGLU);
     const int tile = tiled ? 4 : P >= ROWS16_PAIRS * E ? 16 : PK_ROWS_TILE, max_tiles = P / tile + 1 + E;
     if (tiled || rows)
         PK_TRY(pk_launch_group_pairs(sc.sel, P, E, sc.pairs, sc.tiles, sc.tiles + mt,

@@ -1,17 +1,22 @@
 """Which launches the batched MoE's experts take, on the host side alone
-(hip_host): one per (token, expert) pair while most experts have a single
-pair, grouped by expert beyond."""
+(hip_host): one per (token, expert) pair, or grouped by expert where experts
+have several and their rows fill the device."""
 import pytest
 
 from hip_host import run
 
 
-@pytest.mark.parametrize("E,single,grouped", [(8, 5, 6), (32, 5, 6), (64, 9, 10), (128, 19, 20)])
-def test_pairs_are_grouped_by_pairs_per_expert(E, single, grouped):
+@pytest.mark.parametrize("D,inter,E,single,grouped", [
+    # (136 row blocks of gate_up and down, as many as 2880 / 5760 has but for one)
+    (128, 8576, 8, 5, 6), (128, 8576, 32, 5, 6), (128, 8576, 64, 9, 10), (128, 8576, 128, 19, 20),
+    # small experts: 12 row blocks per CU
+    (128, 256, 8, 127, 128), (256, 512, 8, 63, 64), (1024, 2048, 32, 15, 16)])
+def test_pairs_are_grouped_where_it_pays(D, inter, E, single, grouped):
+    """On 256 CUs."""
     run(f"""
-h = engine(small(n_layers=1, n_experts={E}, vocab=64, ctx_len=64))
-x, out = dev(64 * 128), dev(64 * 128)
-for T, rows in ((1, False), ({single}, False), ({grouped}, True), (64, True)):
+h = engine(small(n_layers=1, n_experts={E}, vocab=64, ctx_len=64, hidden={D}, moe_inter={inter}))
+x, out = dev(256 * {D}), dev(256 * {D})
+for T, rows in ((1, False), ({single}, False), ({grouped}, True), (256, True)):
     hh.hh_clear()
     pa.check(L.pk_moe_forward_batch(h, 0, x, T, out, None, None))
     n = launches()
