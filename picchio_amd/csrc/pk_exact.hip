@@ -50,8 +50,8 @@ namespace {
 //  * NS: the same chains as v_fma, one per lane and input row.
 // The second wave's chains join the first's through LDS for hsum256's tree.
 // Measured (us, fp32, against the kernel before it: 64 rows x 32 outputs per
-// workgroup on v_fma): 5120 x 2880, 1 row 179 -> 17.5, 64 rows 178 -> 55;
-// INT8 201088 x 2880, 1 row 4100 -> 230 (k_gemv_chain8_q8: 132).
+// workgroup on v_fma): 5120 x 2880, 1 row 179 -> 12.2, 64 rows 178 -> 44;
+// INT8 201088 x 2880, 1 row 4100 -> 234 (k_gemv_chain8_q8: 130).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 
@@ -243,8 +243,8 @@ __global__ __launch_bounds__(CH_THREADS) void k_gemm_chain8(const float *__restr
 // 144 bytes apart: 16-byte reads of 16 rows on distinct banks), the next
 // chunk's loads in flight. Per weight one conversion and NS fused
 // multiply-adds (2.2 + 1.25 NS ns per 64 and SIMD), so it is bound by the
-// weight stream. 201088 x 2880, 1 row: 132 us = 4.4 TB/s;
-// k_gemm_chain8 230 (it keeps the weights in LDS as floats).
+// weight stream. 201088 x 2880, 1 row: 130 us = 4.5 TB/s;
+// k_gemm_chain8 234 (it keeps the weights in LDS as floats).
 constexpr int GQ_KC = 128, GQ_P = GQ_KC + 16;
 template <int NS>
 __global__ __launch_bounds__(64) void k_gemv_chain8_q8(const float *__restrict__ X, const int8_t *__restrict__ W,
@@ -306,8 +306,8 @@ __global__ __launch_bounds__(64) void k_gemv_chain8_q8(const float *__restrict__
 // 32 q .. with v_mfma_f32_32x32x1_2b_f32: lane l = 32 b + r reads columns
 // 8k + 4b .. + 3 of weight row r and input row r as one float4 each, and
 // instruction i multiplies component i, its two blocks being chains i and
-// 4 + i. Chunks of 32 columns, staged as above. 5120 x 2880, 512 rows: 183 us
-// (82 TFLOP/s; 367 in 16-row tiles).
+// 4 + i. Chunks of 32 columns, staged as above. 5120 x 2880, 512 rows: 164 us
+// (92 TFLOP/s; 349 in 16-row tiles).
 constexpr int CT_TILE = 64, CT_KC = 32, CT_P = CT_KC + 4;
 template <typename TW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_chain8_tile(
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(128) void k_router_seq(const float *__restrict__ X,
 // multiplied in ~0.3 us, so RQ_PF chunks' loads are in flight in registers.
 // A chunk passes through the wave's own LDS (rows 4 mod 64 floats apart, read
 // as float4): several waves of one workgroup would share the loads but are
-// bound by their LDS reads. 64 rows x 32 experts x 2880: 35 us; 38 with four
+// bound by their LDS reads. 64 rows x 32 experts x 2880: 30 us; 38 with four
 // waves per workgroup, 70 with two and one chunk in flight.
 constexpr int RQ_P = RS_KC + 4;          // padded LDS row (floats)
 constexpr int RQ_PF = 4;                 // chunks in flight
@@ -612,10 +612,23 @@ __global__ __launch_bounds__(64) void k_router_seq4(const float *__restrict__ X,
 
 }  // namespace
 
-// 64 x 64 tiles from about 5 for 8 CUs (a tile's serial columns take ~95 us
-// however few there are; 5120 x 2880: 128 rows 95 against 105 us in 16-row
-// tiles, 512 rows 183 against 367, 64 rows 55 in 16-row tiles); else 16-row
-// tiles, one or two rows on v_fma.
+// Whether more than 32 rows (16-byte loads) run in 64 x 64 tiles: where the
+// 16-row tiles take longer. At 2880 columns those take 8.6 us per workgroup (16
+// outputs x 16 rows) and CU, the 64 x 64 tiles 12 us and 52 per round of the CUs.
+// fp32, 16-row / 64 x 64 tiles, us: 5120 x 2880, 96 rows (7.5 per CU, one round)
+// 61 / 64, 128 rows 87 / 64, 512 rows 349 / 164; 2880 x 4096, 160 rows (7.0) 88 /
+// 90, 192 rows (8.4) 108 / 90; 16000 x 2880, 33 rows 98 / 65, 65 rows 169 / 111;
+// 1000 x 2880, 320 rows (4.9) 51 / 64, 512 rows (7.9) 75 / 65. int8, whose 64 x 64
+// tiles also convert the weights: 5120 x 2880, 96 rows 62 / 72; 1000 x 2880, 512
+// rows 66 / 72; 2880 x 4096, 192 rows 104 / 101.
+static bool chain8_tiled(int S, int O, bool i8) {
+    const int64_t cus = pk_device_cus();
+    const int64_t tiles = (int64_t)((O + CT_TILE - 1) / CT_TILE) * ((S + CT_TILE - 1) / CT_TILE);
+    const int64_t few = (int64_t)((O + CH_OUTS - 1) / CH_OUTS) * ((S + 15) / 16), rounds = (tiles + cus - 1) / cus;
+    return S > 32 && 2 * few > ((i8 ? 5 : 3) + 12 * rounds) * cus;
+}
+
+// (16-row tiles: one or two rows on v_fma)
 template <typename TW>
 static int launch_chain8(const float *X, int64_t ldx, const TW *W, const float *rscale, const float *bias, float *out,
                          int64_t ldo, int S, int I, int O, bool add_res, hipStream_t st) {
@@ -623,7 +636,7 @@ static int launch_chain8(const float *X, int64_t ldx, const TW *W, const float *
     PK_CHECK((S + 63) / 64 <= CH_MAX_Y, PK_ERR_UNSUPPORTED, "gemm chain8: %d rows", S);
     const bool vec = (ldx & 3) == 0 && I % (16 / (int)sizeof(TW)) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0;
     const int64_t ot = (O + CT_TILE - 1) / CT_TILE, rt = (S + CT_TILE - 1) / CT_TILE;
-    if (vec && S > 32 && 8 * ot * rt >= 5 * (int64_t)pk_device_cus()) {
+    if (vec && chain8_tiled(S, O, sizeof(TW) == 1)) {
         hipLaunchKernelGGL(k_gemm_chain8_tile<TW>, dim3((unsigned)ot, (unsigned)rt), dim3(256), 0, st, X, ldx, W,
                            rscale, bias, out, ldo, S, I, O, add_res ? 1 : 0);
         PK_HIP(hipGetLastError());
@@ -654,10 +667,11 @@ int pk_launch_gemm_chain8(const float *X, int64_t ldx, const float *W, const flo
 int pk_launch_gemm_chain8_q8(const float *X, const int8_t *W, const float *scale, float *out, int S, int I, int O,
                              hipStream_t st) {
     PK_CHECK(S > 0 && I > 0 && O > 0 && scale, PK_ERR_ARG, "gemm chain8 q8: bad argument");
-    // a wave per 64 outputs, once that gives every SIMD a wave (16,000 outputs,
-    // 250 waves: 32 against 23 us in k_gemm_chain8)
+    // a wave per 64 outputs from three waves per CU on (k_gemm_chain8 / here, us at
+    // 2880 columns: 16000 outputs, 1 row 23 / 32; 32000, 1 row 42 / 37, 4 rows 63 /
+    // 71; 50000, 1 row 66 / 40, 4 rows 102 / 73; 201088, 1 row 234 / 130)
     if (S <= 4 && (I & 15) == 0 && (((uintptr_t)X | (uintptr_t)W) & 15) == 0 &&
-        (O + 63) / 64 >= 4 * pk_device_cus()) {
+        (O + 63) / 64 >= 3 * pk_device_cus()) {
         const dim3 grid((O + 63) / 64);
         if (S == 1) hipLaunchKernelGGL(k_gemv_chain8_q8<1>, grid, dim3(64), 0, st, X, W, scale, out, S, I, O);
         else if (S == 2) hipLaunchKernelGGL(k_gemv_chain8_q8<2>, grid, dim3(64), 0, st, X, W, scale, out, S, I, O);

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("offset", [0, 1], ids=["aligned", "unaligned"])
 @pytest.mark.parametrize("O,I,S", [(1, 8, 1), (17, 136, 1), (33, 1444, 2), (5, 7, 3), (17, 1441, 16), (300, 2880, 16),
                                    (48, 272, 17), (31, 64, 33), (160, 2880, 64), (16390, 144, 65), (7, 4096, 129), (65700, 48, 1),
-                                   (65700, 144, 3)])
+                                   (65700, 144, 3), (4096, 48, 130), (49090, 80, 2)])
 def test_chain8_bitexact(gpu, oracle, O, I, S, offset):
     import picchio_amd as pa
     import torch
