@@ -588,7 +588,7 @@ static int prefill_rows(pk_engine *e, int seq, const int32_t *ids, const int32_t
 // PREFILL_ROWS, where nothing depends on the chunk (the matrix-core MoE and
 // the router trace keep one chunk per pass; so do windows that
 // k_attn_rows_exact does not hold). 512 tokens, four 20B layers: 17.7 ms
-// in chunks of 64 (each with its lm_head), 8.5 in one pass: full tiles of the
+// in chunks of 64 (each with its lm_head), 7.9 in one pass: full tiles of the
 // experts' rows, 512-row projections, one lm_head.
 constexpr int PREFILL_ROWS = 512;
 
