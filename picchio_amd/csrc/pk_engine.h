@@ -3,7 +3,6 @@
 
 #include "pk_internal.h"
 
-#include <atomic>
 #include <memory>
 #include <vector>
 
@@ -113,10 +112,15 @@ struct pk_engine {
     uint64_t *att_t = nullptr;                // k_attn_oproj hand-over words: [heads x head_dim]
 
     bool capturing = false;                  // inside pk_capture_begin/end
-    // captured graphs (pk_graph) not yet destroyed, and the buffers outgrown
-    // while there were any: their kernels may address them (pk_regrow)
-    std::shared_ptr<std::atomic<int>> live_graphs = std::make_shared<std::atomic<int>>(0);
-    std::vector<void *> outgrown;
+    // One token per set of growing buffers (b_*, g_*): a captured graph
+    // (pk_graph), whose kernels may address the buffers, shares the tokens of its
+    // time. Buffers outgrown meanwhile stay until no graph holds their token.
+    std::shared_ptr<char> b_use = std::make_shared<char>(), g_use = std::make_shared<char>();
+    struct outgrown_set {
+        std::shared_ptr<char> use;
+        std::vector<void *> bufs;
+    };
+    std::vector<outgrown_set> outgrown;
 
     // diagnostics (outside graph capture only): every MoE router launch
     // appends its logits [rows][E] to rtrace (pk_set_router_trace); with
@@ -201,17 +205,17 @@ int pk_noalloc_scratch_init(pk_engine *e);
 
 int pk_dev_alloc(pk_engine *e, void **p, int64_t bytes);
 void pk_dev_free(pk_engine *e, void *p);
-// Larger buffers in the place of *b[i].p (their contents are not kept). Where
-// old and new do not fit together the old ones go first, unless the growth is
-// optional or a captured graph may address them: then, on an error, they stay
-// as they are (else null). Replaced ones are freed, or while a captured graph
-// lives, kept for its kernels until the next growth without one, or the
-// engine's end.
+// Larger buffers in the place of *b[i].p (their contents are not kept), a set
+// whose token is `use`. Where old and new do not fit together the old ones go
+// first, unless the growth is optional or a captured graph may address them:
+// then, on an error, they stay as they are (else null). Replaced ones are freed,
+// or kept while a graph captured over them lives: until the first growth after
+// its end, or the engine's end.
 struct pk_buf_bytes {
     void **p;
     int64_t bytes;
 };
-int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n, bool optional = false);
+int pk_regrow(pk_engine *e, std::shared_ptr<char> &use, const pk_buf_bytes *b, int n, bool optional = false);
 int pk_stage_reserve(pk_engine *e, int64_t bytes);
 
 // kernels defined in pk_dense.hip / pk_attn.hip without a launcher above

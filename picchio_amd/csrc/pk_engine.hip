@@ -44,13 +44,15 @@ void pk_dev_free(pk_engine *e, void *p) {
     if (p) (void)hipFree(p);
 }
 
-int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n, bool optional) {
+int pk_regrow(pk_engine *e, std::shared_ptr<char> &use, const pk_buf_bytes *b, int n, bool optional) {
     PK_HIP(hipStreamSynchronize(e->stream));
-    const bool graphs = e->live_graphs->load() > 0;
-    if (!graphs) {
-        for (void *p : e->outgrown) pk_dev_free(e, p);
-        e->outgrown.clear();
+    auto &og = e->outgrown;
+    for (size_t i = 0; i < og.size();) {
+        if (og[i].use.use_count() > 1) { ++i; continue; }
+        for (void *p : og[i].bufs) pk_dev_free(e, p);
+        og.erase(og.begin() + i);
     }
+    const bool held = use.use_count() > 1;             // by a graph captured over the present buffers
     std::vector<void *> fresh(n, nullptr);
     const auto alloc = [&]() {
         int rc = PK_OK;
@@ -64,12 +66,14 @@ int pk_regrow(pk_engine *e, const pk_buf_bytes *b, int n, bool optional) {
         return rc;
     };
     int rc = alloc();
-    if (rc != PK_OK && (optional || graphs)) return rc;
+    if (rc != PK_OK && (optional || held)) return rc;
+    if (held) og.push_back({use, {}});
     for (int i = 0; i < n; ++i) {
-        if (graphs && *b[i].p) e->outgrown.push_back(*b[i].p);
+        if (held && *b[i].p) og.back().bufs.push_back(*b[i].p);
         else pk_dev_free(e, *b[i].p);
         *b[i].p = nullptr;
     }
+    use = std::make_shared<char>();
     if (rc != PK_OK) PK_TRY(alloc());
     for (int i = 0; i < n; ++i) *b[i].p = fresh[i];
     return PK_OK;
@@ -182,7 +186,8 @@ static void engine_free(pk_engine *e) {
                     e->lm_bval, e->lm_bidx, e->dstate, e->step_out, e->samp, e->samp_av, e->samp_ai, e->samp_ws, e->hn_q, e->act_q, e->b_xq, e->b_actq, e->b_pairs, e->b_tiles,
                     e->moe_act_t, e->moe_eo_t, e->moe_cont_t, e->att_t, e->skinny_ws, e->lm_t};
     for (void *p : ptrs) pk_dev_free(e, p);
-    for (void *p : e->outgrown) pk_dev_free(e, p);
+    for (auto &o : e->outgrown)
+        for (void *p : o.bufs) pk_dev_free(e, p);
     if (e->L) {
         for (int l = 0; l < e->c.n_layers; ++l) {
             pk_layer_dev &d = e->L[l];
@@ -538,7 +543,7 @@ extern "C" int pk_engine_stall(pk_engine *e, int usec) {
 struct pk_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    std::shared_ptr<std::atomic<int>> live;   // the engine's count (which may end before the graph)
+    std::shared_ptr<char> uses[2];            // the engine's buffers' tokens at the capture (pk_regrow)
 };
 
 extern "C" int pk_capture_begin(pk_engine *e) {
@@ -564,8 +569,8 @@ extern "C" int pk_capture_end(pk_engine *e, pk_graph **out) {
         delete g;
         return PK_ERR_HIP;
     }
-    g->live = e->live_graphs;
-    g->live->fetch_add(1);
+    g->uses[0] = e->b_use;
+    g->uses[1] = e->g_use;
     *out = g;
     return PK_OK;
 }
@@ -580,7 +585,6 @@ extern "C" int pk_graph_destroy(pk_graph *g) {
     if (!g) return PK_OK;
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
-    g->live->fetch_sub(1);
     delete g;
     return PK_OK;
 }

@@ -180,7 +180,7 @@ static int batch_reserve(pk_engine *e, int T, bool optional = false) {
         {(void **)&e->b_tiles, (3 * (TK / 4 + 1 + c->n_experts) + 1) * 4},
     };
     if (!e->skinny_ws) PK_TRY(pk_dev_alloc(e, (void **)&e->skinny_ws, PK_SKINNY_WS * 4));
-    const int rc = pk_regrow(e, bufs, sizeof(bufs) / sizeof(bufs[0]), optional);
+    const int rc = pk_regrow(e, e->b_use, bufs, sizeof(bufs) / sizeof(bufs[0]), optional);
     if (!e->b_logits) e->batch_cap = 0;
     PK_TRY(rc);
     e->batch_cap = T;
@@ -332,7 +332,7 @@ static int grouped_reserve(pk_engine *e, int T) {
         {(void **)&e->g_pairs, P * 4},
         {(void **)&e->g_tiles, (5 * max_tiles + 1) * 4},
     };
-    const int rc = pk_regrow(e, bufs, sizeof(bufs) / sizeof(bufs[0]));
+    const int rc = pk_regrow(e, e->g_use, bufs, sizeof(bufs) / sizeof(bufs[0]));
     if (!e->g_limbs) e->g_cap = 0;
     PK_TRY(rc);
     e->g_cap = P;

@@ -70,6 +70,7 @@ extern "C" {
 void hh_budget(int64_t bytes) { budget = bytes; }
 int64_t hh_in_use() { return in_use; }
 int64_t hh_peak(int reset) { const int64_t p = peak; if (reset) peak = in_use; return p; }
+int hh_buffers() { int n = 0; for (auto &m : mem) n += m.second.live; return n; }
 int hh_stale() { return stale; }
 int hh_execs() { return execs; }
 int hh_instantiated() { return instantiated; }

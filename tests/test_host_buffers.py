@@ -47,6 +47,47 @@ assert hh.hh_in_use() == once, (hh.hh_in_use(), once)
 """)
 
 
+@pytest.mark.parametrize("call,bufs", [("pk_moe_forward_batch(h, 1, x, T, out, None, None)", 10),
+                                       ("pk_moe_forward_grouped(h, 1, x, T, None, None, out, None, None)", 14)],
+                         ids=["batch", "grouped"])
+def test_growth_keeps_only_what_a_graph_addresses(call, bufs):
+    """A graph lives over a slow growth: only the buffers of its own time stay
+    beside the present ones, and go at the first growth after its end, while a
+    later graph keeps its own."""
+    run(f"""
+h = engine(small(n_experts=8))
+x, out = dev(300 * 128), dev(300 * 128)
+def call(T):
+    pa.check(L.{call})
+def capture(T):
+    call(T)
+    pa.check(L.pk_capture_begin(h))
+    call(T)
+    g = vp()
+    pa.check(L.pk_capture_end(h, C.byref(g)))
+    return g
+g = capture(64)
+n = hh.hh_buffers()
+for T in range(65, 200):
+    call(T)
+assert hh.hh_buffers() == n + {bufs}, (n, hh.hh_buffers())
+g2 = capture(200)
+call(201)
+assert hh.hh_buffers() == n + 2 * {bufs}
+pa.check(L.pk_graph_launch(h, g))
+pa.check(L.pk_graph_launch(h, g2))
+assert hh.hh_stale() == 0, hh.hh_stale()
+pa.check(L.pk_graph_destroy(g))
+call(202)
+assert hh.hh_buffers() == n + {bufs}
+pa.check(L.pk_graph_launch(h, g2))
+assert hh.hh_stale() == 0
+pa.check(L.pk_graph_destroy(g2))
+call(203)
+assert hh.hh_buffers() == n
+""")
+
+
 def test_graph_may_outlive_its_engine():
     run("""
 h = engine(small())
